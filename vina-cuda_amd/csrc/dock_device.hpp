@@ -43,26 +43,41 @@ __device__ __forceinline__ float u01(uint32_t x) { return (float)(x >> 8) * (1.0
 
 // ----------------------------------------------------------------------------------------
 // Group collectives (G divides 64).  Sums: a row-of-16 all-reduce with DPP (quad_perm xor 1,
-// xor 2, row_half_mirror, row_mirror), then xor-16/xor-32 lane shuffles across rows.  Every step
+// xor 2, row_half_mirror, row_mirror), then across rows the sum of a value with its swapped copy
+// (v_permlane16_swap leaves the even rows' values in both rows of a pair in one register and the
+// odd rows' in the other; v_permlane32_swap does the same with the halves of the wave).  Every step
 // adds the same two operands in both partner lanes, so all lanes of a group hold bit-identical
-// sums (group decisions taken from them agree in every lane).
+// sums (group decisions taken from them agree in every lane).  Nothing here goes through the LDS
+// (as lane shuffles do): an iteration's end takes up to ten dependent sums.  512 chains of one
+// 20-atom ligand: 2.88 -> 2.82 ms; screening batches 1 % shorter.
 template <int CTRL> __device__ __forceinline__ float dpp(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+}
+// v(lane) + v(lane ^ 16), v(lane) + v(lane ^ 32)
+__device__ __forceinline__ float add_xor16(float v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float add_xor32(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 template <int G> __device__ __forceinline__ float gsum(float v) {
   v += dpp<0xB1>(v);    // quad_perm [1,0,3,2]
   v += dpp<0x4E>(v);    // quad_perm [2,3,0,1]
   v += dpp<0x141>(v);   // row_half_mirror
   v += dpp<0x140>(v);   // row_mirror
-  if constexpr (G >= 32) v += __shfl_xor(v, 16);
-  if constexpr (G >= 64) v += __shfl_xor(v, 32);
+  if constexpr (G >= 32) v = add_xor16(v);
+  if constexpr (G >= 64) v = add_xor32(v);
   return v;
 }
 template <int G> __device__ __forceinline__ float gget(float v, int src) { return __shfl(v, src, G); }
 template <int G> __device__ __forceinline__ int ggeti(int v, int src) { return __shfl(v, src, G); }
-// broadcast from a fixed lane of the group (a wave-uniform readlane when the group is the wave)
+// broadcast from a fixed lane of the group: a wave-uniform readlane when the group is the wave, a
+// DPP row_newbcast when it is a row of 16 lanes
 template <int G, int SRC> __device__ __forceinline__ float gbcast(float v) {
   if constexpr (G == 64) return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), SRC));
+  else if constexpr (G == 16) return dpp<0x150 + SRC>(v);
   else return __shfl(v, SRC, G);
 }
 
