@@ -471,9 +471,12 @@ __device__ float pair_terms_scatter(const LigView& L, const Scratch& S, const Ev
 // V11/lib/model.cpp:1324-1334; device form quasi_newton.cuh:1294-1339).
 // Returns e (group-uniform); g = this lane's gradient component.  rg (when given) receives the
 // gyration radius of the evaluated conformation, as gyration_radius computes it.
-template <int G>
+// want(e) says whether the group's caller will look at the gradient of a conformation of energy e;
+// where no group of the wavefront does, the adjoint is left out and g is 0.
+struct AlwaysWant { __device__ bool operator()(float) const { return true; } };
+template <int G, class Want = AlwaysWant>
 __device__ float eval_deriv(const LigView& L, const Scratch& S, const EvalK& K, const Conf& c, int l, float& g,
-                            float* rg = nullptr) {
+                            float* rg = nullptr, Want want = Want()) {
   float3 ax, org;
   kinematics<G>(L, S, c, l, ax, org);
   __syncthreads();
@@ -513,6 +516,8 @@ __device__ float eval_deriv(const LigView& L, const Scratch& S, const EvalK& K, 
   __syncthreads();
   // intramolecular pairs (eval_interacting_pairs_deriv, V11/lib/model.cpp:1241-1259)
   const float e_intra = L.rows ? pair_terms_rows<G>(L, S, K, l) : pair_terms_scatter<G>(L, S, K, l);
+  const float e_sum = gsum<G>(e_inter + e_intra);
+  if (!__any(want(e_sum))) { g = 0.0f; return e_sum; }
   __syncthreads();
   // adjoint: per-node force and moment (about the root origin) sums.  A node's atoms are one
   // contiguous range, so the sums are a segmented inclusive scan over the atom lanes (segment =
@@ -558,7 +563,7 @@ __device__ float eval_deriv(const LigView& L, const Scratch& S, const EvalK& K, 
   const int c6 = l - (G - 6);
   g = (l >= 1 && l <= L.T) ? gt
       : c6 == 0 ? r0 : c6 == 1 ? r1 : c6 == 2 ? r2 : c6 == 3 ? r3 : c6 == 4 ? r4 : c6 == 5 ? r5 : 0.0f;
-  return gsum<G>(e_inter + e_intra);
+  return e_sum;
 }
 
 // x <- x (+) factor*d (output_type_cl_increment, V11/inc/cuda/mutate_conf.cuh:8-29;
