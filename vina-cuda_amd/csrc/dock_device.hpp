@@ -189,7 +189,7 @@ struct EvalK {
   const float4* __restrict__ corners; vd_grid_desc gd;
   int cd0, cd01;                 // cells per x-row, per z-plane
   long long cplane;              // cells per type
-  const float2* __restrict__ lutp;  // pair table, (e, dor) per bin: [tp][bin]
+  const float2* __restrict__ lutp;  // pair table, (e, dor) per bin: [row][bin]
   float v_intra, v_inter, slope;
   // the interpolation quad (e_i, dor_i, e_{i+1}, dor_{i+1}) of entry i: one 16-byte load at 8-byte
   // alignment (global memory takes unaligned vector loads), half the table's footprint in the

@@ -120,6 +120,24 @@ double score_terms(int t1, int t2, double r, const double w[5]) {
   return s;
 }
 
+const PairTableRows& pair_table_rows() {
+  static const PairTableRows rows = [] {
+    PairTableRows r;
+    r.first.push_back(-1);   // row 0: zeros
+    std::map<std::tuple<double, bool, bool>, int> seen;
+    for (int b = 0; b < VD_XS_SIZE; ++b)
+      for (int a = 0; a <= b; ++a) {
+        const auto key = std::make_tuple(kXsRadius[a] + kXsRadius[b], xs_is_hydrophobic(a) && xs_is_hydrophobic(b),
+                                         (xs_is_donor(a) && xs_is_acceptor(b)) || (xs_is_donor(b) && xs_is_acceptor(a)));
+        const auto it = seen.emplace(key, (int)r.first.size());
+        if (it.second) r.first.push_back(type_pair_index(a, b));
+        r.row[type_pair_index(a, b)] = (uint8_t)it.first->second;
+      }
+    return r;
+  }();
+  return rows;
+}
+
 void Precalculated::build(const double w[5]) {
   const int n = VD_LUT_BINS;
   smooth_e.assign((size_t)VD_NUM_TYPE_PAIRS * n, 0.0);
@@ -154,15 +172,18 @@ void Precalculated::grid_rows(std::vector<float>& out) const {
 }
 
 void Precalculated::pair_bins(std::vector<float>& out) const {
-  // one extra all-zero row after the 153 type pairs, whose first entry is VD_ZERO_QUAD: empty pair
-  // slots and pairs beyond the cutoff read it and contribute nothing.  A pair inside the cutoff
-  // has r^2 < 64, so 32 r^2 < 2048 (scaling by 32 is exact) and its bin is at most 2047: the
-  // entry after it (bin + 1 <= 2048) lies in the same row.
-  out.assign(((size_t)VD_NUM_TYPE_PAIRS + 1) * VD_LUT_BINS * 2, 0.0f);
-  for (size_t i = 0; i < (size_t)VD_NUM_TYPE_PAIRS * VD_LUT_BINS; ++i) {
-    out[2 * i] = (float)smooth_e[i];
-    out[2 * i + 1] = (float)smooth_dor[i];
-  }
+  // row 0 is all zeros, its first entry VD_ZERO_QUAD: empty pair slots and pairs beyond the cutoff
+  // read it and contribute nothing.  A pair inside the cutoff has r^2 < 64, so 32 r^2 < 2048
+  // (scaling by 32 is exact) and its bin is at most 2047: the entry after it (bin + 1 <= 2048)
+  // lies in the same row.
+  const std::vector<int>& first = pair_table_rows().first;
+  out.assign(first.size() * VD_LUT_BINS * 2, 0.0f);
+  for (size_t r = 1; r < first.size(); ++r)
+    for (size_t b = 0; b < VD_LUT_BINS; ++b) {
+      const size_t i = (size_t)first[r] * VD_LUT_BINS + b, o = r * VD_LUT_BINS + b;
+      out[2 * o] = (float)smooth_e[i];
+      out[2 * o + 1] = (float)smooth_dor[i];
+    }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -641,13 +662,15 @@ vd_lig_header pack_ligand(const Ligand& L, std::vector<float>& blob, int G) {
   // rows: slot l holds pair (l, b); its word carries, in place of the first atom (= l), the slot
   // whose pair has second atom l in the same chunk (G: none), from which lane l pulls that
   // pair's force on atom l.  A slot without a pair names a written coordinate row as partner
-  // (atom l, or atom 0 for lanes beyond the ligand) and the all-zero row of the pair table
-  // (VD_NUM_TYPE_PAIRS) as type pair, so the device reads every word without decoding it.
+  // (atom l, or atom 0 for lanes beyond the ligand) and row 0 of the pair table, all zeros,
+  // as its own, so the device reads every word without decoding it.
   const int A = (int)L.atoms.size();
   auto empty_row = [&](int l, uint32_t src) {
-    return src | ((uint32_t)(l < A ? l : 0) << 8) | ((uint32_t)VD_NUM_TYPE_PAIRS << 16);
+    return src | ((uint32_t)(l < A ? l : 0) << 8);
   };
   std::vector<uint32_t> words(pairs);
+  for (uint32_t& w : words)
+    if (w != VD_NO_PAIR) w = (w & 0xFFFFu) | (uint32_t)pair_table_rows().row[w >> 16] << 16;
   if (h.pair_rows) {
     for (int ch = 0; ch < h.n_chunks; ++ch) {
       std::vector<uint32_t> inv(G, (uint32_t)G);
@@ -657,7 +680,8 @@ vd_lig_header pack_ligand(const Ligand& L, std::vector<float>& blob, int G) {
       }
       for (int l = 0; l < G; ++l) {
         const uint32_t w = pairs[(size_t)ch * G + l];
-        words[(size_t)ch * G + l] = w == VD_NO_PAIR ? empty_row(l, inv[l]) : (inv[l] | (w & 0xFFFFFF00u));
+        uint32_t& out = words[(size_t)ch * G + l];
+        out = w == VD_NO_PAIR ? empty_row(l, inv[l]) : (inv[l] | (out & 0xFFFFFF00u));
       }
     }
   }

@@ -10,7 +10,7 @@
 #define VD_LUT_BINS 2051             // int(32 * 64) + 3
 #define VD_LUT_FACTOR 32.0f
 #define VD_CUTOFF_SQR 64.0f
-#define VD_ZERO_QUAD (VD_NUM_TYPE_PAIRS * VD_LUT_BINS)   // first entry of the all-zero row after the pair table
+#define VD_ZERO_QUAD 0               // first entry of the pair table's all-zero row, row 0
 #define VD_GRID_ROW 16               // per (t1, bin) row of the map LUT: the values of t2 = 0..15 (64 B,
                                      // four aligned 16-byte loads); the t2 = 16 values follow all rows
                                      // as a [t1][bin] column
@@ -24,14 +24,14 @@
 //             (node | xs << 8 | heavy << 16 | heavy slot << 17).
 // Node words: o = (rel_origin xyz, parent); a = (rel_axis xyz, subtree_end) -- preorder, the
 //             subtree of node k is the node range [k, subtree_end).
-// Pair word:  a | b << 8 | tp << 16.  Pairs are stored in chunks of `chunk_lanes` slots (one per
+// Pair word:  a | b << 8 | row << 16 (row of the pair table, see pair_table_rows).  Pairs are stored in chunks of `chunk_lanes` slots (one per
 //             lane of a chain group); within a chunk every atom is the `a` of at most one pair
 //             and the `b` of at most one pair, so the force scatter of a chunk needs no atomics.
 //             Unused slots hold VD_NO_PAIR.  When the ligand has at most chunk_lanes atoms
 //             (pair_rows = 1), the pair in slot l has first atom l and its word is
-//             src | b << 8 | tp << 16 instead: src = the slot of the same chunk whose pair has
+//             src | b << 8 | row << 16 instead: src = the slot of the same chunk whose pair has
 //             second atom l (chunk_lanes: none); a slot without a pair has b = l (0 for lanes
-//             beyond the ligand) and tp = VD_NUM_TYPE_PAIRS, the all-zero row of the pair table.
+//             beyond the ligand) and row 0, the all-zero row of the pair table.
 //             The area is laid out in groups of four chunks, [group][lane][4].
 #define VD_NO_PAIR 0xFFFFFFFFu
 struct vd_lig_header {
