@@ -184,8 +184,7 @@ struct vd_ctx {
   vd_box box{};
   vd_grid_desc gd{};
   DevBuf<float> maps;
-  DevBuf<float4> corners;   // the maps as the searches read them: eight corners per cell
-  double corners_ms = 0.0;
+  DevBuf<float4> edges;     // the maps as the searches read them: edge records (vdk::EvalK)
   DevBuf<float4> grid_atoms;
   DevBuf<int2> grid_cells;
   double grid_ms = 0, eval_ms = 0;
@@ -432,8 +431,8 @@ vd_mc_consts make_consts(vd_ctx* c, const vd_dock_params* p, int depth, int bfgs
 
 vdk::EvalK make_evalk(vd_ctx* c, float v_intra, float v_inter, float slope) {
   vdk::EvalK k;
-  k.corners = c->corners.p; k.gd = c->gd; k.lutp = reinterpret_cast<const float2*>(c->lutp.p);
-  k.cd0 = c->gd.dim[0] - 1; k.cd01 = (c->gd.dim[0] - 1) * (c->gd.dim[1] - 1);
+  k.edges = c->edges.p; k.gd = c->gd; k.lutp = reinterpret_cast<const float2*>(c->lutp.p);
+  k.cd0 = c->gd.dim[0]; k.cd01 = c->gd.dim[0] * (c->gd.dim[1] - 1);
   k.cplane = (long long)k.cd01 * (c->gd.dim[2] - 1);
   k.v_intra = v_intra; k.v_inter = v_inter; k.slope = slope;
   return k;
@@ -461,14 +460,12 @@ double elapsed_ms(vd_ctx* c) {
   return ms;
 }
 
-// The corner records of the context's maps, timed on the context's stream.
-void make_corners(vd_ctx* c) {
-  c->corners.ensure((size_t)2 * VD_XS_SIZE * (c->gd.dim[0] - 1) * (c->gd.dim[1] - 1) * (c->gd.dim[2] - 1));
-  HIP_CHECK(hipEventRecord(c->ev0, c->stream));
-  HIP_CHECK(vdl::launch_corners(c->maps.p, c->corners.p, c->gd, c->stream));
-  HIP_CHECK(hipEventRecord(c->ev1, c->stream));
+// The edge records of the context's maps (grow the buffer before work is in flight: it may free).
+size_t edge_records(const vd_grid_desc& g) { return (size_t)VD_XS_SIZE * g.dim[0] * (g.dim[1] - 1) * (g.dim[2] - 1); }
+void make_edges(vd_ctx* c) {
+  c->edges.ensure(edge_records(c->gd));
+  HIP_CHECK(vdl::launch_edges(c->maps.p, c->edges.p, c->gd, c->stream));
   HIP_CHECK(hipStreamSynchronize(c->stream));
-  c->corners_ms = elapsed_ms(c);
 }
 
 // Algorithmic bytes of one evaluation in the MC kernel: the eight map corners of every typed
@@ -1078,7 +1075,7 @@ void vd_destroy(vd_ctx* c) {
   if (c->host_only) { delete c; return; }
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
-  c->lut_rows.release(); c->lutp.release(); c->maps.release(); c->corners.release(); c->grid_atoms.release();
+  c->lut_rows.release(); c->lutp.release(); c->maps.release(); c->edges.release(); c->grid_atoms.release();
   c->grid_cells.release();
   c->graphs.clear();
   for (hipStream_t& cs : c->cap)
@@ -1228,7 +1225,7 @@ int vd_grid_populate(vd_ctx* c, const vd_box* box) {
     HIP_CHECK(hipEventRecord(c->ev1, c->stream));
     HIP_CHECK(hipStreamSynchronize(c->stream));
     c->grid_ms = elapsed_ms(c);
-    make_corners(c);
+    make_edges(c);
     c->maps_ready = true;
     c->nc_ready = false;
   });
@@ -1254,7 +1251,7 @@ int vd_grid_upload(vd_ctx* c, const vd_box* box, const float* maps) {
     c->gd = make_desc(*box);
     c->maps.ensure((size_t)VD_XS_SIZE * c->gd.plane);
     HIP_CHECK(hipMemcpy(c->maps.p, maps, (size_t)VD_XS_SIZE * c->gd.plane * 4, hipMemcpyHostToDevice));
-    make_corners(c);
+    make_edges(c);
     c->maps_ready = true;
     c->nc_ready = false;
   });

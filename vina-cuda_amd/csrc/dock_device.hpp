@@ -181,14 +181,16 @@ struct Scratch {               // per chain, LDS
   float4* nacc;                // 2N: per-node force and moment sums
   float* stash;                // per wave: conformations parked out of registers, [slot][field][lane]
 };
-// Maps as the searches read them (corner records): per type, one 32-byte record per grid cell (cell (i,j,k) spans
-// points i..i+1, j..j+1, k..k+1), [type][k][j][i], holding the cell's eight corner values as
-// {f000, f100, f010, f110} {f001, f101, f011, f111}.  One lookup is then two 16-byte loads from
-// one cache line instead of four row gathers.
+// Maps as the searches read them (edge records): per type, one 16-byte record per point i of every
+// row (j, k) of grid cells, [type][k][j][i], holding the four values on the cell edges that cross
+// x = i: {f(i,j,k), f(i,j+1,k), f(i,j,k+1), f(i,j+1,k+1)}.  The records i and i + 1 are the eight
+// corners of cell (i,j,k): one lookup is two adjacent 16-byte loads instead of four row gathers,
+// and half the bytes of a record of eight corners per cell, for the caches and for the kernel that
+// writes them.
 struct EvalK {
-  const float4* __restrict__ corners; vd_grid_desc gd;
-  int cd0, cd01;                 // cells per x-row, per z-plane
-  long long cplane;              // cells per type
+  const float4* __restrict__ edges; vd_grid_desc gd;
+  int cd0, cd01;                 // records per x-row, per z-plane
+  long long cplane;              // records per type
   const float2* __restrict__ lutp;  // pair table, (e, dor) per bin: [row][bin]
   float v_intra, v_inter, slope;
   // the interpolation quad (e_i, dor_i, e_{i+1}, dor_{i+1}) of entry i: one 16-byte load at 8-byte
@@ -211,7 +213,7 @@ __device__ __forceinline__ float mul_rn(float a, float b) {
 }
 
 // Trilinear map value and derivative at p (grid::evaluate_aux, V11/lib/grid.cpp:50-167), from the
-// corner records of one type (cd0, cd01: cells per x-row, per z-plane).
+// edge records of one type (cd0, cd01: records per x-row, per z-plane).
 // prel = position relative to the map origin.  NaN/inf inputs stay in bounds.
 __device__ __forceinline__ float map_eval(const float4* __restrict__ m, int cd0, int cd01, const vd_grid_desc& gd,
                                           float3 prel, float slope, float v, float3& deriv) {
@@ -229,10 +231,10 @@ __device__ __forceinline__ float map_eval(const float4* __restrict__ m, int cd0,
     }
   }
   const float penalty = slope * (miss[0] * gd.factor_inv[0] + miss[1] * gd.factor_inv[1] + miss[2] * gd.factor_inv[2]);
-  const float4* b = m + 2 * ((long long)cd01 * a[2] + cd0 * a[1] + a[0]);
+  const float4* b = m + ((long long)cd01 * a[2] + cd0 * a[1] + a[0]);
   const float4 lo = b[0], hi = b[1];
-  const float f000 = lo.x, f100 = lo.y, f010 = lo.z, f110 = lo.w;
-  const float f001 = hi.x, f101 = hi.y, f011 = hi.z, f111 = hi.w;
+  const float f000 = lo.x, f010 = lo.y, f001 = lo.z, f011 = lo.w;
+  const float f100 = hi.x, f110 = hi.y, f101 = hi.z, f111 = hi.w;
   const float x = s[0], y = s[1], z = s[2], mx = 1 - x, my = 1 - y, mz = 1 - z;
   float f = f000 * mx * my * mz + f100 * x * my * mz + f010 * mx * y * mz + f110 * x * y * mz +
             f001 * mx * my * z + f101 * x * my * z + f011 * mx * y * z + f111 * x * y * z;
@@ -497,7 +499,7 @@ __device__ float eval_deriv(const LigView& L, const Scratch& S, const EvalK& K, 
         heavy[u] = (meta >> 16) & 1u;
         const int xs = (meta >> 8) & 255;
         if (xs < VD_XS_SIZE)
-          ev[u] = map_eval(K.corners + 2 * xs * K.cplane, K.cd0, K.cd01, K.gd,
+          ev[u] = map_eval(K.edges + xs * K.cplane, K.cd0, K.cd01, K.gd,
                            make_float3(prel.x + y[u].x, prel.y + y[u].y, prel.z + y[u].z), K.slope, K.v_inter, d[u]);
       }
     }
