@@ -215,7 +215,8 @@ struct vd_ctx {
   vdr::NcD nck{};
   DevBuf<double4> nc_atoms;
   DevBuf<int> nc_start;
-  DevBuf<double> lutd;                       // FP64 pair table quads of the refinement
+  DevBuf<double> lutd;                       // FP64 pair table of the refinement
+  DevBuf<uint8_t> ref_rows;                  // its row of each XS type pair
   DevBuf<double4> ref_geo;
   DevBuf<uint32_t> ref_pairs;
   DevBuf<vdr::RefHeader> ref_hdr;
@@ -291,16 +292,16 @@ void upload_lut(vd_ctx* c) {
   c->lutp.ensure(bins.size());
   HIP_CHECK(hipMemcpy(c->lut_rows.p, rows.data(), rows.size() * 4, hipMemcpyHostToDevice));
   HIP_CHECK(hipMemcpy(c->lutp.p, bins.data(), bins.size() * 4, hipMemcpyHostToDevice));
-  // FP64 quads (e_i, dor_i, e_i+1, dor_i+1) for the refinement after the search
-  std::vector<double> qd((size_t)VD_NUM_TYPE_PAIRS * VD_LUT_BINS * 4);
-  for (int tp = 0; tp < VD_NUM_TYPE_PAIRS; ++tp)
-    for (int b = 0; b < VD_LUT_BINS; ++b) {
-      const size_t o = (size_t)tp * VD_LUT_BINS, b1 = std::min(b + 1, VD_LUT_BINS - 1);
-      double* q = &qd[(o + b) * 4];
-      q[0] = c->pre.smooth_e[o + b]; q[1] = c->pre.smooth_dor[o + b]; q[2] = c->pre.smooth_e[o + b1]; q[3] = c->pre.smooth_dor[o + b1];
-    }
-  c->lutd.ensure(qd.size());
-  HIP_CHECK(hipMemcpy(c->lutd.p, qd.data(), qd.size() * 8, hipMemcpyHostToDevice));
+  // the same table in FP64, and the row of every (t1, t2), for the refinement after the search
+  std::vector<double> bd;
+  c->pre.pair_bins(bd);
+  c->lutd.ensure(bd.size());
+  HIP_CHECK(hipMemcpy(c->lutd.p, bd.data(), bd.size() * 8, hipMemcpyHostToDevice));
+  uint8_t rows_of[VD_XS_SIZE * VD_XS_SIZE];
+  for (int a = 0; a < VD_XS_SIZE; ++a)
+    for (int b = 0; b < VD_XS_SIZE; ++b) rows_of[a * VD_XS_SIZE + b] = vd::pair_table_rows().row[vd::type_pair_index(a, b)];
+  c->ref_rows.ensure(sizeof rows_of);
+  HIP_CHECK(hipMemcpy(c->ref_rows.p, rows_of, sizeof rows_of, hipMemcpyHostToDevice));
 }
 
 vd_grid_desc make_desc(const vd_box& b) {
@@ -884,7 +885,8 @@ vdr::RefHeader pack_ref(const vd::Ligand& L, std::vector<double4>& geo, std::vec
   const std::vector<uint32_t>& ch = vd::pair_chunks(L, 64);
   h.C = (int)(ch.size() / 64);
   h.off_pairs = (long long)pw.size();
-  pw.insert(pw.end(), ch.begin(), ch.end());
+  const uint8_t* row = vd::pair_table_rows().row;
+  for (uint32_t w : ch) pw.push_back(w == VD_NO_PAIR ? w : (w & 0xFFFFu) | (uint32_t)row[w >> 16] << 16);
   return h;
 }
 
@@ -956,7 +958,8 @@ RefineOut run_refine(vd_ctx* c, const std::vector<int>& ids, const std::vector<i
   a.conf_off = c->ref_coff.p; a.coords_off = c->ref_xoff.p;
   a.conf_in = c->ref_in.p; a.conf_out = c->ref_out.p; a.coords_out = c->ref_xyz.p;
   a.res = c->ref_res.p; a.evals = c->ref_evals.p;
-  a.K.lut = reinterpret_cast<const double4*>(c->lutd.p);
+  a.K.lut = reinterpret_cast<const double2*>(c->lutd.p);
+  a.K.rows = c->ref_rows.p;
   a.K.nc = c->nck;
   a.K.v = p->v;
   a.final_slope = p->slope;
@@ -1090,7 +1093,7 @@ void vd_destroy(vd_ctx* c) {
   c->tune_e.release(); c->tune_conf.release(); c->tune_heavy.release();
   c->nc_atoms.release(); c->nc_start.release(); c->ref_in.release(); c->ref_out.release(); c->ref_xyz.release();
   c->ref_res.release(); c->ref_lig.release(); c->ref_evals.release(); c->ref_coff.release(); c->ref_xoff.release();
-  c->lutd.release(); c->ref_geo.release(); c->ref_pairs.release(); c->ref_hdr.release();
+  c->lutd.release(); c->ref_rows.release(); c->ref_geo.release(); c->ref_pairs.release(); c->ref_hdr.release();
   c->pin_e.release(); c->pin_conf.release(); c->pin_heavy.release();
   c->pin_cout.release(); c->pin_xout.release(); c->pin_res.release();
   if (c->ev0) (void)hipEventDestroy(c->ev0);

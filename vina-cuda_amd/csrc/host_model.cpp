@@ -171,20 +171,25 @@ void Precalculated::grid_rows(std::vector<float>& out) const {
     }
 }
 
-void Precalculated::pair_bins(std::vector<float>& out) const {
+namespace {
+template <class Real>
+void fill_pair_bins(const std::vector<double>& smooth_e, const std::vector<double>& smooth_dor, std::vector<Real>& out) {
   // row 0 is all zeros, its first entry VD_ZERO_QUAD: empty pair slots and pairs beyond the cutoff
   // read it and contribute nothing.  A pair inside the cutoff has r^2 < 64, so 32 r^2 < 2048
   // (scaling by 32 is exact) and its bin is at most 2047: the entry after it (bin + 1 <= 2048)
   // lies in the same row.
   const std::vector<int>& first = pair_table_rows().first;
-  out.assign(first.size() * VD_LUT_BINS * 2, 0.0f);
+  out.assign(first.size() * VD_LUT_BINS * 2, Real(0));
   for (size_t r = 1; r < first.size(); ++r)
     for (size_t b = 0; b < VD_LUT_BINS; ++b) {
       const size_t i = (size_t)first[r] * VD_LUT_BINS + b, o = r * VD_LUT_BINS + b;
-      out[2 * o] = (float)smooth_e[i];
-      out[2 * o + 1] = (float)smooth_dor[i];
+      out[2 * o] = (Real)smooth_e[i];
+      out[2 * o + 1] = (Real)smooth_dor[i];
     }
 }
+}  // namespace
+void Precalculated::pair_bins(std::vector<float>& out) const { fill_pair_bins(smooth_e, smooth_dor, out); }
+void Precalculated::pair_bins(std::vector<double>& out) const { fill_pair_bins(smooth_e, smooth_dor, out); }
 
 // ---------------------------------------------------------------------------------------
 // Receptor (V11/lib/parse_pdbqt.cpp:258-284 + model.cpp:644-797 with every pair FIXED).

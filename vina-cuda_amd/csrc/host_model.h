@@ -52,6 +52,8 @@ struct Precalculated {
   //              (e_i, dor_i, e_{i+1}, dor_{i+1})
   void grid_rows(std::vector<float>& out) const;
   void pair_bins(std::vector<float>& out) const;
+  // the same rows and layout in FP64
+  void pair_bins(std::vector<double>& out) const;
 };
 
 struct LigAtom {

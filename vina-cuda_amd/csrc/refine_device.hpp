@@ -54,7 +54,8 @@ struct NcD {
   int n[3];
 };
 struct Consts {
-  const double4* __restrict__ lut;   // FP64 pair table quads (e_i, dor_i, e_i+1, dor_i+1), [tp][bin]
+  const double2* __restrict__ lut;   // FP64 pair table (e, dor), [row][bin], rows as the FP32 table's
+  const uint8_t* __restrict__ rows;  // row of the XS types (t1, t2): rows[t1 * VD_XS_SIZE + t2]
   NcD nc;
   double v;                          // curl cap of inter and intra (authentic_v)
 };
@@ -118,17 +119,48 @@ __device__ __forceinline__ double lane_value(double v, int j) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// Butterfly sum over `width` lanes (a power of two up to 64); every lane ends with the same sum.
+// Butterfly sum over `width` lanes (16 or 64); every lane ends with the same sum.  Partners at
+// distance 1, 2, 4, 8 by DPP (once the lanes of a quad agree, the half-row mirror pairs a quad with
+// the other one; once the lanes of a half row agree, the row mirror pairs it with the other half),
+// at distance 16 and 32 by the row and half swaps: no LDS shuffles, the same sums.
+template <int CTRL>
+__device__ __forceinline__ double dpp(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, 0xF, 0xF, false);
+  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, 0xF, 0xF, false);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
 template <int WIDTH>
 __device__ __forceinline__ double lane_sum(double v) {
-#pragma unroll
-  for (int m = 1; m < WIDTH; m <<= 1) v += __shfl_xor(v, m);
+  static_assert(WIDTH == 16 || WIDTH == 64, "");
+  v += dpp<0xB1>(v);    // quad_perm [1,0,3,2]
+  v += dpp<0x4E>(v);    // quad_perm [2,3,0,1]
+  v += dpp<0x141>(v);   // row_half_mirror
+  v += dpp<0x140>(v);   // row_mirror
+  if constexpr (WIDTH == 64) {
+    const auto join = [](unsigned lo, unsigned hi) {
+      return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+    };
+    unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    auto l = __builtin_amdgcn_permlane16_swap((unsigned)b, (unsigned)b, false, false);
+    auto h = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+    v = join(l[0], h[0]) + join(l[1], h[1]);
+    b = (unsigned long long)__double_as_longlong(v);
+    l = __builtin_amdgcn_permlane32_swap((unsigned)b, (unsigned)b, false, false);
+    h = __builtin_amdgcn_permlane32_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+    v = join(l[0], h[0]) + join(l[1], h[1]);
+  }
   return v;
+}
+// The interpolation quad (e_i, dor_i, e_i+1, dor_i+1) of entry i.
+__device__ __forceinline__ double4 quad(const Consts& K, int i) {
+  const double2 a = K.lut[i], b = K.lut[i + 1];
+  return make_double4(a.x, a.y, b.x, b.y);
 }
 
 // LDS of one pose (doubles): atoms 4A, frames 20N (R row-major 9, origin 3, lab axis 3, q 4, pad),
 // xyz 4A, frc 4A, node sums 8N, tree links N (one int per node: previous sibling + 1), torsion
-// half-angle cosines 64 and sines 64, gradient 64, H n x n.
+// half-angle cosines 64 and sines 64, gradient 64, table rows of the type pairs 37, H n x n.
 struct Pose {
   const double4* atom;      // LDS copy of the atom words
   const double4* node_o;    // global: rel_origin xyz + (parent + 1) | begin << 8 | end << 16
@@ -136,9 +168,12 @@ struct Pose {
   const uint32_t* pairs;    // global
   int A, N, T, C, n;
   double* frame; double4* xyz; double4* frc; double4* nsum; int* sib;
-  double* tcos; double* tsin; double* grad; double* H;
+  double* tcos; double* tsin; double* grad; uint8_t* rows; double* H;
 };
-__host__ __device__ inline int pose_lds_doubles(int A, int N, int n) { return 12 * A + 29 * N + 3 * 64 + n * n; }
+constexpr int kRowsDoubles = (VD_XS_SIZE * VD_XS_SIZE + 7) / 8;
+__host__ __device__ inline int pose_lds_doubles(int A, int N, int n) {
+  return 12 * A + 29 * N + 3 * 64 + kRowsDoubles + n * n;
+}
 
 __device__ inline void carve(Pose& P, double* lds, int Amax, int Nmax) {
   double* p = lds;
@@ -151,6 +186,7 @@ __device__ inline void carve(Pose& P, double* lds, int Amax, int Nmax) {
   P.tcos = p; p += 64;
   P.tsin = p; p += 64;
   P.grad = p; p += 64;
+  P.rows = reinterpret_cast<uint8_t*>(p); p += kRowsDoubles;
   P.H = p;
 }
 
@@ -267,16 +303,15 @@ __device__ inline double nc_inter(const Pose& P, const Consts& K, double slope, 
           rx[u] = p[0] - a[u].x; ry[u] = p[1] - a[u].y; rz[u] = p[2] - a[u].z;
           const double r2 = rx[u] * rx[u] + ry[u] * ry[u] + rz[u] * rz[u];
           ok[u] = k0 + 16 * u < end && r2 < VD_CUTOFF_SQR;
-          const int t2 = (int)a[u].w;
-          const int tp = t1 <= t2 ? t1 + t2 * (t2 + 1) / 2 : t2 + t1 * (t1 + 1) / 2;
+          const int tr = P.rows[t1 * VD_XS_SIZE + (int)a[u].w];
           const double rf = 32.0 * r2;
           const int b = ok[u] ? (int)rf : 0;
           rem[u] = rf - b;
-          idx[u] = ok[u] ? tp * VD_LUT_BINS + b : 0;
+          idx[u] = ok[u] ? tr * VD_LUT_BINS + b : 0;
         }
         double4 q[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) q[u] = K.lut[idx[u]];
+        for (int u = 0; u < U; ++u) q[u] = quad(K, idx[u]);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           if (!ok[u]) continue;
@@ -326,7 +361,7 @@ __device__ inline double pair_terms(const Pose& P, const Consts& K, int l) {
     if (ok && r2 < VD_CUTOFF_SQR) {
       const double rf = 32.0 * r2;
       const int bin = (int)rf;
-      const double4 q = K.lut[(int)(w >> 16) * VD_LUT_BINS + bin];
+      const double4 q = quad(K, (int)(w >> 16) * VD_LUT_BINS + bin);
       if constexpr (FAST) {
         double t = (q.z + q.x) / 2;
         if (t > 0 && K.v < 0.1 * kMaxFl) t *= K.v < kEps ? 0 : K.v / (K.v + t);
@@ -433,13 +468,14 @@ __device__ inline double ordered_dot(const Pose& P, double a, double b, int l) {
   return s;
 }
 // -(H v) for this lane's row, summed in index order.  The rows are read after a fence, so every
-// update of H before the call is seen.
+// update of H before the call is seen.  H is symmetric to the last bit (see the update): lane l
+// reads column l, consecutive words of the wavefront, where rows would be n doubles apart.
 __device__ inline double minus_hv(const Pose& P, double v, int l) {
   __syncthreads();
   double s = 0;
   for (int j = 0; j < P.n; ++j) {
     const double vj = lane_value(v, j);
-    if (l < P.n) s += P.H[l * P.n + j] * vj;
+    if (l < P.n) s += P.H[j * P.n + l] * vj;
   }
   return -s;
 }
@@ -488,14 +524,14 @@ __device__ inline double bfgs(const Pose& P, const Consts& K, double slope, Conf
     const double mhy = minus_hv(P, y, l);
     const double yhy = -ordered_dot(P, y, mhy, l);
     const double r = 1 / (alpha * yp);
-    // lane l updates H[l][j] for j >= l and mirrors it, as the reference's packed triangle
+    // lane l updates column l; both triangles take the products in the order of the reference's
+    // packed triangle (smaller index first), so H stays symmetric
     __syncthreads();
     for (int j = 0; j < n; ++j) {
       const double pj = lane_value(p, j), mhyj = lane_value(mhy, j);
-      if (l < n && j >= l) {
-        const double h = P.H[l * n + j] + (alpha * r * (mhy * pj + mhyj * p) + alpha * alpha * (r * r * yhy + r) * p * pj);
-        P.H[l * n + j] = h;
-        P.H[j * n + l] = h;
+      if (l < n) {
+        const double lo = j >= l ? p : pj, hi = j >= l ? pj : p;
+        P.H[j * n + l] += alpha * r * (mhy * pj + mhyj * p) + alpha * alpha * (r * r * yhy + r) * lo * hi;
       }
     }
     __syncthreads();
