@@ -219,6 +219,7 @@ struct vd_ctx {
   DevBuf<uint8_t> ref_rows;                  // its row of each XS type pair
   DevBuf<double4> ref_geo;
   DevBuf<uint32_t> ref_pairs;
+  DevBuf<uint16_t> ref_ent;
   DevBuf<vdr::RefHeader> ref_hdr;
   DevBuf<double> ref_in, ref_out, ref_xyz;
   DevBuf<double4> ref_res;
@@ -855,7 +856,10 @@ void check_post(const vd_post_params* p) {
 // heavy << 16), node origin words (rel_origin, (parent + 1) | begin << 8 | end << 16), node axis
 // words (rel_axis, subtree end | depth << 8 | (last child + 1) << 16 | (previous sibling + 1) << 24);
 // pair words in the conflict-free chunks of 64.
-vdr::RefHeader pack_ref(const vd::Ligand& L, std::vector<double4>& geo, std::vector<uint32_t>& pw, int max_steps) {
+// ent (teams): per (chunk, atom) the slot whose first atom it is, or 64, and the slot whose second
+// atom it is, or 65, in the high byte.
+vdr::RefHeader pack_ref(const vd::Ligand& L, std::vector<double4>& geo, std::vector<uint32_t>& pw,
+                        std::vector<uint16_t>* ent, int max_steps) {
   vdr::RefHeader h{};
   h.A = (int)L.atoms.size(); h.N = (int)L.nodes.size(); h.T = L.n_torsions(); h.heavy = L.n_heavy;
   h.max_steps = max_steps;
@@ -887,7 +891,31 @@ vdr::RefHeader pack_ref(const vd::Ligand& L, std::vector<double4>& geo, std::vec
   h.off_pairs = (long long)pw.size();
   const uint8_t* row = vd::pair_table_rows().row;
   for (uint32_t w : ch) pw.push_back(w == VD_NO_PAIR ? w : (w & 0xFFFFu) | (uint32_t)row[w >> 16] << 16);
+  if (ent) {
+    h.off_ent = (long long)ent->size();
+    ent->resize(ent->size() + (size_t)h.C * h.A, (uint16_t)(64 | 65 << 8));
+    uint16_t* t = ent->data() + h.off_ent;
+    for (size_t k = 0; k < ch.size(); ++k) {
+      if (ch[k] == VD_NO_PAIR) continue;
+      uint16_t& a = t[k / 64 * h.A + (ch[k] & 255)];
+      a = (uint16_t)((a & 0xFF00u) | k % 64);
+      uint16_t& b = t[k / 64 * h.A + ((ch[k] >> 8) & 255)];
+      b = (uint16_t)((b & 0xFFu) | k % 64 << 8);
+    }
+  }
   return h;
+}
+
+// Wavefronts per pose of a refinement launch.  A pose takes some 100 evaluations one after the other,
+// so a launch takes at least as long as its longest pose: four wavefronts per pose halve that
+// (20 poses of a 63-atom ligand 4.1 -> 2.0 ms), at the price of the slots in which three wait while
+// the first walks the tree.  As long as one wavefront per pose would leave no pose waiting for a slot
+// (eight per CU at the kernel's registers) the shorter pose is the shorter launch: 2,000 poses of
+// 63-atom ligands 14.8 -> 12.6 ms, of 41-atom ones 7.5 -> 6.8, of 21-atom ones 3.0 -> 3.2; beyond,
+// throughput counts (5,120 poses 19.7 -> 20.5, 10.7 -> 12.1, 4.4 -> 6.6 ms).  Ligands whose team does
+// not fit the LDS of a workgroup take one wavefront.
+int refine_waves(const vd_ctx* c, long long poses, int Amax, int Nmax, int nmax) {
+  return poses <= 8LL * c->n_cu && vdl::refine_lds_bytes(4, Amax, Nmax, nmax) <= c->lds_max ? 4 : 1;
 }
 
 // One refinement launch over poses of several ligands: ligand ids[k] owns poses[k] poses, their
@@ -907,15 +935,22 @@ RefineOut run_refine(vd_ctx* c, const std::vector<int>& ids, const std::vector<i
   if (!c->nc_ready) build_nc(c);
   std::vector<double4> geo;
   std::vector<uint32_t> pw;
+  std::vector<uint16_t> ent;
   std::vector<vdr::RefHeader> hdr;
   int Amax = 1, Nmax = 1, nmax = 1;
+  long long n_poses = 0;
+  for (size_t k = 0; k < ids.size(); ++k) {
+    const vd::Ligand& L = lig_at(c, ids[k]);
+    Amax = std::max(Amax, (int)L.atoms.size()); Nmax = std::max(Nmax, (int)L.nodes.size());
+    nmax = std::max(nmax, 6 + L.n_torsions());
+    n_poses += std::max(poses[k], 0);
+  }
+  const int waves = refine_waves(c, n_poses, Amax, Nmax, nmax);
   for (int id : ids) {
     const vd::Ligand& L = lig_at(c, id);
     if (L.n_torsions() + 7 > 64) throw ArgError(VD_ERR_CAPACITY, "ligand has too many torsions for the refinement");
     const int steps = p->max_steps > 0 ? p->max_steps : heur_bfgs((int)L.atoms.size(), p->local_search);
-    hdr.push_back(pack_ref(L, geo, pw, steps));
-    Amax = std::max(Amax, (int)L.atoms.size()); Nmax = std::max(Nmax, (int)L.nodes.size());
-    nmax = std::max(nmax, 6 + L.n_torsions());
+    hdr.push_back(pack_ref(L, geo, pw, waves > 1 ? &ent : nullptr, steps));
   }
   RefineOut r;
   std::vector<int> pose_lig;
@@ -937,7 +972,7 @@ RefineOut run_refine(vd_ctx* c, const std::vector<int>& ids, const std::vector<i
     if (!std::isfinite(conf[i])) throw ArgError(VD_ERR_ARG, "non-finite conformation value");
     cin[i] = conf[i];
   }
-  const int lds = vdl::refine_lds_bytes(Amax, Nmax, nmax);
+  const int lds = vdl::refine_lds_bytes(waves, Amax, Nmax, nmax);
   if (lds > c->lds_max)
     throw ArgError(VD_ERR_CAPACITY, "ligand too large for the refinement's LDS layout (" + std::to_string(lds) +
                                         " bytes of " + std::to_string(c->lds_max) + " per workgroup)");
@@ -948,13 +983,17 @@ RefineOut run_refine(vd_ctx* c, const std::vector<int>& ids, const std::vector<i
   c->ref_in.ensure(nc); c->ref_out.ensure(nc); c->ref_xyz.ensure(nx);
   HIP_CHECK(hipMemcpyAsync(c->ref_geo.p, geo.data(), geo.size() * sizeof(double4), hipMemcpyHostToDevice, c->stream));
   HIP_CHECK(hipMemcpyAsync(c->ref_pairs.p, pw.data(), pw.size() * 4, hipMemcpyHostToDevice, c->stream));
+  if (!ent.empty()) {
+    c->ref_ent.ensure(ent.size());
+    HIP_CHECK(hipMemcpyAsync(c->ref_ent.p, ent.data(), ent.size() * 2, hipMemcpyHostToDevice, c->stream));
+  }
   HIP_CHECK(hipMemcpyAsync(c->ref_hdr.p, hdr.data(), hdr.size() * sizeof(vdr::RefHeader), hipMemcpyHostToDevice, c->stream));
   HIP_CHECK(hipMemcpyAsync(c->ref_lig.p, pose_lig.data(), n * sizeof(int), hipMemcpyHostToDevice, c->stream));
   HIP_CHECK(hipMemcpyAsync(c->ref_coff.p, r.coff.data(), n * sizeof(long long), hipMemcpyHostToDevice, c->stream));
   HIP_CHECK(hipMemcpyAsync(c->ref_xoff.p, r.xoff.data(), n * sizeof(long long), hipMemcpyHostToDevice, c->stream));
   HIP_CHECK(hipMemcpyAsync(c->ref_in.p, cin.data(), nc * sizeof(double), hipMemcpyHostToDevice, c->stream));
   RefineArgs a{};
-  a.geo = c->ref_geo.p; a.pairs = c->ref_pairs.p; a.hdr = c->ref_hdr.p; a.pose_lig = c->ref_lig.p;
+  a.geo = c->ref_geo.p; a.pairs = c->ref_pairs.p; a.ent = c->ref_ent.p; a.hdr = c->ref_hdr.p; a.pose_lig = c->ref_lig.p;
   a.conf_off = c->ref_coff.p; a.coords_off = c->ref_xoff.p;
   a.conf_in = c->ref_in.p; a.conf_out = c->ref_out.p; a.coords_out = c->ref_xyz.p;
   a.res = c->ref_res.p; a.evals = c->ref_evals.p;
@@ -965,7 +1004,7 @@ RefineOut run_refine(vd_ctx* c, const std::vector<int>& ids, const std::vector<i
   a.final_slope = p->slope;
   a.Amax = Amax; a.Nmax = Nmax; a.nmax = nmax;
   HIP_CHECK(hipEventRecord(c->ev0, c->stream));
-  HIP_CHECK(vdl::launch_refine(a, n, c->stream));
+  HIP_CHECK(vdl::launch_refine(waves, a, n, c->stream));
   HIP_CHECK(hipEventRecord(c->ev1, c->stream));
   std::vector<int> ev(n);
   c->pin_cout.ensure(nc); c->pin_xout.ensure(nx); c->pin_res.ensure(n);
@@ -1093,7 +1132,7 @@ void vd_destroy(vd_ctx* c) {
   c->tune_e.release(); c->tune_conf.release(); c->tune_heavy.release();
   c->nc_atoms.release(); c->nc_start.release(); c->ref_in.release(); c->ref_out.release(); c->ref_xyz.release();
   c->ref_res.release(); c->ref_lig.release(); c->ref_evals.release(); c->ref_coff.release(); c->ref_xoff.release();
-  c->lutd.release(); c->ref_rows.release(); c->ref_geo.release(); c->ref_pairs.release(); c->ref_hdr.release();
+  c->lutd.release(); c->ref_rows.release(); c->ref_geo.release(); c->ref_ent.release(); c->ref_pairs.release(); c->ref_hdr.release();
   c->pin_e.release(); c->pin_conf.release(); c->pin_heavy.release();
   c->pin_cout.release(); c->pin_xout.release(); c->pin_res.release();
   if (c->ev0) (void)hipEventDestroy(c->ev0);

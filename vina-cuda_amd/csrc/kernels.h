@@ -48,6 +48,7 @@ struct EvalArgs {
 struct RefineArgs {
   const double4* geo;               // ligand atom and node words (refine_device.hpp RefHeader)
   const uint32_t* pairs;            // pair chunks of 64 words
+  const uint16_t* ent;              // slots per (chunk, atom), several wavefronts per pose only
   const vdr::RefHeader* hdr;        // per ligand slot; max_steps = the step budget per stage
   const int* pose_lig;              // ligand slot per pose
   const long long* conf_off;        // per pose: offset of its conformation (7 + T doubles)
@@ -62,8 +63,8 @@ struct RefineArgs {
 };
 
 namespace vdl {
-int refine_lds_bytes(int Amax, int Nmax, int nmax);
-hipError_t launch_refine(const RefineArgs& a, int poses, hipStream_t s);
+int refine_lds_bytes(int waves, int Amax, int Nmax, int nmax);
+hipError_t launch_refine(int waves, const RefineArgs& a, int poses, hipStream_t s);   // waves per pose: 1 or 4
 int mc_lds_bytes(int G, int Amax, int Nmax, int dense);
 int max_resident_mc_blocks(int G, int W, int mode, int lds_bytes);
 hipError_t launch_grid(const float4* atoms, const int2* cells, const GridCells& gc, const float4* lut_rows, float* maps,

@@ -566,41 +566,60 @@ __global__ __launch_bounds__(64) void vd_eval_kernel(EvalArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------
-// After the search: refine_structure (V11/main/main.cpp:139-157) of one pose per workgroup (one
-// wavefront), in FP64: dense BFGS on the receptor atoms themselves with the out-of-box slope
+// After the search: refine_structure (V11/main/main.cpp:139-157) of one pose per workgroup of NW
+// wavefronts, in FP64: dense BFGS on the receptor atoms themselves with the out-of-box slope
 // raised 1e2 -> 1e10 until the heavy atoms lie within the box (a pose that never gets inside
 // reports max_fl), then the parts of the final score at the refined pose (fast tables, slope
 // a.final_slope).
-__global__ __launch_bounds__(64) void vd_refine_kernel(RefineArgs a) {
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void vd_refine_kernel(RefineArgs a) {
   extern __shared__ double lds_d[];
-  const int pose = blockIdx.x, l = threadIdx.x;
+  const int pose = blockIdx.x, l = threadIdx.x & 63, w = threadIdx.x >> 6;
   const vdr::RefHeader h = a.hdr[a.pose_lig[pose]];
   vdr::Pose P;
   vdr::carve(P, lds_d, a.Amax, a.Nmax);
-  P.node_o = a.geo + h.off_atoms + h.A;
-  P.node_a = a.geo + h.off_atoms + h.A + h.N;
+  vdr::Team M{};
   P.pairs = a.pairs + h.off_pairs;
   P.A = h.A; P.N = h.N; P.T = h.T; P.C = h.C; P.n = 6 + h.T;
-  for (int i = l; i < h.A; i += 64) const_cast<double4*>(P.atom)[i] = a.geo[h.off_atoms + i];
-  for (int i = l; i < VD_XS_SIZE * VD_XS_SIZE; i += 64) P.rows[i] = a.K.rows[i];
+  for (int i = threadIdx.x; i < h.A; i += 64 * NW) const_cast<double4*>(P.atom)[i] = a.geo[h.off_atoms + i];
+  for (int i = threadIdx.x; i < h.N; i += 64 * NW) {
+    const_cast<double4*>(P.node_o)[i] = a.geo[h.off_atoms + h.A + i];
+    const_cast<double4*>(P.node_a)[i] = a.geo[h.off_atoms + h.A + h.N + i];
+  }
+  for (int i = threadIdx.x; i < VD_XS_SIZE * VD_XS_SIZE; i += 64 * NW) P.rows[i] = a.K.rows[i];
+  if constexpr (NW > 1) {
+    vdr::carve_team(M, lds_d + vdr::pose_lds_doubles(a.Amax, a.Nmax, a.nmax));
+    M.ent = a.ent + h.off_ent;
+    for (int i = threadIdx.x; i < 3 * vdr::kTeamChunks; i += 64 * NW) {
+      double* z = M.f + i / 3 * vdr::kTeamChunkDoubles + i % 3 * 66 + 64;
+      z[0] = 0.0; z[1] = -0.0;
+    }
+    __syncthreads();
+    if (w > 0) { vdr::team_serve<NW>(P, a.K, M, w, l); return; }
+  }
+  vdr::wave_sync();
   vdr::load_links(P, l);
   const double* ci = a.conf_in + a.conf_off[pose];
   vdr::Conf x;
   x.pos = vdr::D3{ci[0], ci[1], ci[2]};
   x.q = vdr::DQ{ci[3], ci[4], ci[5], ci[6]};
   x.tor = (l >= 6 && l < 6 + h.T) ? ci[7 + (l - 6)] : 0.0;
-  __syncthreads();
+  vdr::wave_sync();
   double e = 0, slope = 100;
   bool inside = false;
   int evals = 0;
   for (int p = 0; p < 5; ++p, slope *= 100) {
-    e = vdr::bfgs(P, a.K, slope, x, h.max_steps, l, evals);
-    vdr::set_coords(P, x, l);
+    e = vdr::bfgs<NW>(P, a.K, M, slope, x, h.max_steps, l, evals);
+    vdr::set_coords(P, a.K, x, l);
     inside = vdr::within(P, a.K, l);
     if (inside) break;
   }
+  if constexpr (NW > 1) {
+    if (l == 0) *M.serve = 0;
+    __syncthreads();
+  }
   if (!inside) e = vdr::kMaxFl;
-  const double e_inter = vdr::lane_sum<64>(vdr::nc_inter<true>(P, a.K, a.final_slope, l));
+  const double e_inter = vdr::lane_sum<64>(vdr::nc_inter<true>(P, a.K, a.final_slope, l >> 4, 4, l));
   const double e_intra = vdr::lane_sum<64>(vdr::pair_terms<true>(P, a.K, l));
   double* co = a.conf_out + a.conf_off[pose];
   if (l == 0) {
@@ -627,10 +646,17 @@ namespace vdl {
 
 hipError_t scratch_address(void** p) { return hipGetSymbolAddress(p, HIP_SYMBOL(scratch)); }
 
-int refine_lds_bytes(int Amax, int Nmax, int nmax) { return 8 * vdr::pose_lds_doubles(Amax, Nmax, nmax); }
+int refine_lds_bytes(int waves, int Amax, int Nmax, int nmax) {
+  return 8 * (vdr::pose_lds_doubles(Amax, Nmax, nmax) + (waves > 1 ? vdr::team_lds_doubles() : 0));
+}
 
-hipError_t launch_refine(const RefineArgs& a, int poses, hipStream_t s) {
-  hipLaunchKernelGGL(vd_refine_kernel, dim3(poses), dim3(64), refine_lds_bytes(a.Amax, a.Nmax, a.nmax), s, a);
+hipError_t launch_refine(int waves, const RefineArgs& a, int poses, hipStream_t s) {
+  const int lds = refine_lds_bytes(waves, a.Amax, a.Nmax, a.nmax);
+  switch (waves) {
+    case 1: hipLaunchKernelGGL(vd_refine_kernel<1>, dim3(poses), dim3(64), lds, s, a); break;
+    case 4: hipLaunchKernelGGL(vd_refine_kernel<4>, dim3(poses), dim3(256), lds, s, a); break;
+    default: return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 

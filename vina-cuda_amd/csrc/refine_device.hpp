@@ -42,6 +42,7 @@ struct RefHeader {
   int A, N, T, C;          // atoms, nodes, torsions, pair chunks
   long long off_atoms;     // double4 index of A atom words, then N origin words, N axis words
   long long off_pairs;     // uint32 index of C * 64 pair words
+  long long off_ent;       // uint16 index of C * A slot words (teams)
   int max_steps, heavy;
 };
 // Receptor atoms of the direct evaluation: cells n[0] x n[1] x n[2] over the box [lo, hi]
@@ -119,6 +120,14 @@ __device__ __forceinline__ double lane_value(double v, int j) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
+// Orders the LDS accesses of one wavefront (they complete in order; this keeps the compiler from
+// moving them): everything below that is not marked "team" runs on one wavefront, also where a
+// workgroup has several.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Butterfly sum over `width` lanes (16 or 64); every lane ends with the same sum.  Partners at
 // distance 1, 2, 4, 8 by DPP (once the lanes of a quad agree, the half-row mirror pairs a quad with
 // the other one; once the lanes of a half row agree, the row mirror pairs it with the other half),
@@ -158,30 +167,34 @@ __device__ __forceinline__ double4 quad(const Consts& K, int i) {
   return make_double4(a.x, a.y, b.x, b.y);
 }
 
-// LDS of one pose (doubles): atoms 4A, frames 20N (R row-major 9, origin 3, lab axis 3, q 4, pad),
-// xyz 4A, frc 4A, node sums 8N, tree links N (one int per node: previous sibling + 1), torsion
-// half-angle cosines 64 and sines 64, gradient 64, table rows of the type pairs 37, H n x n.
+// LDS of one pose (doubles): atoms 4A, node words 8N, frames 20N (R row-major 9, origin 3, lab axis
+// 3, q 4, pad), xyz 4A, frc 4A, receptor lists A, node sums 12N, tree links N (one int per node:
+// previous sibling + 1), torsion half-angle cosines 64 and sines 64, gradient 64, table rows of the
+// type pairs 37, H n x n.
 struct Pose {
   const double4* atom;      // LDS copy of the atom words
-  const double4* node_o;    // global: rel_origin xyz + (parent + 1) | begin << 8 | end << 16
-  const double4* node_a;    // global: rel_axis xyz + subtree end
+  const double4* node_o;    // LDS copy: rel_origin xyz + (parent + 1) | begin << 8 | end << 16
+  const double4* node_a;    // LDS copy: rel_axis xyz + tree links
   const uint32_t* pairs;    // global
   int A, N, T, C, n;
-  double* frame; double4* xyz; double4* frc; double4* nsum; int* sib;
+  double* frame; double4* xyz; double4* frc; int2* list; double* nsum; int* sib;
   double* tcos; double* tsin; double* grad; uint8_t* rows; double* H;
 };
 constexpr int kRowsDoubles = (VD_XS_SIZE * VD_XS_SIZE + 7) / 8;
 __host__ __device__ inline int pose_lds_doubles(int A, int N, int n) {
-  return 12 * A + 29 * N + 3 * 64 + kRowsDoubles + n * n;
+  return 13 * A + 41 * N + 3 * 64 + kRowsDoubles + n * n;
 }
 
 __device__ inline void carve(Pose& P, double* lds, int Amax, int Nmax) {
   double* p = lds;
   P.atom = reinterpret_cast<const double4*>(p); p += 4 * Amax;
+  P.node_o = reinterpret_cast<const double4*>(p); p += 4 * Nmax;
+  P.node_a = reinterpret_cast<const double4*>(p); p += 4 * Nmax;
   P.frame = p; p += 20 * Nmax;
   P.xyz = reinterpret_cast<double4*>(p); p += 4 * Amax;
   P.frc = reinterpret_cast<double4*>(p); p += 4 * Amax;
-  P.nsum = reinterpret_cast<double4*>(p); p += 8 * Nmax;
+  P.list = reinterpret_cast<int2*>(p); p += Amax;
+  P.nsum = p; p += 12 * Nmax;
   P.sib = reinterpret_cast<int*>(p); p += Nmax;
   P.tcos = p; p += 64;
   P.tsin = p; p += 64;
@@ -203,7 +216,7 @@ __device__ __forceinline__ Links links_of(const Pose& P, int k) {
 // once per pose, before the first evaluation.
 __device__ inline void load_links(const Pose& P, int l) {
   if (l < P.N) P.sib[l] = links_of(P, l).prev_sibling;
-  __syncthreads();
+  wave_sync();
 }
 // Depth of the deepest node (wave-uniform).
 __device__ __forceinline__ int max_depth(const Pose& P, int l) {
@@ -219,8 +232,8 @@ __device__ __forceinline__ int max_depth(const Pose& P, int l) {
 // every node of the depth above is done (the operations of the reference's preorder walk, each
 // node's from its parent's frame); then every lane places its atoms, x_i = o_node + R_node
 // local_i.  The half-angle cosine and sine of angle_to_quaternion are computed beforehand by each
-// torsion's own lane.  Leaves frames and absolute coordinates in LDS.
-__device__ inline void set_coords(const Pose& P, const Conf& c, int l) {
+// torsion's own lane.  Leaves frames (set_frames) and absolute coordinates (set_coords) in LDS.
+__device__ inline void set_frames(const Pose& P, const Conf& c, int l) {
   if (l >= 6 && l < 6 + P.T) {
     const double a = normalize_angle(c.tor);
     P.tcos[l - 6] = cos(a / 2);
@@ -234,7 +247,7 @@ __device__ inline void set_coords(const Pose& P, const Conf& c, int l) {
   }
   const int depth = l < P.N ? links_of(P, l).depth : 0;
   for (int d = 1; __any(d <= depth); ++d) {
-    __syncthreads();
+    wave_sync();
     if (l >= 1 && l < P.N && depth == d) {
       const int k = l;
       const double4 no = P.node_o[k], na = P.node_a[k];
@@ -250,27 +263,52 @@ __device__ inline void set_coords(const Pose& P, const Conf& c, int l) {
       fk[15] = q.a; fk[16] = q.b; fk[17] = q.c; fk[18] = q.d;
     }
   }
-  __syncthreads();
-  for (int i = l; i < P.A; i += 64) {
-    const double4 a = P.atom[i];
-    const double* f = P.frame + 20 * (int)(meta_of(a.w) & 255u);
-    const D3 y = add(D3{f[9], f[10], f[11]}, mat_vec(f, D3{a.x, a.y, a.z}));
-    P.xyz[i] = make_double4(y.x, y.y, y.z, 0.0);
+  wave_sync();
+}
+// Clamps p to the box: pen += distance outside, ob = side.
+__device__ __forceinline__ void clamp_to_box(const Consts& K, double (&p)[3], double (&ob)[3], double& pen) {
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    if (p[k] < K.nc.lo[k]) { pen += fabs(p[k] - K.nc.lo[k]); p[k] = K.nc.lo[k]; ob[k] = -1; }
+    else if (p[k] > K.nc.hi[k]) { pen += fabs(p[k] - K.nc.hi[k]); p[k] = K.nc.hi[k]; ob[k] = 1; }
   }
-  __syncthreads();
+}
+// Coordinates of atom i and, where it is typed, the range of its cell's receptor atoms (looked up
+// here, for all atoms at once, so that the direct term does not wait for it atom by atom).
+__device__ inline void place_atom(const Pose& P, const Consts& K, int i) {
+  const double4 a = P.atom[i];
+  const double* f = P.frame + 20 * (int)(meta_of(a.w) & 255u);
+  const D3 y = add(D3{f[9], f[10], f[11]}, mat_vec(f, D3{a.x, a.y, a.z}));
+  P.xyz[i] = make_double4(y.x, y.y, y.z, 0.0);
+  double p[3] = {y.x, y.y, y.z}, ob[3], pen = 0;
+  clamp_to_box(K, p, ob, pen);
+  int ci[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const double cf = (p[k] - K.nc.lo[k]) * K.nc.inv_cell[k];   // NaN lands in cell 0, overflow in the last
+    ci[k] = cf >= 0 ? (int)fmin(cf, (double)(K.nc.n[k] - 1)) : 0;
+  }
+  const int cell = (ci[2] * K.nc.n[1] + ci[1]) * K.nc.n[0] + ci[0];
+  P.list[i] = make_int2(K.nc.start[cell], K.nc.start[cell + 1]);
+}
+__device__ inline void set_coords(const Pose& P, const Consts& K, const Conf& c, int l) {
+  set_frames(P, c, l);
+  for (int i = l; i < P.A; i += 64) place_atom(P, K, i);
+  wave_sync();
 }
 
 // non_cache::eval_deriv (FAST = false) / non_cache::eval (FAST = true), V11/lib/non_cache.cpp:
 // 38-128: each typed atom is clamped to the box (slope x the distance outside joins the energy,
 // +-slope the force); the receptor atoms listed for the cell of the clamped point are scored
 // with the table (interpolated value and dor, or the bin's fast value); the atom's sum is capped
-// by curl.  One atom per row of 16 lanes.  FAST = false writes dE/dx of every atom to frc.
-// Returns this lane's share of the energy.
+// by curl.  One atom per row of 16 lanes: atoms i0 + row of `rows` rows in all.  FAST = false
+// writes dE/dx of every atom to frc, and its energy to frc's w.  Returns this lane's share of the
+// energy.
 template <bool FAST>
-__device__ inline double nc_inter(const Pose& P, const Consts& K, double slope, int l) {
-  const int row = l >> 4, rl = l & 15;
+__device__ inline double nc_inter(const Pose& P, const Consts& K, double slope, int row, int rows, int l) {
+  const int rl = l & 15;
   double e_lane = 0;
-  for (int i0 = 0; i0 < P.A; i0 += 4) {
+  for (int i0 = 0; i0 < P.A; i0 += rows) {
     const int i = i0 + row;
     const int t1 = i < P.A ? (int)((meta_of(P.atom[i].w) >> 8) & 255u) : VD_XS_SIZE;
     double e = 0, dx = 0, dy = 0, dz = 0, pen = 0;
@@ -278,20 +316,13 @@ __device__ inline double nc_inter(const Pose& P, const Consts& K, double slope, 
     if (t1 < VD_XS_SIZE) {
       const double4 y = P.xyz[i];
       double p[3] = {y.x, y.y, y.z};
-      int ci[3];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        if (p[k] < K.nc.lo[k]) { pen += fabs(p[k] - K.nc.lo[k]); p[k] = K.nc.lo[k]; ob[k] = -1; }
-        else if (p[k] > K.nc.hi[k]) { pen += fabs(p[k] - K.nc.hi[k]); p[k] = K.nc.hi[k]; ob[k] = 1; }
-        const double cf = (p[k] - K.nc.lo[k]) * K.nc.inv_cell[k];   // NaN lands in cell 0, overflow in the last
-        ci[k] = cf >= 0 ? (int)fmin(cf, (double)(K.nc.n[k] - 1)) : 0;
-      }
-      const int cell = (ci[2] * K.nc.n[1] + ci[1]) * K.nc.n[0] + ci[0];
-      const int end = K.nc.start[cell + 1];
+      clamp_to_box(K, p, ob, pen);
+      const int2 range = P.list[i];
+      const int end = range.y;
       // four candidates per pass: their atom words, then their table quads, are all loaded
       // before the first is used; each lane still adds its candidates in list order
       constexpr int U = 4;
-      for (int k0 = K.nc.start[cell] + rl; k0 < end; k0 += 16 * U) {
+      for (int k0 = range.x + rl; k0 < end; k0 += 16 * U) {
         double4 a[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) a[u] = K.nc.atoms[k0 + 16 * u < end ? k0 + 16 * u : k0];
@@ -334,8 +365,9 @@ __device__ inline double nc_inter(const Pose& P, const Consts& K, double slope, 
       dx *= t2; dy *= t2; dz *= t2;
     }
     if (rl == 0 && i < P.A) {
-      if constexpr (!FAST) P.frc[i] = make_double4(dx + slope * ob[0], dy + slope * ob[1], dz + slope * ob[2], 0.0);
-      e_lane += e + pen * slope;
+      const double ea = e + pen * slope;
+      if constexpr (!FAST) P.frc[i] = make_double4(dx + slope * ob[0], dy + slope * ob[1], dz + slope * ob[2], ea);
+      e_lane += ea;
     }
   }
   return e_lane;
@@ -388,18 +420,138 @@ __device__ inline double pair_terms(const Pose& P, const Consts& K, int l) {
   return e_lane;
 }
 
+// ---- Several wavefronts per pose (a team).  The first runs the optimiser, the kinematics and the
+// adjoint's tree walks; the direct term, the pairs and the sums of the pair forces over the atoms
+// are shared.  Every value is computed by the operations of the one-wave form and summed in its
+// order, so the results are the same bit for bit:
+//   atoms     one per row of 16 lanes, as in one wave; energies are kept per atom and summed at the end
+//   pairs     a wave takes every NW-th chunk; a pair's force and energy go to its slot's entry in LDS
+//             (kTeamChunks chunks per round), and then the thread that owns a component of an atom's
+//             force adds, chunk by chunk, the force of the slot whose first atom it is (minus) and of
+//             the slot whose second atom it is (plus).  `ent` names the two slots per (chunk, atom);
+//             entries 64 and 65 of a chunk are +0 and -0: subtracting the one and adding the other
+//             leave any value as it is.
+// What bounds an evaluation is the length of its chain (63 atoms, cycles of wave 0 before the tree
+// walks were shortened: frames 6,400, direct term 15,800, pairs 5,900, their sums 10,200, adjoint
+// 9,000); eight candidates per pass in place of four, or 168 registers for three workgroups per CU,
+// lengthened it (5.8 -> 8.6 and 7.1 ms for 1,200 poses of a library).
+struct Team {
+  double* slope; int* serve;          // the request: serve 1 = evaluate at *slope, 0 = end
+  double* f;                          // kTeamChunks x (3 x 66 force components, 64 energies)
+  const uint16_t* ent;                // global: [chunk][atom] slot as first atom | slot as second << 8
+};
+constexpr int kTeamChunks = 16;
+constexpr int kTeamChunkDoubles = 3 * 66 + 64;
+__host__ __device__ inline int team_lds_doubles() { return 2 + kTeamChunks * kTeamChunkDoubles; }
+__device__ inline void carve_team(Team& M, double* p) {
+  M.slope = p; M.serve = reinterpret_cast<int*>(p + 1); M.f = p + 2;
+}
+__device__ __forceinline__ void team_sync() { __syncthreads(); }
+
+template <int NW>
+__device__ inline void team_forces(const Pose& P, const Consts& K, const Team& M, double slope, int w, int l, double& e_pairs) {
+  const int tid = 64 * w + l;
+  for (int i = tid; i < P.A; i += 64 * NW) place_atom(P, K, i);
+  team_sync();
+  nc_inter<false>(P, K, slope, 4 * w + (l >> 4), 4 * NW, l);
+  e_pairs = 0;
+  for (int c0 = 0; c0 == 0 || c0 < P.C; c0 += kTeamChunks) {
+    const int c1 = min(c0 + kTeamChunks, P.C);
+    constexpr int U = kTeamChunks / NW;   // this wave's chunks of the round, their table reads in flight together
+    uint32_t pw[U];
+    double rx[U], ry[U], rz[U], rf[U];
+    double4 q[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) pw[u] = c0 + w + NW * u < c1 ? P.pairs[(c0 + w + NW * u) * 64 + l] : VD_NO_PAIR;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool ok = pw[u] != VD_NO_PAIR;
+      const double4 pa = P.xyz[ok ? (pw[u] & 255u) : 0u], pb = P.xyz[ok ? ((pw[u] >> 8) & 255u) : 0u];
+      rx[u] = pb.x - pa.x; ry[u] = pb.y - pa.y; rz[u] = pb.z - pa.z;
+      const double r2 = rx[u] * rx[u] + ry[u] * ry[u] + rz[u] * rz[u];
+      rf[u] = ok && r2 < VD_CUTOFF_SQR ? 32.0 * r2 : -1.0;
+      q[u] = quad(K, rf[u] >= 0 ? (int)(pw[u] >> 16) * VD_LUT_BINS + (int)rf[u] : 0);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (c0 + w + NW * u >= c1) break;
+      double e = 0, fx = 0, fy = 0, fz = 0;
+      if (rf[u] >= 0) {
+        const double rem = rf[u] - (int)rf[u];
+        e = q[u].x + rem * (q[u].z - q[u].x);
+        const double dor = q[u].y + rem * (q[u].w - q[u].y);
+        fx = dor * rx[u]; fy = dor * ry[u]; fz = dor * rz[u];
+        if (e > 0 && K.v < 0.1 * kMaxFl) {
+          const double t = K.v < kEps ? 0 : K.v / (K.v + e);
+          e *= t;
+          const double t2 = t * t;
+          fx *= t2; fy *= t2; fz *= t2;
+        }
+      }
+      double* f = M.f + (w + NW * u) * kTeamChunkDoubles;
+      f[l] = fx; f[66 + l] = fy; f[132 + l] = fz; f[198 + l] = e;
+    }
+    // this thread's part of the sums over the atoms: wave 0, 1, 2 the force component of that number,
+    // wave 3 the energies; the first slot words are on their way before the wait
+    uint32_t en[kTeamChunks];
+    const int i0 = min(l, P.A - 1);
+#pragma unroll
+    for (int u = 0; u < kTeamChunks; ++u) en[u] = w < 3 && c0 + u < c1 ? M.ent[(c0 + u) * P.A + i0] : 64u | 65u << 8;
+    team_sync();
+    if (w < 3) {
+      for (int i = l; i < P.A; i += 64) {
+        double* fi = reinterpret_cast<double*>(P.frc + i) + w;
+        double F = *fi;
+#pragma unroll
+        for (int u = 0; u < kTeamChunks; ++u) {
+          const uint32_t word = i == l ? en[u] : c0 + u < c1 ? M.ent[(c0 + u) * P.A + i] : 64u | 65u << 8;
+          const double* f = M.f + u * kTeamChunkDoubles + 66 * w;
+          F -= f[word & 255u];
+          F += f[word >> 8];
+        }
+        *fi = F;
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < kTeamChunks; ++u)
+        if (c0 + u < c1) e_pairs += M.f[u * kTeamChunkDoubles + 198 + l];
+    }
+    team_sync();
+  }
+  // every atom's moment about its node's origin; the pair energies on their way to the first wave
+  for (int i = tid; i < P.A; i += 64 * NW) {
+    const double4 x = P.xyz[i], F = P.frc[i];
+    const double* fr = P.frame + 20 * (int)(meta_of(P.atom[i].w) & 255u);
+    const D3 t = cross(sub(D3{x.x, x.y, x.z}, D3{fr[9], fr[10], fr[11]}), D3{F.x, F.y, F.z});
+    P.xyz[i] = make_double4(t.x, t.y, t.z, 0.0);
+  }
+  if (w == 3) M.f[198 + l] = e_pairs;
+  team_sync();
+  e_pairs = M.f[198 + l];
+}
+
+// The other wavefronts: evaluate on request until the first one is done.
+template <int NW>
+__device__ inline void team_serve(const Pose& P, const Consts& K, const Team& M, int w, int l) {
+  for (;;) {
+    team_sync();
+    if (!*M.serve) return;
+    double e;
+    team_forces<NW>(P, K, M, *M.slope, w, l, e);
+  }
+}
+
 // model::eval_deriv over non_cache with the intramolecular pairs (model.cpp:1324-1334) at the
 // given slope.  Returns e (wave-uniform); g = this lane's gradient component (0 beyond n).
 // The adjoint follows the oracle's order: per-node force and torque sums over the node's atoms
 // in index order, then every parent folds in its children in decreasing index order, which is
 // the order the reference's reverse-preorder walk adds them in; parents one depth at a time from
 // the deepest, so a child is complete before it is folded.
-__device__ inline double eval_deriv(const Pose& P, const Consts& K, double slope, const Conf& c, int l, double& g) {
-  set_coords(P, c, l);
-  double e = nc_inter<false>(P, K, slope, l);
-  __syncthreads();
-  e += pair_terms<false>(P, K, l);
-  __syncthreads();
+// Node sums, fold and gradient, once the atoms' forces are in frc.  TORQUE: xyz holds each atom's
+// moment about its node's origin in place of its coordinates.
+template <bool TORQUE>
+__device__ inline void adjoint(const Pose& P, int l, double& g) {
+  D3 F0{0, 0, 0}, T0{0, 0, 0};   // this lane's node
   if (l < P.N) {
     const double4 no = P.node_o[l];
     const uint32_t bits = meta_of(no.w);
@@ -407,40 +559,76 @@ __device__ inline double eval_deriv(const Pose& P, const Consts& K, double slope
     const double* f = P.frame + 20 * l;
     const D3 o{f[9], f[10], f[11]};
     D3 F{0, 0, 0}, T{0, 0, 0};
+#pragma unroll 4
     for (int i = begin; i < end; ++i) {
       const double4 fr = P.frc[i], x = P.xyz[i];
-      const D3 fi{fr.x, fr.y, fr.z};
+      const D3 fi{fr.x, fr.y, fr.z}, xi{x.x, x.y, x.z};
       F = add(F, fi);
-      T = add(T, cross(sub(D3{x.x, x.y, x.z}, o), fi));
+      T = add(T, TORQUE ? xi : cross(sub(xi, o), fi));
     }
-    P.nsum[2 * l] = make_double4(F.x, F.y, F.z, 0.0);
-    P.nsum[2 * l + 1] = make_double4(T.x, T.y, T.z, 0.0);
+    F0 = F; T0 = T;
   }
+  // fold, one depth at a time from the deepest: the lanes of the depth's nodes hand over their sums
+  // and the moment of their force about the parent's origin, and the parents' lanes add them
   const Links lk = l < P.N ? links_of(P, l) : Links{-1, -1, -1};
-  for (int d = max_depth(P, l) - 1; d >= 0; --d) {
-    __syncthreads();
-    if (l < P.N && lk.depth == d && lk.last_child >= 0) {
-      const double* fp = P.frame + 20 * l;
-      double4 Fp = P.nsum[2 * l], Tp = P.nsum[2 * l + 1];
-      for (int k = lk.last_child; k >= 0; k = P.sib[k]) {
-        const double* f = P.frame + 20 * k;
-        const double4 Fk = P.nsum[2 * k], Tk = P.nsum[2 * k + 1];
-        P.grad[6 + k - 1] = dot(D3{Tk.x, Tk.y, Tk.z}, D3{f[12], f[13], f[14]});
-        const D3 arm = sub(D3{f[9], f[10], f[11]}, D3{fp[9], fp[10], fp[11]});
-        const D3 c = cross(arm, D3{Fk.x, Fk.y, Fk.z});
-        Fp.x += Fk.x; Fp.y += Fk.y; Fp.z += Fk.z;
-        Tp.x = (Tp.x + c.x) + Tk.x; Tp.y = (Tp.y + c.y) + Tk.y; Tp.z = (Tp.z + c.z) + Tk.z;
-      }
-      P.nsum[2 * l] = Fp; P.nsum[2 * l + 1] = Tp;
-    }
+  D3 arm{0, 0, 0}, axis{0, 0, 0};
+  if (l >= 1 && l < P.N) {
+    const double* f = P.frame + 20 * l;
+    const double* fp = P.frame + 20 * ((int)(meta_of(P.node_o[l].w) & 255u) - 1);
+    arm = sub(D3{f[9], f[10], f[11]}, D3{fp[9], fp[10], fp[11]});
+    axis = D3{f[12], f[13], f[14]};
   }
-  __syncthreads();
+  for (int d = max_depth(P, l); d >= 1; --d) {
+    if (lk.depth == d) {
+      double* n = P.nsum + 12 * l;
+      const D3 c = cross(arm, F0);
+      n[0] = F0.x; n[1] = F0.y; n[2] = F0.z; n[3] = c.x; n[4] = c.y; n[5] = c.z; n[6] = T0.x; n[7] = T0.y; n[8] = T0.z;
+      P.grad[6 + l - 1] = dot(T0, axis);
+    }
+    wave_sync();
+    if (lk.depth == d - 1) {
+      for (int k = lk.last_child; k >= 0; k = P.sib[k]) {
+        const double* n = P.nsum + 12 * k;
+        F0.x += n[0]; F0.y += n[1]; F0.z += n[2];
+        T0.x = (T0.x + n[3]) + n[6]; T0.y = (T0.y + n[4]) + n[7]; T0.z = (T0.z + n[5]) + n[8];
+      }
+    }
+    wave_sync();
+  }
   if (l == 0) {
-    const double4 F0 = P.nsum[0], T0 = P.nsum[1];
     P.grad[0] = F0.x; P.grad[1] = F0.y; P.grad[2] = F0.z; P.grad[3] = T0.x; P.grad[4] = T0.y; P.grad[5] = T0.z;
   }
-  __syncthreads();
+  wave_sync();
   g = l < P.n ? P.grad[l] : 0.0;
+}
+
+// NW = 1: this wavefront alone.  NW > 1: called by the team's first wavefront, the others being in
+// team_serve.
+template <int NW>
+__device__ inline double eval_deriv(const Pose& P, const Consts& K, const Team& M, double slope, const Conf& c, int l,
+                                    double& g) {
+  double e;
+  if constexpr (NW == 1) {
+    set_coords(P, K, c, l);
+    e = nc_inter<false>(P, K, slope, l >> 4, 4, l);
+    wave_sync();
+    e += pair_terms<false>(P, K, l);
+    wave_sync();
+  } else {
+    set_frames(P, c, l);
+    if (l == 0) { *M.slope = slope; *M.serve = 1; }
+    double pairs;
+    team_sync();
+    team_forces<NW>(P, K, M, slope, 0, l, pairs);
+    // the lane sums of the one-wave form: lane 16 r holds atoms r, r + 4, ...; pairs by slot
+    e = 0;
+    if ((l & 15) == 0) {
+#pragma unroll 4
+      for (int i = l >> 4; i < P.A; i += 4) e += P.frc[i].w;
+    }
+    e += pairs;
+  }
+  adjoint<(NW > 1)>(P, l, g);
   return lane_sum<64>(e);
 }
 
@@ -471,7 +659,7 @@ __device__ inline double ordered_dot(const Pose& P, double a, double b, int l) {
 // update of H before the call is seen.  H is symmetric to the last bit (see the update): lane l
 // reads column l, consecutive words of the wavefront, where rows would be n doubles apart.
 __device__ inline double minus_hv(const Pose& P, double v, int l) {
-  __syncthreads();
+  wave_sync();
   double s = 0;
   for (int j = 0; j < P.n; ++j) {
     const double vj = lane_value(v, j);
@@ -484,12 +672,14 @@ __device__ inline double minus_hv(const Pose& P, double v, int l) {
 // at most 10 halvings from alpha = 1 with the Armijo constant 1e-4, the first step rescales the
 // diagonal, the rank-two update skips steps with alpha y.p < epsilon; a result above the start
 // reverts to the start.  No early stop beyond the gradient-norm test.  Returns f; x is updated.
-__device__ inline double bfgs(const Pose& P, const Consts& K, double slope, Conf& x, int max_steps, int l, int& evals) {
+template <int NW>
+__device__ inline double bfgs(const Pose& P, const Consts& K, const Team& M, double slope, Conf& x, int max_steps, int l,
+                              int& evals) {
   const int n = P.n;
   if (l < n)
     for (int j = 0; j < n; ++j) P.H[l * n + j] = (j == l) ? 1.0 : 0.0;
   double g;
-  double f0 = eval_deriv(P, K, slope, x, l, g);
+  double f0 = eval_deriv<NW>(P, K, M, slope, x, l, g);
   ++evals;
   const double f_orig = f0;
   const Conf x_orig = x;
@@ -500,7 +690,7 @@ __device__ inline double bfgs(const Pose& P, const Consts& K, double slope, Conf
     Conf x_new = x;
     for (int trial = 0; trial < 10; ++trial) {
       x_new = increment(x, p, alpha, l, P.T);
-      f1 = eval_deriv(P, K, slope, x_new, l, g_new);
+      f1 = eval_deriv<NW>(P, K, M, slope, x_new, l, g_new);
       ++evals;
       if (f1 - f0 < 1e-4 * alpha * pg) break;
       alpha *= 0.5;
@@ -514,9 +704,9 @@ __device__ inline double bfgs(const Pose& P, const Consts& K, double slope, Conf
       const double yy = ordered_dot(P, y, y, l);
       if (fabs(yy) > kEps) {
         const double dg = alpha * ordered_dot(P, y, p, l) / yy;
-        __syncthreads();
+        wave_sync();
         if (l < n) P.H[l * n + l] = dg;
-        __syncthreads();
+        wave_sync();
       }
     }
     const double yp = ordered_dot(P, y, p, l);
@@ -526,7 +716,7 @@ __device__ inline double bfgs(const Pose& P, const Consts& K, double slope, Conf
     const double r = 1 / (alpha * yp);
     // lane l updates column l; both triangles take the products in the order of the reference's
     // packed triangle (smaller index first), so H stays symmetric
-    __syncthreads();
+    wave_sync();
     for (int j = 0; j < n; ++j) {
       const double pj = lane_value(p, j), mhyj = lane_value(mhy, j);
       if (l < n) {
@@ -534,7 +724,7 @@ __device__ inline double bfgs(const Pose& P, const Consts& K, double slope, Conf
         P.H[j * n + l] += alpha * r * (mhy * pj + mhyj * p) + alpha * alpha * (r * r * yhy + r) * lo * hi;
       }
     }
-    __syncthreads();
+    wave_sync();
   }
   if (!(f0 <= f_orig)) { f0 = f_orig; x = x_orig; }
   return f0;
