@@ -117,6 +117,7 @@ struct McSlot {
     ev0 = ev1 = nullptr; stream = nullptr;   // the streams are the process's (device_stream)
   }
 };
+constexpr size_t kEvalDirectBytes = 4u << 20;   // vd_eval's host arrays the kernel reads and writes in place
 constexpr int kMcSlots = 4;   // at most four hardware queues per process on these devices
 
 // A persistent batch captured as a hipGraph (vd_set_graphs): every stage of one vd_dock_batch
@@ -187,7 +188,7 @@ struct vd_ctx {
   DevBuf<float4> edges;     // the maps as the searches read them: edge records (vdk::EvalK)
   DevBuf<float4> grid_atoms;
   DevBuf<int2> grid_cells;
-  double grid_ms = 0, eval_ms = 0;
+  double grid_ms = 0;
   // ligands
   std::vector<vd::Ligand> ligs;
   // MC launches: slot 0 runs on `stream`, slots 1.. on their own streams (created on first use)
@@ -197,8 +198,14 @@ struct vd_ctx {
   bool graphs_on = false;                    // persistent batches run as captured graphs (vd_set_graphs)
   hipStream_t cap[2] = {nullptr, nullptr};   // this context's capture-only streams (nothing runs on them)
   std::vector<std::unique_ptr<GraphEntry>> graphs;   // least recently used first
-  DevBuf<float4> blob;                       // ligand record of vd_eval
-  DevBuf<vd_lig_header> headers;
+  DevBuf<float4> blob;                       // record of the ligand vd_eval scored last: eval_id for groups
+  int eval_id = -1, eval_G = 0;              // of eval_G lanes (-1: none)
+  vd_lig_header eval_header{};
+  // vd_eval's kernel takes its own start and end from the device's constant clock: a pair of events
+  // around it lengthened every call by 18 us
+  DevBuf<unsigned long long> eval_clock;
+  int clock_khz = 100000;
+  bool eval_timed = false;
   DevBuf<float> io_a, io_b, io_c;
   BatchState batch;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -226,6 +233,7 @@ struct vd_ctx {
   DevBuf<int> ref_lig, ref_evals;
   DevBuf<long long> ref_coff, ref_xoff;
   PostState post;
+  PinnedBuf<float> pin_eval;                     // vd_eval's small host arrays, read and written by the kernel
   PinnedBuf<float> pin_e, pin_conf, pin_heavy;   // per-chain results of a batch, for pose lists
   PinnedBuf<double> pin_cout, pin_xout;          // refinement outputs
   PinnedBuf<double4> pin_res;
@@ -1095,6 +1103,9 @@ int vd_create(int device, vd_ctx** out) {
     HIP_CHECK(hipEventCreate(&c->ev0));
     HIP_CHECK(hipEventCreate(&c->ev1));
     HIP_CHECK(hipEventCreate(&c->ev_base));
+    c->eval_clock.ensure(2);
+    HIP_CHECK(hipMemset(c->eval_clock.p, 0, 16));
+    HIP_CHECK(hipDeviceGetAttribute(&c->clock_khz, hipDeviceAttributeWallClockRate, device));
     for (int k = 0; k < kMcSlots; ++k) {
       HIP_CHECK(hipEventCreate(&c->mc[k].ev0));
       HIP_CHECK(hipEventCreate(&c->mc[k].ev1));
@@ -1127,12 +1138,13 @@ void vd_destroy(vd_ctx* c) {
     c->mc[k].release();
   }
   if (c->ev_base) (void)hipEventDestroy(c->ev_base);
-  c->blob.release(); c->headers.release(); c->io_a.release(); c->io_b.release(); c->io_c.release();
+  c->blob.release(); c->io_a.release(); c->io_b.release(); c->io_c.release();
   c->batch.e.release(); c->batch.conf.release(); c->batch.heavy.release();
   c->tune_e.release(); c->tune_conf.release(); c->tune_heavy.release();
   c->nc_atoms.release(); c->nc_start.release(); c->ref_in.release(); c->ref_out.release(); c->ref_xyz.release();
   c->ref_res.release(); c->ref_lig.release(); c->ref_evals.release(); c->ref_coff.release(); c->ref_xoff.release();
   c->lutd.release(); c->ref_rows.release(); c->ref_geo.release(); c->ref_ent.release(); c->ref_pairs.release(); c->ref_hdr.release();
+  c->pin_eval.release(); c->eval_clock.release();
   c->pin_e.release(); c->pin_conf.release(); c->pin_heavy.release();
   c->pin_cout.release(); c->pin_xout.release(); c->pin_res.release();
   if (c->ev0) (void)hipEventDestroy(c->ev0);
@@ -1359,37 +1371,59 @@ int vd_eval(vd_ctx* c, int id, long long n, const float* conf, float* e, float* 
     const vd::Ligand& L = lig_at(c, id);
     if (n == 0) return;
     const int T = L.n_torsions();
-    int G = pick_group(c, L, cpw);
-    Packed pk = pack(c, G, {id});
-    c->blob.ensure(pk.blob.size() / 4 + 1);
-    c->headers.ensure(1);
-    HIP_CHECK(hipMemcpyAsync(c->blob.p, pk.blob.data(), pk.blob.size() * 4, hipMemcpyHostToDevice, c->stream));
-    HIP_CHECK(hipMemcpyAsync(c->headers.p, pk.headers.data(), sizeof(vd_lig_header), hipMemcpyHostToDevice, c->stream));
-    const float* d_conf = conf; float* d_e = e; float* d_g = grad;
-    if (!device_ptrs) {
-      c->io_a.ensure((size_t)n * (7 + T)); c->io_b.ensure(n); c->io_c.ensure((size_t)n * (6 + T));
-      HIP_CHECK(hipMemcpyAsync(c->io_a.p, conf, (size_t)n * (7 + T) * 4, hipMemcpyHostToDevice, c->stream));
-      d_conf = c->io_a.p; d_e = c->io_b.p; d_g = c->io_c.p;
+    const int G = pick_group(c, L, cpw);
+    // the record of the ligand last scored stays on the device (a ligand never changes)
+    if (c->eval_id != id || c->eval_G != G) {
+      c->eval_id = -1;
+      Packed pk = pack(c, G, {id});
+      c->blob.ensure(pk.blob.size() / 4 + 1);
+      HIP_CHECK(hipMemcpyAsync(c->blob.p, pk.blob.data(), pk.blob.size() * 4, hipMemcpyHostToDevice, c->stream));
+      HIP_CHECK(hipStreamSynchronize(c->stream));   // the copy's source ends with this block
+      c->eval_header = pk.headers[0];
+      c->eval_id = id; c->eval_G = G;
     }
+    const size_t n_in = (size_t)n * (7 + T), n_out = (size_t)n * (6 + T);
     EvalArgs a{};
-    a.blob = c->blob.p; a.header = c->headers.p; a.host_header = pk.headers[0];
+    a.clock = c->eval_clock.p;
+    a.blob = c->blob.p; a.header = c->eval_header;
     a.K = make_evalk(c, v_intra, v_inter, slope);
-    a.conf = d_conf; a.n_conf = n; a.e = d_e; a.grad = d_g;
+    a.conf = conf; a.n_conf = n; a.e = e; a.grad = grad;
+    // Host arrays up to kEvalDirectBytes go through page-locked memory that the kernel reads and
+    // writes itself: no copies to wait for (one pose of a 34-atom ligand 88 -> 27 us, 5,003 poses of a
+    // 75-atom one 190 -> 146 us).  Larger ones are copied to the device: a staging area of their size
+    // and a second pass over them on the host would cost more than the copies.
+    const bool direct = !device_ptrs && (n_in + n_out + (size_t)n) * 4 <= kEvalDirectBytes;
+    if (direct) {
+      c->pin_eval.ensure(n_in + n_out + (size_t)n);
+      std::memcpy(c->pin_eval.p, conf, n_in * 4);
+      a.conf = c->pin_eval.p; a.grad = c->pin_eval.p + n_in; a.e = c->pin_eval.p + n_in + n_out;
+    } else if (!device_ptrs) {
+      c->io_a.ensure(n_in); c->io_b.ensure(n); c->io_c.ensure(n_out);
+      HIP_CHECK(hipMemcpyAsync(c->io_a.p, conf, n_in * 4, hipMemcpyHostToDevice, c->stream));
+      a.conf = c->io_a.p; a.e = c->io_b.p; a.grad = c->io_c.p;
+    }
     const long long per_block = 64 / G;
     const int blocks = (int)std::min<long long>((n + per_block - 1) / per_block, (long long)c->n_cu * 16);
-    HIP_CHECK(hipEventRecord(c->ev0, c->stream));
     HIP_CHECK(vdl::launch_eval(G, a, blocks, c->stream));
-    HIP_CHECK(hipEventRecord(c->ev1, c->stream));
-    if (!device_ptrs) {
-      HIP_CHECK(hipMemcpyAsync(e, d_e, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream));
-      HIP_CHECK(hipMemcpyAsync(grad, d_g, (size_t)n * (6 + T) * 4, hipMemcpyDeviceToHost, c->stream));
+    c->eval_timed = true;
+    if (!direct && !device_ptrs) {
+      HIP_CHECK(hipMemcpyAsync(e, a.e, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream));
+      HIP_CHECK(hipMemcpyAsync(grad, a.grad, n_out * 4, hipMemcpyDeviceToHost, c->stream));
     }
     HIP_CHECK(hipStreamSynchronize(c->stream));
-    c->eval_ms = elapsed_ms(c);
+    if (direct) {
+      std::memcpy(grad, a.grad, n_out * 4);
+      std::memcpy(e, a.e, (size_t)n * 4);
+    }
   });
 }
 
-double vd_eval_last_ms(const vd_ctx* c) { return c ? c->eval_ms : 0.0; }
+double vd_eval_last_ms(const vd_ctx* c) {
+  unsigned long long t[2];
+  if (!c || !c->eval_timed || hipSetDevice(c->device) != hipSuccess) return 0.0;
+  if (hipMemcpy(t, c->eval_clock.p, sizeof t, hipMemcpyDeviceToHost) != hipSuccess) return 0.0;
+  return t[1] > t[0] ? (double)(t[1] - t[0]) / c->clock_khz : 0.0;
+}
 
 int vd_dock_params_default(vd_dock_params* p) {
   if (!p) return VD_ERR_ARG;

@@ -37,11 +37,11 @@ struct McArgs {
 
 struct EvalArgs {
   const float4* blob;
-  const vd_lig_header* header;      // device copy
-  vd_lig_header host_header;
+  vd_lig_header header;
   vdk::EvalK K;
   const float* conf; long long n_conf;
   float* e; float* grad;
+  unsigned long long* clock;        // the launch's first and last device clock tick (the second only grows)
 };
 
 // Refinement launch (vd_refine_kernel, FP64): one pose per workgroup.

@@ -541,19 +541,28 @@ __global__ __launch_bounds__(64) void vd_eval_kernel(EvalArgs a) {
   float* lds = reinterpret_cast<float*>(lds4);
   constexpr int CPW = 64 / G;
   const int lane = threadIdx.x, group = lane / G, l = lane % G;
-  const vd_lig_header h = *a.header;
-  stage_ligand<G>(a.blob, h, lds, lane);
-  __syncthreads();
+  if (blockIdx.x == 0 && lane == 0) a.clock[0] = (unsigned long long)wall_clock64();
+  const vd_lig_header& h = a.header;
   LigView L; Scratch S; float* H;
   make_views<G>(a.blob, h, lds, h.n_atoms, h.n_nodes, 0, group, L, S, H);
   const int T = h.n_torsions, nc = 7 + T, ng = 6 + T;
-  for (long long base = (long long)blockIdx.x * CPW; base < a.n_conf; base += (long long)gridDim.x * CPW) {
+  // a conformation's 7 + T <= G numbers in one load, a number per lane, a conformation ahead: they
+  // may lie in host memory, two microseconds away
+  const auto numbers = [&](long long c) { return l < nc ? a.conf[(c < a.n_conf ? c : 0) * nc + l] : 0.0f; };
+  const long long stride = (long long)gridDim.x * CPW;
+  float next = numbers((long long)blockIdx.x * CPW + group);
+  stage_ligand<G>(a.blob, h, lds, lane);
+  __syncthreads();
+  for (long long base = (long long)blockIdx.x * CPW; base < a.n_conf; base += stride) {
     const long long c = base + group;
     const bool valid = c < a.n_conf;
-    const float* x = a.conf + (valid ? c : 0) * nc;
+    const float x = next;
+    if (base + stride < a.n_conf) next = numbers(c + stride);
     Conf cf;
-    cf.px = x[0]; cf.py = x[1]; cf.pz = x[2]; cf.q = Quat{x[3], x[4], x[5], x[6]};
-    cf.tor = (l >= 1 && l <= T) ? x[6 + l] : 0.0f;
+    cf.px = gbcast<G, 0>(x); cf.py = gbcast<G, 1>(x); cf.pz = gbcast<G, 2>(x);
+    cf.q = Quat{gbcast<G, 3>(x), gbcast<G, 4>(x), gbcast<G, 5>(x), gbcast<G, 6>(x)};
+    const float tor = gget<G>(x, min(l + 6, G - 1));
+    cf.tor = (l >= 1 && l <= T) ? tor : 0.0f;
     float g;
     const float e = eval_deriv<G>(L, S, a.K, cf, l, g);
     if (valid) {
@@ -563,6 +572,7 @@ __global__ __launch_bounds__(64) void vd_eval_kernel(EvalArgs a) {
       if (l >= G - 6) go[l - (G - 6)] = g;
     }
   }
+  if (lane == 0) atomicMax(a.clock + 1, (unsigned long long)wall_clock64());
 }
 
 // ------------------------------------------------------------------------------------------
@@ -686,8 +696,7 @@ hipError_t launch_edges(const float* maps, float4* edges, const vd_grid_desc& gd
 }
 
 hipError_t launch_eval(int G, const EvalArgs& a, int blocks, hipStream_t s) {
-  const int A = a.host_header.n_atoms, N = a.host_header.n_nodes;
-  const int lds = mc_lds_bytes(G, A, N, 0);
+  const int lds = mc_lds_bytes(G, a.header.n_atoms, a.header.n_nodes, 0);
   switch (G) {
     case 64: hipLaunchKernelGGL(vd_eval_kernel<64>, dim3(blocks), dim3(64), lds, s, a); break;
     case 32: hipLaunchKernelGGL(vd_eval_kernel<32>, dim3(blocks), dim3(64), lds, s, a); break;
