@@ -73,3 +73,24 @@ def test_every_atom_type_scores_as_the_oracle(ctx, n, start, step):
             ref, gref, _, _ = orc.eval_deriv(grid, lig, conf[k].astype(np.float64))
             assert abs(energy[k] - ref) <= max(1e-4, 1e-3 * abs(ref)) + intra_cutoff_bound(lig, conf[k])
             assert np.abs(grad[k] - gref).max() <= 1e-3 * max(1.0, np.abs(gref).max()) + 1e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("types", [range(17), (0,), (1, 10, 11, 2, 6), (12, 13, 14, 15), (3, 7, 16), (4, 8), (5, 9)])
+def test_maps_of_every_receptor_type(module_ctx, types):
+    """The map kernel's rows, by class of receptor type: plain, hydrophobic, donor, acceptor, both.
+    Tolerance as test_gpu_core.py: 1e-4 relative plus the change of an r^2 within 0.003 bins of an edge."""
+    import vdock
+    print("receptor types", list(types), flush=True)
+    xyz, _ = vdock.synth_receptor(700, 26.0, 3.0, 9)
+    xs = np.array([list(types)[i % len(types)] for i in range(len(xyz))], dtype=np.int32)
+    box = vdock.box_from_center([1.0, -2.0, 0.5], [5.5, 3.0, 4.2], 0.375)
+    module_ctx.set_receptor(xyz, xs)
+    module_ctx.grid_populate(box)
+    maps = module_ctx.grid_download()
+    b, e, n = box.as_tuple()
+    grid = orc.Grid(orc.Lut(), b, e, n)
+    grid.set_receptor(xyz.astype(np.float64), xs)
+    slack = grid.populate_with_slack(0.003)
+    ref = grid.maps()
+    assert (np.abs(maps - ref) <= 1e-4 * np.maximum(1.0, np.abs(ref)) + slack).all()

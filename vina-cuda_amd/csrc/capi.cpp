@@ -178,6 +178,7 @@ struct vd_ctx {
   double weights[6] = {-0.035579, -0.005156, 0.840245, -0.035069, -0.587439, 0.05846};
   vd::Precalculated pre;
   DevBuf<float> lut_rows, lutp;
+  uint32_t grid_meta[VD_XS_SIZE] = {};   // per receptor type, what its atoms carry to the grid kernel
   std::vector<double> rec_xyz;   // receptor coordinates as parsed (FP64)
   std::vector<int> rec_xs;
   // maps
@@ -295,7 +296,7 @@ void upload_lut(vd_ctx* c) {
   c->pre.build(c->weights);
   if (c->host_only) return;
   std::vector<float> rows, bins;
-  c->pre.grid_rows(rows);
+  c->pre.grid_rows(rows, c->grid_meta);
   c->pre.pair_bins(bins);
   c->lut_rows.ensure(rows.size());
   c->lutp.ensure(bins.size());
@@ -1265,7 +1266,7 @@ int vd_grid_populate(vd_ctx* c, const vd_box* box) {
       if (cidx[i] < 0) continue;
       float4 a;
       a.x = (float)(c->rec_xyz[3 * i] - org[0]); a.y = (float)(c->rec_xyz[3 * i + 1] - org[1]); a.z = (float)(c->rec_xyz[3 * i + 2] - org[2]);
-      uint32_t t = (uint32_t)c->rec_xs[i]; std::memcpy(&a.w, &t, 4);
+      std::memcpy(&a.w, &c->grid_meta[c->rec_xs[i]], 4);
       sorted[fill[cidx[i]]++] = a;
     }
     c->grid_atoms.ensure(sorted.size());
@@ -1274,7 +1275,7 @@ int vd_grid_populate(vd_ctx* c, const vd_box* box) {
     HIP_CHECK(hipMemcpyAsync(c->grid_cells.p, ranges.data(), ranges.size() * sizeof(int2), hipMemcpyHostToDevice, c->stream));
     c->maps.ensure((size_t)VD_XS_SIZE * c->gd.plane);
     HIP_CHECK(hipEventRecord(c->ev0, c->stream));
-    HIP_CHECK(vdl::launch_grid(c->grid_atoms.p, c->grid_cells.p, gcl, reinterpret_cast<const float4*>(c->lut_rows.p), c->maps.p,
+    HIP_CHECK(vdl::launch_grid(c->grid_atoms.p, c->grid_cells.p, gcl, c->lut_rows.p, c->maps.p,
                                c->gd, c->stream));
     HIP_CHECK(hipEventRecord(c->ev1, c->stream));
     HIP_CHECK(hipStreamSynchronize(c->stream));

@@ -157,18 +157,30 @@ void Precalculated::build(const double w[5]) {
     }
 }
 
-void Precalculated::grid_rows(std::vector<float>& out) const {
-  const size_t rows = (size_t)VD_XS_SIZE * VD_LUT_BINS;
-  out.assign(rows * VD_GRID_ROW + rows, 0.0f);
-  for (int t1 = 0; t1 < VD_XS_SIZE; ++t1)
+const int kGridTypes[2][VD_GRID_PER_HALF] = {VD_GRID_TYPES};
+// Br and S have one radius, Cl and N another; Met takes the hydrogen bond of an acceptor t1, as a
+// donor's value (P has its place in half 1 and never takes one)
+const int kGridPick[VD_GRID_CLASSES][VD_GRID_PER_HALF] = {{VD_GRID_PICK_PLAIN}, {VD_GRID_PICK_HYDROPHOBIC},
+                                                          {VD_GRID_PICK_BONDING}};
+
+void Precalculated::grid_rows(std::vector<float>& out, uint32_t meta[VD_XS_SIZE]) const {
+  out.clear();
+  for (int t1 = 0; t1 < VD_XS_SIZE; ++t1) {
+    const bool acc = xs_is_acceptor(t1), don = xs_is_donor(t1);
+    const int cls = xs_is_hydrophobic(t1) ? 1 : acc || don ? 2 : 0;
+    const int half = VD_GRID_HALF(cls);
+    meta[t1] = (uint32_t)(out.size() / 4) | (uint32_t)cls << 24 | (don ? VD_GRID_DONOR : 0u);
     for (int b = 0; b < VD_LUT_BINS; ++b) {
-      const size_t r = (size_t)t1 * VD_LUT_BINS + b;
-      for (int t2 = 0; t2 < VD_XS_SIZE; ++t2) {
-        const float v = (float)fast[(size_t)type_pair_index(t1, t2) * VD_LUT_BINS + b];
-        if (t2 < VD_GRID_ROW) out[r * VD_GRID_ROW + t2] = v;
-        else out[rows * VD_GRID_ROW + r] = v;
-      }
+      const size_t row = out.size();
+      out.resize(row + 2 * half, 0.0f);
+      for (int h = 0; h < 2; ++h)
+        for (int k = VD_GRID_PER_HALF - 1; k >= 0; --k)   // a value shared by several types is the first one's
+          if (kGridTypes[h][k] >= 0 && !(cls == 2 && k == 5))
+            out[row + h * half + kGridPick[cls][k]] = (float)fast[(size_t)type_pair_index(t1, kGridTypes[h][k]) * VD_LUT_BINS + b];
     }
+    while (out.size() % 4) out.push_back(0.0f);
+  }
+  out.resize(out.size() + 4, 0.0f);   // the kernel reads six floats of every half
 }
 
 namespace {

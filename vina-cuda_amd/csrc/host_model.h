@@ -39,6 +39,10 @@ inline int type_pair_index(int a, int b) { if (a > b) { int t = a; a = b; b = t;
 struct PairTableRows { uint8_t row[VD_NUM_TYPE_PAIRS]; std::vector<int> first; };
 const PairTableRows& pair_table_rows();
 
+// The halves of a map LUT row: the types of each, and the value each takes by class of t1.
+extern const int kGridTypes[2][VD_GRID_PER_HALF];
+extern const int kGridPick[VD_GRID_CLASSES][VD_GRID_PER_HALF];
+
 // Weighted sum of the five Vina terms for XS types t1, t2 at distance r.
 double score_terms(int t1, int t2, double r, const double w[5]);
 
@@ -47,10 +51,11 @@ struct Precalculated {
   std::vector<double> smooth_e, smooth_dor, fast;   // [153][VD_LUT_BINS]
   void build(const double w[5]);
   // FP32 device layouts:
-  //   grid rows  [t1][bin][VD_GRID_ROW]: fast value for t2 = 0..15, then the column [t1][bin] of t2 = 16
+  //   grid rows  the map LUT (vd_common.h, "Rows of the map LUT"); meta[t1] = what a receptor atom of
+  //              type t1 carries to the kernel: first 16-byte word of its rows | class << 24
   //   pair bins  [row][bin] = (e_i, dor_i), row 0 zero (pair_table_rows); the 16 bytes at bin i are the interpolation quad
   //              (e_i, dor_i, e_{i+1}, dor_{i+1})
-  void grid_rows(std::vector<float>& out) const;
+  void grid_rows(std::vector<float>& out, uint32_t meta[VD_XS_SIZE]) const;
   void pair_bins(std::vector<float>& out) const;
   // the same rows and layout in FP64
   void pair_bins(std::vector<double>& out) const;

@@ -21,18 +21,22 @@ namespace {
 
 // ------------------------------------------------------------------------------------------
 // Grid maps.  A workgroup is one wavefront and owns a compact tile of points (x fastest), LP
-// lanes per point: lane l works on point l / LP and on the maps t2 = (l % LP) * 16/LP ..
-// +16/LP-1, the first lane of a point also on t2 = 16.  The receptor atoms that can reach the tile
+// lanes per point: lane l works on point l / LP and, with LP = 2, on half l % 2 of the map types
+// (with LP = 1 on both).  The receptor atoms that can reach the tile
 // come from a host-built cell list (cells of VD_GCELL A over the box grown by the 8 A cutoff, one
 // contiguous atom range per x-row of cells).  Each range is read 64 atoms at a time, one per lane
 // in a single coalesced load; a ballot of the lanes whose atom lies within the cutoff of the tile
 // box lists the atoms worth a pass, and the loop takes them in index order (GU per pass, all their
 // table reads in flight before any is added), reading each atom from its lane with readlane.  For
-// every atom within the cutoff of a point, one 16-float row of the map LUT (rows indexed
-// [t1][bin]) and one value of the column after the rows give the contribution to all 17 maps;
-// the LP lanes of the point read the row's 16-byte chunks side by side, so one load instruction
-// fetches whole rows of 64 / LP points, one cache line each.  Every point adds its atoms in the
+// every atom within the cutoff of a point, one row of the map LUT gives the contribution to all 17
+// maps: 4 values per half for a receptor type that neither is hydrophobic nor bonds, up to 6 for the
+// others, 16 and 8 bytes per lane.  Every point adds its atoms in the
 // order of the cell list, whatever the tile shape or LP, so neither changes a map value.
+// What bounds it is the L2's delivery to the L1s (a wavefront's 32 points read 32 rows far apart:
+// 4e7 requests at 81^3, some 20 TB/s), with the vector units 70 % busy.  Rows of all 17 values (68
+// bytes) took 232 us at 81^3 and 1.91 ms at 188^3, these 202 us and 1.64 ms; one lane per point
+// 236 us and 1.79 ms, four atoms per pass 224 us and 1.79 ms, loads not masked by the cutoff 210 us
+// and 1.70 ms.
 constexpr int GU = 2;   // receptor atoms per pass of the grid kernel's loop
 
 __device__ __forceinline__ float lane_f(float v, int j) {
@@ -42,17 +46,50 @@ __device__ __forceinline__ float lane_f(float v, int j) {
 template <int LP> struct GridTile {
   static constexpr int NP = 64 / LP;                 // points per wavefront
   static constexpr int TX = 4, TY = NP >= 32 ? 4 : 2, TZ = NP / (TX * TY);
-  static constexpr int K = VD_GRID_ROW / LP;         // row values per lane
-  static constexpr int CH = K / 4;                   // 16-byte chunks per lane
+  static constexpr int H = 2 / LP;                   // halves per lane
 };
+
+// One lane's half of a row, and its addition to the lane's sums: acc[k] += value of index pick k.
+struct HalfRow { float4 a; float2 b; };
+template <int I> __device__ __forceinline__ float value(const HalfRow& v) {
+  if constexpr (I == 0) return v.a.x;
+  else if constexpr (I == 1) return v.a.y;
+  else if constexpr (I == 2) return v.a.z;
+  else if constexpr (I == 3) return v.a.w;
+  else if constexpr (I == 4) return v.b.x;
+  else return v.b.y;
+}
+struct HalfSums { float s0, s1, s2, s3, s4, s5, s6, s7, s8; };
+template <int P0, int P1, int P2, int P3, int P4, int P5, int P6, int P7, int P8>
+__device__ __forceinline__ void add_picked(HalfSums& s, const HalfRow v, float v5) {
+  s.s0 += value<P0>(v); s.s1 += value<P1>(v); s.s2 += value<P2>(v);
+  s.s3 += value<P3>(v); s.s4 += value<P4>(v); s.s5 += v5;
+  s.s6 += value<P6>(v); s.s7 += value<P7>(v); s.s8 += value<P8>(v);
+}
+// The classes are uniform branches of nine additions each.  The empty asm statements keep the
+// additions in their branches (merged behind them, they took up to eleven register moves).
+#define VD_KEEP(text)   asm volatile(text : "+v"(s.s0), "+v"(s.s1), "+v"(s.s2), "+v"(s.s3), "+v"(s.s4), "+v"(s.s5), "+v"(s.s6), "+v"(s.s7), "+v"(s.s8))
+__device__ __forceinline__ void add_row(uint32_t meta, HalfSums& s, const HalfRow v) {
+  const uint32_t cls = (meta >> 24) & 3u;
+  if (cls == 0) {
+    add_picked<VD_GRID_PICK_PLAIN>(s, v, v.a.y);
+    VD_KEEP("; plain");
+  } else if (cls == 1) {
+    add_picked<VD_GRID_PICK_HYDROPHOBIC>(s, v, v.a.z);
+    VD_KEEP("; hydrophobic");
+  } else {
+    add_picked<VD_GRID_PICK_BONDING>(s, v, (meta & VD_GRID_DONOR) ? v.a.w : v.a.z);
+    VD_KEEP("; bonding");
+  }
+}
+#undef VD_KEEP
 
 template <int LP>
 __global__ __launch_bounds__(64) void vd_grid_kernel(const float4* __restrict__ atoms, const int2* __restrict__ cells,
-                                                     GridCells gc, const float4* __restrict__ lut_rows,
-                                                     const float* __restrict__ lut_last, float* __restrict__ maps,
+                                                     GridCells gc, const float* __restrict__ lut, float* __restrict__ maps,
                                                      vd_grid_desc gd, int tiles_x, int tiles_y) {
   using T = GridTile<LP>;
-  constexpr int TX = T::TX, TY = T::TY, TZ = T::TZ, K = T::K, CH = T::CH;
+  constexpr int TX = T::TX, TY = T::TY, TZ = T::TZ, H = T::H;
   const int tile = blockIdx.x, lane = threadIdx.x;
   const int pt = lane / LP, q = lane % LP;
   const int tx0 = (tile % tiles_x) * TX, ty0 = ((tile / tiles_x) % tiles_y) * TY, tz0 = (tile / (tiles_x * tiles_y)) * TZ;
@@ -71,10 +108,7 @@ __global__ __launch_bounds__(64) void vd_grid_kernel(const float4* __restrict__ 
   const int cx0 = max(0, (int)floorf((lo_x - cut) * inv)), cx1 = min(gc.n[0] - 1, (int)floorf((hi_x + cut) * inv));
   const int cy0 = max(0, (int)floorf((lo_y - cut) * inv)), cy1 = min(gc.n[1] - 1, (int)floorf((hi_y + cut) * inv));
   const int cz0 = max(0, (int)floorf((lo_z - cut) * inv)), cz1 = min(gc.n[2] - 1, (int)floorf((hi_z + cut) * inv));
-  const bool first = q == 0;   // this lane also sums t2 = 16
-  float acc[K], acc16 = 0.0f;
-#pragma unroll
-  for (int t = 0; t < K; ++t) acc[t] = 0.0f;
+  HalfSums acc[H] = {};
   for (int cz = cz0; cz <= cz1; ++cz)
     for (int cy = cy0; cy <= cy1; ++cy) {
       const int row = (cz * gc.n[1] + cy) * gc.n[0];
@@ -97,43 +131,51 @@ __global__ __launch_bounds__(64) void vd_grid_kernel(const float4* __restrict__ 
             j[u] = has[u] ? __builtin_ctzll(todo) : 0;
             todo &= todo - 1;
           }
-          float4 rv[GU][CH];
-          float last[GU];
+          HalfRow v[GU][H];
+          uint32_t meta[GU];
           bool use[GU];
 #pragma unroll
           for (int u = 0; u < GU; ++u) {
             const float ax = lane_f(mine.x, j[u]), ay = lane_f(mine.y, j[u]), az = lane_f(mine.z, j[u]);
-            const int t1 = __builtin_amdgcn_readlane(__float_as_int(mine.w), j[u]);
+            meta[u] = (uint32_t)__builtin_amdgcn_readlane(__float_as_int(mine.w), j[u]);
+            const float* rows = lut + 4 * (meta[u] & 0xFFFFFFu);
             const float dx = ax - px, dy = ay - py, dz = az - pz;
             const float r2 = dx * dx + dy * dy + dz * dz;
             use[u] = has[u] && inside && r2 <= VD_CUTOFF_SQR;
-            last[u] = 0.0f;
             if (use[u]) {
-              const size_t r = (size_t)t1 * VD_LUT_BINS + (int)(VD_LUT_FACTOR * r2);
-              const float4* rw = lut_rows + r * (VD_GRID_ROW / 4) + q * CH;
+              // a plain row's lane reads past its own 16 bytes; the table ends with room for that
+              const uint32_t bin = (uint32_t)(VD_LUT_FACTOR * r2);
+              const uint32_t half = ((meta[u] >> 24) & 3u) == 0 ? 4u : 6u;   // uniform
 #pragma unroll
-              for (int c = 0; c < CH; ++c) rv[u][c] = rw[c];
-              if (first) last[u] = lut_last[r];
+              for (int h = 0; h < H; ++h) {
+                const float* r = rows + (__umul24(bin, 2 * half) + half * (LP == 2 ? q : h));
+                v[u][h].a = *reinterpret_cast<const float4*>(r);
+                v[u][h].b = *reinterpret_cast<const float2*>(r + 4);
+              }
             }
           }
 #pragma unroll
           for (int u = 0; u < GU; ++u) {
             if (!use[u]) continue;
 #pragma unroll
-            for (int c = 0; c < CH; ++c) {
-              acc[4 * c] += rv[u][c].x; acc[4 * c + 1] += rv[u][c].y;
-              acc[4 * c + 2] += rv[u][c].z; acc[4 * c + 3] += rv[u][c].w;
-            }
-            acc16 += last[u];
+            for (int h = 0; h < H; ++h) add_row(meta[u], acc[h], v[u][h]);
           }
         }
       }
     }
   if (inside) {
     const size_t o = (size_t)x + (size_t)gd.dim[0] * ((size_t)y + (size_t)gd.dim[1] * z);
+    constexpr int types[2][VD_GRID_PER_HALF] = {VD_GRID_TYPES};
 #pragma unroll
-    for (int t = 0; t < K; ++t) maps[(size_t)(q * K + t) * gd.plane + o] = acc[t];
-    if (first) maps[(size_t)VD_GRID_ROW * gd.plane + o] = acc16;
+    for (int h = 0; h < H; ++h) {
+      const HalfSums& s = acc[h];
+      const float sum[VD_GRID_PER_HALF] = {s.s0, s.s1, s.s2, s.s3, s.s4, s.s5, s.s6, s.s7, s.s8};
+#pragma unroll
+      for (int k = 0; k < VD_GRID_PER_HALF; ++k) {
+        const int t = LP == 1 ? types[h][k] : q ? types[1][k] : types[0][k];
+        if (t >= 0) maps[(size_t)t * gd.plane + o] = sum[k];
+      }
+    }
   }
 }
 
@@ -677,13 +719,12 @@ int mc_lds_bytes(int G, int Amax, int Nmax, int dense) {
 // Lanes per grid point of the grid kernel.
 constexpr int kGridLanesPerPoint = 2;
 
-hipError_t launch_grid(const float4* atoms, const int2* cells, const GridCells& gc, const float4* lut_rows, float* maps,
+hipError_t launch_grid(const float4* atoms, const int2* cells, const GridCells& gc, const float* lut, float* maps,
                        const vd_grid_desc& gd, hipStream_t s) {
   using T = GridTile<kGridLanesPerPoint>;
   const int tx = (gd.dim[0] + T::TX - 1) / T::TX, ty = (gd.dim[1] + T::TY - 1) / T::TY, tz = (gd.dim[2] + T::TZ - 1) / T::TZ;
-  const float* lut_last = reinterpret_cast<const float*>(lut_rows) + (size_t)VD_XS_SIZE * VD_LUT_BINS * VD_GRID_ROW;
-  hipLaunchKernelGGL(vd_grid_kernel<kGridLanesPerPoint>, dim3(tx * ty * tz), dim3(64), 0, s, atoms, cells, gc, lut_rows,
-                     lut_last, maps, gd, tx, ty);
+  hipLaunchKernelGGL(vd_grid_kernel<kGridLanesPerPoint>, dim3(tx * ty * tz), dim3(64), 0, s, atoms, cells, gc, lut, maps, gd,
+                     tx, ty);
   return hipGetLastError();
 }
 

@@ -11,9 +11,22 @@
 #define VD_LUT_FACTOR 32.0f
 #define VD_CUTOFF_SQR 64.0f
 #define VD_ZERO_QUAD 0               // first entry of the pair table's all-zero row, row 0
-#define VD_GRID_ROW 16               // per (t1, bin) row of the map LUT: the values of t2 = 0..15 (64 B,
-                                     // four aligned 16-byte loads); the t2 = 16 values follow all rows
-                                     // as a [t1][bin] column
+// Rows of the map LUT.  For one receptor type t1 the 17 map types take few different values: they
+// differ by radius, by the hydrophobic match (only if t1 is hydrophobic) and by the hydrogen bond
+// (only if t1 is a donor or an acceptor).  A row (t1, bin) holds each value once, in two halves of
+// VD_GRID_HALF(class) floats, for the types kGridTypes[half]; type k of either half takes the half's
+// value of index VD_GRID_PICK_<class>[k].
+#define VD_GRID_CLASSES 3            // of t1: 0 plain, 1 hydrophobic, 2 bonding (donor or acceptor)
+#define VD_GRID_PER_HALF 9           // types per half (half 1 has 8: its entry 7 is none, -1)
+#define VD_GRID_HALF(cls) ((cls) == 0 ? 4 : 6)
+// the types of the halves, by XS number
+#define VD_GRID_TYPES {0, 1, 2, 3, 4, 5, 12, 13, 16}, {14, 10, 6, 7, 8, 9, 15, -1, 11}
+#define VD_GRID_PICK_PLAIN 0, 0, 1, 1, 1, 1, 2, 1, 3         // C N F Met / S O I P
+#define VD_GRID_PICK_HYDROPHOBIC 0, 1, 2, 2, 2, 2, 3, 4, 5   // C_H C_P N F Cl Met / Br S O I - P
+// bonding: C N_P N_D N_A F Met / S O_P O_D O_A I P; N_DA and O_DA bond with any t1 of the class: they
+// take N_A's and O_A's value if t1 is a donor, else N_D's and O_D's
+#define VD_GRID_PICK_BONDING 0, 0, 1, 2, 3, 3, 4, 1, 5
+#define VD_GRID_DONOR 0x80000000u    // bit of meta: t1 is a donor
 #define VD_MAX_ATOMS 255             // per ligand: atom indices are 8-bit fields of the pair words and node
                                      // atom ranges (the reference caps at 128, MAX_NUM_OF_ATOMS, V11/inc/kernel2.h:35)
 #define VD_MAX_NODES 64              // rigid nodes (torsions + 1)
