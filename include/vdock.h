@@ -160,7 +160,8 @@ typedef struct {
 /* One MC kernel launch of the last vd_dock / vd_dock_batch / vd_dock_batch_plain call (the
  * autotuner's trial launches excluded), in launch order.  The kernel is
  * vd_mc_kernel<lanes_per_chain, mode, waves_per_simd>; mode 0 dense BFGS, 1 RILC-BFGS,
- * 2 RILC-BFGS with the QuickVina2 history.  eval_bytes = algorithmic bytes of its evaluations:
+ * 2 RILC-BFGS with the QuickVina2 history; a first record of lanes_per_chain 16 with one item per
+ * chain is vd_mc_wide_kernel<mode> (vd_set_class_overlap).  eval_bytes = algorithmic bytes of its evaluations:
  * per evaluation 32 B per heavy atom (eight map corners) and 16 B per intramolecular pair (one
  * interpolation quad of the pair table).  No counterpart in the reference (which prints only
  * per-ligand kernel times, V11/lib/main_procedure_cu.cpp:975-994); it serves the roofline measurement. */
@@ -179,8 +180,11 @@ int vd_last_launches(vd_ctx* ctx, int max, vd_launch* out);
  * at the same time, each on its own stream: the narrower class takes half of its resident blocks
  * per CU and the wider class fills the rest, so that a class whose waves mostly wait shares every
  * CU with one that keeps the vector units busy, and the wider class's waiting workgroups take
- * over the slots the other gives up when its queue runs dry.  Batches of one class, or of three
- * or more, run one class after the other.  on = 0: always one after the other.  No counterpart
+ * over the slots the other gives up when its queue runs dry.  Beside one or two classes, the
+ * heaviest 16-lane ligands of a batch, which would otherwise run on after the rest has ended, get a
+ * launch of their own at the same time, one chain per wavefront in the arithmetic of 16 lanes and
+ * with the same results (not under QuickVina-W, with graphs or with a launch shape of the caller's).
+ * Batches of three or more classes run one class after the other.  on = 0: always one after the other.  No counterpart
  * in the reference (one kernel_monte launch per ligand). */
 int vd_set_class_overlap(vd_ctx* ctx, int on);
 /* on = 1: vd_dock_batch runs as a captured hipGraph.  The first call for a set of ligands and

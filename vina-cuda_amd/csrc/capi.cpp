@@ -107,6 +107,7 @@ struct McSlot {
   std::vector<unsigned long long> h_evals;
   McArgs a{};
   int G = 0, W = 0, blocks = 0;
+  bool wide = false;                         // one chain per wavefront in 16-lane arithmetic
   bool persistent = false, timed = false, busy = false;
   vd_launch rec{};
   void release() {
@@ -451,11 +452,11 @@ vdk::EvalK make_evalk(vd_ctx* c, float v_intra, float v_inter, float slope) {
 
 // Ligand records for chain groups of G lanes.
 Packed pack(vd_ctx* c, int G, const std::vector<int>& ids, const std::vector<int>* depth = nullptr,
-            const std::vector<int>* bfgs = nullptr) {
+            const std::vector<int>* bfgs = nullptr, bool wide = false) {
   Packed pk;
   for (size_t k = 0; k < ids.size(); ++k) {
     const vd::Ligand& L = lig_at(c, ids[k]);
-    pk.headers.push_back(vd::pack_ligand(L, pk.blob, G));
+    pk.headers.push_back(vd::pack_ligand(L, pk.blob, G, wide));
     if (depth) pk.headers.back().search_depth = (*depth)[k];
     if (bfgs) pk.headers.back().bfgs_steps = (*bfgs)[k];
     pk.Amax = std::max(pk.Amax, (int)L.atoms.size());
@@ -505,7 +506,7 @@ int loosest_budget(int G, int W, int mode, int lds) {
 // the kernel on the slot's stream; mc_collect waits for it and reads its evaluation counts.
 void mc_prepare(vd_ctx* c, McSlot& s, int G, int W, Packed&& pk, std::vector<uint32_t>&& streams,
                 std::vector<int2>&& items, std::vector<longlong4>&& off, const vd_mc_consts& P, float* d_e,
-                float* d_conf, float* d_heavy, bool persistent, bool timed, double share = 1.0) {
+                float* d_conf, float* d_heavy, bool persistent, bool timed, double share = 1.0, bool wide = false) {
   // a launch left in flight by a call that failed part-way still reads this slot's host copies
   if (s.busy) { (void)hipStreamSynchronize(s.stream); s.busy = false; }
   s.pk = std::move(pk); s.h_streams = std::move(streams); s.h_items = std::move(items);
@@ -541,16 +542,18 @@ void mc_prepare(vd_ctx* c, McSlot& s, int G, int W, Packed&& pk, std::vector<uin
   a.out_e = d_e; a.out_conf = d_conf; a.out_heavy = d_heavy; a.out_off = s.offs.p;
   a.slot_evals = s.evals.p;
   a.Amax = s.pk.Amax; a.Nmax = s.pk.Nmax;
-  const int lds = vdl::mc_lds_bytes(G, s.pk.Amax, s.pk.Nmax, P.local_search == 0);
+  const int lds = wide ? vdl::wide_lds_bytes(s.pk.Amax, s.pk.Nmax, P.local_search == 0)
+                       : vdl::mc_lds_bytes(G, s.pk.Amax, s.pk.Nmax, P.local_search == 0);
   if (lds > c->lds_max)
     throw ArgError(VD_ERR_CAPACITY, "ligand too large for the LDS layout (" + std::to_string(lds) + " bytes of " +
                                         std::to_string(c->lds_max) + " per workgroup)");
   const int mode = mc_mode(P);
-  W = loosest_budget(G, W, mode, lds);
+  W = wide ? 2 : loosest_budget(G, W, mode, lds);
   int blocks = (int)s.h_items.size();
   if (persistent) {
     a.queue = s.queue.p;
-    const int per_cu = std::max(1, (int)std::ceil(share * vdl::max_resident_mc_blocks(G, W, mode, lds)));
+    const int resident = wide ? vdl::max_resident_wide_blocks(mode, lds) : vdl::max_resident_mc_blocks(G, W, mode, lds);
+    const int per_cu = std::max(1, (int)std::ceil(share * resident));
     blocks = std::min<long long>((long long)per_cu * c->n_cu, (long long)s.h_items.size());
     blocks = std::max(blocks, 1);
   }
@@ -558,11 +561,11 @@ void mc_prepare(vd_ctx* c, McSlot& s, int G, int W, Packed&& pk, std::vector<uin
     // one visited-history region per chain slot of every launched block (blocks keep their
     // slot for all the items they take from the queue)
     a.hist_stride = vdk::History::floats_per_chain(s.pk.Tmax, P.policy == VD_MC_QVINAW ? 5 : 10);
-    s.hist.ensure((size_t)blocks * (64 / G) * a.hist_stride);
+    s.hist.ensure((size_t)blocks * (wide ? 1 : 64 / G) * a.hist_stride);
     a.hist = s.hist.p;
   }
   if (P.policy == VD_MC_QVINAW) a.glob = s.glob.p;
-  s.G = G; s.W = W; s.blocks = blocks; s.persistent = persistent;
+  s.G = G; s.W = W; s.wide = wide; s.blocks = blocks; s.persistent = persistent;
   s.rec = vd_launch{};
   s.rec.lanes_per_chain = G; s.rec.waves_per_simd = W; s.rec.blocks = blocks; s.rec.items = (int)s.h_items.size();
   s.rec.ligands = (int)s.h_headers.size(); s.rec.persistent = persistent ? 1 : 0;
@@ -593,7 +596,7 @@ void mc_enqueue_copies(McSlot& s) {
 void mc_enqueue_kernel(McSlot& s) {
   hipStream_t st = s.stream;
   if (s.timed) HIP_CHECK(hipEventRecord(s.ev0, st));
-  HIP_CHECK(vdl::launch_mc(s.G, s.W, s.a, s.blocks, st));
+  HIP_CHECK(s.wide ? vdl::launch_mc_wide(s.a, s.blocks, st) : vdl::launch_mc(s.G, s.W, s.a, s.blocks, st));
   if (s.timed) HIP_CHECK(hipEventRecord(s.ev1, st));
   s.busy = true;
 }
@@ -622,7 +625,7 @@ void mc_collect(vd_ctx* c, McSlot& s, vd_stats* st, hipEvent_t base, bool add_ms
   if (st) {
     st->evals += rec.evals;
     st->blocks += s.blocks;
-    st->chains_per_wave = 64 / s.G;
+    st->chains_per_wave = s.wide ? 1 : 64 / s.G;
     if (add_ms) st->kernel_ms += rec.kernel_ms;
   }
 }
@@ -642,7 +645,7 @@ void run_mc(vd_ctx* c, int G, int W, const Packed& pk, const std::vector<uint32_
   mc_collect(c, s, st, nullptr);
 }
 
-struct LigPlan { int id, G, W, depth, bfgs, T, H, chains; };
+struct LigPlan { int id, G, W, depth, bfgs, T, H, chains; bool wide = false; };
 // single_launch: the ligand gets a launch of its own (vd_dock, the plain per-ligand loop).  Its
 // only parallelism is its chains, so unless they fill two waves per SIMD at the tuned width, it
 // runs one chain per wavefront, the most wavefronts such a launch can have.
@@ -1625,20 +1628,76 @@ int vd_dock_noalloc(vd_ctx* c, int id, const vd_dock_params* p, const float* d_i
 
 namespace {
 
-// The launch classes of a persistent batch: ligand indices per (lanes per chain, waves per SIMD).
-using Classes = std::map<std::pair<int, int>, std::vector<int>>;
+// The launch classes of a persistent batch: ligand indices per launch form, wide launches first.
+struct ClassKey {
+  int narrow, G, W;   // narrow: 0 for a wide launch; lanes per chain, waves per SIMD
+  bool operator<(const ClassKey& o) const { return std::tie(narrow, G, W) < std::tie(o.narrow, o.G, o.W); }
+};
+using Classes = std::map<ClassKey, std::vector<int>>;
 Classes batch_classes(const std::vector<LigPlan>& plans) {
   Classes classes;
-  for (size_t k = 0; k < plans.size(); ++k) classes[std::make_pair(plans[k].G, plans[k].W)].push_back((int)k);
+  for (size_t k = 0; k < plans.size(); ++k) classes[ClassKey{plans[k].wide ? 0 : 1, plans[k].G, plans[k].W}].push_back((int)k);
   return classes;
 }
 
-// Overlap applies to batches of exactly two classes.  Measured on the screening batch (a 16-lane
-// class whose waves mostly wait, a 64-lane class that keeps the vector units busy): 3 % shorter
-// steps.  With more classes it lost: on a 4,096-ligand batch of five classes a fourth stream
+// Estimated cost of a work item (the chains of one wavefront): steps x iterations x (atoms + pairs).
+double item_cost(const LigPlan& pl, int atoms, int pair_slots) { return (double)pl.depth * pl.bfgs * (atoms + 0.5 * pair_slots + 16); }
+
+// Marks the ligands of the 16-lane class that a batch docks wide: one chain per wavefront, in a
+// launch of its own beside the others, with the same results.  A chain of the 16-lane class runs its
+// evaluations one after the other, 32 us each for 69 atoms, and its wavefront with it; a wide one runs
+// them in a third of that, but a wavefront then carries one chain instead of four, and the batch's work
+// grows.  So only what would end the batch after the rest has kept the GPU full goes wide.
+//   rest    the launches' work at the rates at which they fill the GPU together, fitted on eleven
+//           screening batches of 256 to 1,024 ligands (within 4 %): 4.74e-8 ms per unit of a 16-lane
+//           item, a unit being steps x iterations x (atoms + half the pair slots + 146), and 9.2e-7 ms
+//           per step, iteration and evaluation microsecond of a 64-lane chain (on 256 CUs)
+//   item    7.6e-5 ms per unit by itself, 1.6 times that among others
+// Dense BFGS takes 2.5 times the rest's and 3.3 times the item's figure, which is nearly the same ratio.
+// An item goes wide when its own time passes 0.7 of the rest's: over 20 batches of 256 dense-BFGS
+// ligands 184 ms a batch without wide launches, 170, 169, 169 with the line at 0.6, 0.7, 0.8, and over
+// 21 of 512 ligands under QuickVina2 173 ms, 160, 161, 166 (0.7 is the best of both sets together).  Every
+// ligand of a small batch goes wide.  Kernels, ms, narrow -> wide: 3 ligands of 32 chains 5.1 -> 3.4,
+// 30 of 128 40 -> 25, 64 of 256 78 -> 50 (dense BFGS 172 -> 120), 128 of 256 88 -> 71.
+// Half of its residency for the wide launch, so that the narrow one's half fits beside it from the
+// start: with all of it, narrow wavefronts waited behind the 64-lane class's (256 ligands under
+// QuickVina2 189 ms instead of 144).  Not under QuickVina-W (whose chains share a buffer in the order
+// they run), not for a caller's own launch shape, not in captured graphs, and not where the launches
+// would run one after another (overlap off, or more than two classes beside the wide one).
+void wide_ligands(vd_ctx* c, std::vector<LigPlan>& plans, const vd_dock_params* p) {
+  if (p->policy == VD_MC_QVINAW || p->chains_per_wave != 0 || p->waves_per_simd != 0 || c->graphs_on ||
+      !c->overlap_classes || batch_classes(plans).size() > 2)
+    return;
+  double rest = 0;
+  std::vector<double> units(plans.size(), 0.0);
+  for (size_t k = 0; k < plans.size(); ++k) {
+    const LigPlan& pl = plans[k];
+    if (pl.G != 16 && pl.G != 64) return;
+    const vd::Ligand& L = lig_at(c, pl.id);
+    const double A = (double)L.atoms.size(), slots = (double)vd::pair_chunks(L, pl.G).size(), its = (double)pl.depth * pl.bfgs;
+    if (pl.G == 16) {
+      units[k] = its * (A + 0.5 * slots + 146.0);
+      rest += 4.74e-8 * units[k] * ((pl.chains + 3) / 4);
+    } else {
+      rest += 9.2e-7 * its * (5.0 + (A <= 64 ? 0.14 : 0.25) * slots / 64) * pl.chains;
+    }
+  }
+  rest *= 256.0 / std::max(1, c->n_cu);
+  for (size_t k = 0; k < plans.size(); ++k) {
+    const int A = (int)lig_at(c, plans[k].id).atoms.size();
+    if (plans[k].G == 16 && A > 16 && A <= vdk::kWideAtoms && 7.6e-5 * units[k] > 0.7 * rest) plans[k].wide = true;
+  }
+}
+
+// Overlap applies to batches of exactly two classes, besides a wide launch.  Measured on the
+// screening batch (a 16-lane class whose waves mostly wait, a 64-lane class that keeps the vector
+// units busy): 3 % shorter steps.  With more classes it lost: on a 4,096-ligand batch of five classes a fourth stream
 // shared a hardware queue with the third (four queues per process), and capped classes that
 // outlast the uncapped one keep half their CU slots empty to the end.
-bool overlap_of(const vd_ctx* c, const Classes& classes) { return c->overlap_classes && classes.size() == 2; }
+bool overlap_of(const vd_ctx* c, const Classes& classes) {
+  const size_t wide = !classes.empty() && classes.begin()->first.narrow == 0;
+  return c->overlap_classes && (classes.size() == 2 || (wide && classes.size() == 3));
+}
 
 // Host work of one class of a persistent batch -- its ligand records, launch tables and work items
 // in decreasing estimated cost -- prepared into launch slot s.  share: the fraction of its resident
@@ -1647,26 +1706,27 @@ bool overlap_of(const vd_ctx* c, const Classes& classes) { return c->overlap_cla
 // full grid, whose blocks that do not fit at first take over the CU slots the others give up when
 // their queues run dry.  Measured on the screening batch (16- and 64-lane classes): 0.5 to 0.75 of
 // the residency are equally good, below 0.4 the first class runs too long.
-void prepare_class(vd_ctx* c, McSlot& s, int G, int W, const std::vector<int>& ks, const std::vector<LigPlan>& plans,
+void prepare_class(vd_ctx* c, McSlot& s, const ClassKey& key, const std::vector<int>& ks, const std::vector<LigPlan>& plans,
                    const vd_dock_params* p, double share) {
+  const int G = key.G, W = key.W;
+  const bool wide = key.narrow == 0;
   std::vector<int> lig_ids, dv, bv;
   for (int k : ks) { lig_ids.push_back(plans[k].id); dv.push_back(plans[k].depth); bv.push_back(plans[k].bfgs); }
-  Packed pk = pack(c, G, lig_ids, &dv, &bv);
+  Packed pk = pack(c, G, lig_ids, &dv, &bv, wide);
   std::vector<uint32_t> streams;
   std::vector<longlong4> off;
   for (int k : ks) { streams.push_back((uint32_t)plans[k].id); off.push_back(c->batch.off[k]); }
-  // cost estimate per chain: steps x iterations x (atoms + pairs)
   std::vector<std::pair<double, int>> order;
   for (size_t s = 0; s < ks.size(); ++s)
-    order.push_back({-(double)dv[s] * bv[s] * (pk.headers[s].n_atoms + 0.5 * pk.headers[s].n_chunks * G + 16), (int)s});
+    order.push_back({-item_cost(plans[ks[s]], pk.headers[s].n_atoms, pk.headers[s].n_chunks * G), (int)s});
   std::stable_sort(order.begin(), order.end());
-  const int cpw = 64 / G;
+  const int cpw = wide ? 1 : 64 / G;
   std::vector<int2> items;
   for (auto& o : order)
     for (int c0 = 0; c0 < p->chains; c0 += cpw) items.push_back(make_int2(o.second, c0));
   if (!s.stream) s.stream = device_stream(c->device, (int)(&s - c->mc));
   mc_prepare(c, s, G, W, std::move(pk), std::move(streams), std::move(items), std::move(off), make_consts(c, p, 0, 0),
-             c->batch.e.p, c->batch.conf.p, c->batch.heavy.p, true, true, share);
+             c->batch.e.p, c->batch.conf.p, c->batch.heavy.p, true, true, share, wide);
 }
 
 // Every device buffer of a launch slot that a captured graph reads or writes.  DevBuf::ensure
@@ -1819,7 +1879,7 @@ bool graph_dock(vd_ctx* c, const std::vector<int>& ids, const std::vector<LigPla
     int slot = 0;
     for (auto& cl : classes) {
       const bool last = std::next(classes.find(cl.first)) == classes.end();
-      prepare_class(c, c->mc[slot++], cl.first.first, cl.first.second, cl.second, plans, p, (overlap && !last) ? 0.5 : 1.0);
+      prepare_class(c, c->mc[slot++], cl.first, cl.second, plans, p, (overlap && !last) ? 0.5 : 1.0);
     }
     g = capture_batch(c, classes, overlap);
     g->ids = ids; g->p = key; g->shapes = shapes; g->overlap = overlap; g->outs = outs;
@@ -1899,6 +1959,7 @@ static int dock_many(vd_ctx* c, int n, const int* ids, const vd_dock_params* p, 
     // one persistent launch per (group width, register budget) class; items ordered by decreasing
     // estimated cost.  With class overlap the launches are all prepared first (buffer growth may
     // synchronise the device), then enqueued on one stream each, then collected.
+    wide_ligands(c, plans, p);
     const Classes classes = batch_classes(plans);
     const bool overlap = overlap_of(c, classes);
     if (c->graphs_on && graph_dock(c, std::vector<int>(ids, ids + n), plans, classes, p, st)) return;
@@ -1922,7 +1983,7 @@ static int dock_many(vd_ctx* c, int n, const int* ids, const vd_dock_params* p, 
     for (auto& cl : classes) {
       if (used == (overlap ? kMcSlots : 1)) flush();
       const bool last = std::next(classes.find(cl.first)) == classes.end();
-      prepare_class(c, c->mc[used], cl.first.first, cl.first.second, cl.second, plans, p, (overlap && !last) ? 0.5 : 1.0);
+      prepare_class(c, c->mc[used], cl.first, cl.second, plans, p, (overlap && !last) ? 0.5 : 1.0);
       ++used;
     }
     flush();

@@ -170,13 +170,14 @@ struct LigView {               // one ligand, staged in LDS for the wave
   const float4* node_o;        // N: rel_origin xyz + bits (parent+1 | atom begin << 8 | atom end << 16)
   const float4* node_a;        // N: rel_axis xyz + subtree_end
   const uint4* pairs;          // C chunks of G pair words in groups of four, [group][lane][4], global
+  const uint2* ent;            // wide launches: slot words, [pass][atom], global
   int A, N, C, T, H, rounds;
   int rows;                    // 1: slot l of every chunk holds a pair whose first atom is l
 };
 struct Scratch {               // per chain, LDS
   float4* xyz;                 // A, coordinates relative to the root origin (w unused)
   float4* frc;                 // A, dE/dx (w unused)
-  float4* fx;                  // G + 1: pair-force exchange row (entry G stays zero)
+  float4* fx;                  // G + 1: pair-force exchange row (entry G stays zero); wide: 64 + 1
   float4* frame;               // 3N rows (R row, origin component)
   float4* nacc;                // 2N: per-node force and moment sums
   float* stash;                // per wave: conformations parked out of registers, [slot][field][lane]
@@ -211,6 +212,9 @@ __device__ __forceinline__ float mul_rn(float a, float b) {
 #pragma clang fp contract(off)
   return a * b;
 }
+
+// |v|^2, the same roundings wherever it is used
+__device__ __forceinline__ float norm2(float3 v) { return fmaf(v.z, v.z, fmaf(v.y, v.y, mul_rn(v.x, v.x))); }
 
 // Trilinear map value and derivative at p (grid::evaluate_aux, V11/lib/grid.cpp:50-167), from the
 // edge records of one type (cd0, cd01: records per x-row, per z-plane).
@@ -469,6 +473,87 @@ __device__ float pair_terms_scatter(const LigView& L, const Scratch& S, const Ev
   return e_intra;
 }
 
+// ---- Wide launches: one chain per wavefront with the arithmetic of a 16-lane group.
+// Four rows of 16 lanes carry the same chain.  What a 16-lane group does in turn -- atoms l, l + 16,
+// ...; chunk after chunk of pairs; the passes of the node scan -- the rows do side by side, and the
+// sums over them are taken in the order of the group's turns, so every number is the group's bit for
+// bit (a chain gives the same result in either launch).  Everything else (kinematics, tree sums, the
+// search) the rows do alike, on the same LDS areas.  A chain of the heaviest 16-lane ligands of a
+// batch thus ends in a third of the time, on lanes that would idle; see wide_ligands for when.
+constexpr int kWideAtoms = 128;   // two atoms per lane
+// The values of v in this lane's place of rows 0 to 3.
+__device__ __forceinline__ void row_values(float v, float (&r)[4]) {
+  const auto e = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  const auto a = __builtin_amdgcn_permlane32_swap(e[0], e[0], false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(e[1], e[1], false, false);
+  r[0] = __uint_as_float(a[0]); r[1] = __uint_as_float(b[0]); r[2] = __uint_as_float(a[1]); r[3] = __uint_as_float(b[1]);
+}
+// s + the rows' v, row by row (a row without a term passes 0, which leaves s: s is never -0)
+__device__ __forceinline__ float add_rows(float s, float v) {
+  float r[4];
+  row_values(v, r);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) s += r[k];
+  return s;
+}
+
+// Pair terms of a wide launch: row u takes chunk u of every pass of four.  Each pair's separation
+// and force factor go to its slot of the exchange row, from where the lanes that own its atoms add the
+// force in the order of the chunks, first atoms before second ones: the forces stay in registers,
+// with no read-modify-write of LDS per chunk.  A pass's table reads are issued a pass ahead.
+__device__ inline float pair_terms_wide(const LigView& L, const Scratch& S, const EvalK& K, int lane) {
+  const int groups = (L.C + 3) / 4, l = lane & 15, row = lane >> 4;
+  if (groups <= 0) return 0.0f;
+  const uint32_t* pw = reinterpret_cast<const uint32_t*>(L.pairs) + l * 4 + row;
+  const CurlK ck(K.v_intra);
+  const bool two = L.A > 64;               // wave-uniform
+  const int i0 = min(lane, L.A - 1), i1 = min(lane + 64, L.A - 1);
+  float4 f0 = S.frc[i0], f1 = two ? S.frc[i1] : make_float4(0, 0, 0, 0);
+  if (lane == 0) S.fx[64] = make_float4(0, 0, 0, 0);
+  float e_intra = 0.0f;
+  struct Pass { bool ok; float rx, ry, rz, rem; float4 q; uint2 s0, s1; } p, n;
+  uint32_t w_next = pw[0];
+  auto issue = [&](int cg, Pass& t) {
+    const uint32_t w = w_next;
+    if (cg + 1 < groups) w_next = pw[(cg + 1) * 64];
+    t.s0 = L.ent[cg * L.A + i0];
+    if (two) t.s1 = L.ent[cg * L.A + i1];
+    const bool has = w != VD_NO_PAIR;
+    const float4 pa = S.xyz[has ? (w & 255u) : 0u], pb = S.xyz[has ? ((w >> 8) & 255u) : 0u];
+    t.rx = pb.x - pa.x; t.ry = pb.y - pa.y; t.rz = pb.z - pa.z;
+    const float r2 = t.rx * t.rx + t.ry * t.ry + t.rz * t.rz;
+    t.ok = has && r2 < VD_CUTOFF_SQR;
+    const float rf = VD_LUT_FACTOR * r2;
+    t.rem = __builtin_amdgcn_fractf(rf);   // rf - trunc(rf), exact for rf >= 0
+    t.q = K.quad(t.ok ? (w >> 16) * (uint32_t)VD_LUT_BINS + (uint32_t)rf : (uint32_t)VD_ZERO_QUAD);
+  };
+  auto take = [&](float4& f, uint32_t s, bool second) {   // f -= / += the force of a slot
+    const float4 x = S.fx[s];
+    const float d = second ? x.w : -x.w;
+    f.x = fmaf(d, x.x, f.x); f.y = fmaf(d, x.y, f.y); f.z = fmaf(d, x.z, f.z);
+  };
+  auto take8 = [&](float4& f, uint2 s) {
+    take(f, s.x & 255u, false); take(f, (s.x >> 8) & 255u, true);
+    take(f, (s.x >> 16) & 255u, false); take(f, s.x >> 24, true);
+    take(f, s.y & 255u, false); take(f, (s.y >> 8) & 255u, true);
+    take(f, (s.y >> 16) & 255u, false); take(f, s.y >> 24, true);
+  };
+  issue(0, p);
+  for (int cg = 0; cg < groups; ++cg) {
+    if (cg + 1 < groups) issue(cg + 1, n);
+    float e, dor;
+    pair_term(p.q, p.rem, ck, e, dor);
+    S.fx[lane] = p.ok ? make_float4(p.rx, p.ry, p.rz, dor) : make_float4(0, 0, 0, 0);
+    e_intra = add_rows(e_intra, p.ok ? e : 0.0f);
+    take8(f0, p.s0);
+    if (two) take8(f1, p.s1);
+    p = n;
+  }
+  if (lane < L.A) S.frc[lane] = f0;
+  if (lane + 64 < L.A) S.frc[lane + 64] = f1;
+  return e_intra;
+}
+
 // Energy and gradient of one conformation per group (model::eval_deriv,
 // V11/lib/model.cpp:1324-1334; device form quasi_newton.cuh:1294-1339).
 // Returns e (group-uniform); g = this lane's gradient component.  rg (when given) receives the
@@ -476,15 +561,36 @@ __device__ float pair_terms_scatter(const LigView& L, const Scratch& S, const Ev
 // want(e) says whether the group's caller will look at the gradient of a conformation of energy e;
 // where no group of the wavefront does, the adjoint is left out and g is 0.
 struct AlwaysWant { __device__ bool operator()(float) const { return true; } };
-template <int G, class Want = AlwaysWant>
+template <int G, bool WIDE = false, class Want = AlwaysWant>
 __device__ float eval_deriv(const LigView& L, const Scratch& S, const EvalK& K, const Conf& c, int l, float& g,
                             float* rg = nullptr, Want want = Want()) {
   float3 ax, org;
+  const int lane = threadIdx.x & 63;
   kinematics<G>(L, S, c, l, ax, org);
   __syncthreads();
   // intermolecular term: trilinear maps (cache::eval_deriv, V11/lib/cache.cpp:73-88)
   const float3 prel = make_float3(c.px - K.gd.init[0], c.py - K.gd.init[1], c.pz - K.gd.init[2]);
   float e_inter = 0.0f, racc = 0.0f;
+  if constexpr (WIDE) {
+    for (int i0 = 0; i0 < L.A; i0 += 64) {
+      const int i = i0 + lane;
+      float ev = 0.0f, rv = 0.0f;
+      if (i < L.A) {
+        float3 d = make_float3(0, 0, 0);
+        uint32_t meta;
+        const float3 y = atom_position(L, S, i, meta);
+        const int xs = (meta >> 8) & 255;
+        if (xs < VD_XS_SIZE)
+          ev = map_eval(K.edges + xs * K.cplane, K.cd0, K.cd01, K.gd,
+                        make_float3(prel.x + y.x, prel.y + y.y, prel.z + y.z), K.slope, K.v_inter, d);
+        S.xyz[i] = make_float4(y.x, y.y, y.z, 0.0f);
+        S.frc[i] = make_float4(d.x, d.y, d.z, 0.0f);
+        if ((meta >> 16) & 1u) rv = norm2(y);
+      }
+      e_inter = add_rows(e_inter, ev);
+      racc = add_rows(racc, rv);
+    }
+  } else
   // two atoms per lane in flight: both sets of map reads are issued before either is consumed
   for (int i0 = l; i0 < L.A; i0 += 2 * G) {
     float3 d[2], y[2];
@@ -510,14 +616,16 @@ __device__ float eval_deriv(const LigView& L, const Scratch& S, const EvalK& K, 
         S.xyz[i] = make_float4(y[u].x, y[u].y, y[u].z, 0.0f);
         S.frc[i] = make_float4(d[u].x, d[u].y, d[u].z, 0.0f);
         e_inter += ev[u];
-        if (heavy[u]) racc += y[u].x * y[u].x + y[u].y * y[u].y + y[u].z * y[u].z;
+        if (heavy[u]) racc += norm2(y[u]);
       }
     }
   }
   if (rg) { const float acc = gsum<G>(racc); *rg = L.H > 0 ? sqrtf(acc / (float)L.H) : 0.0f; }
   __syncthreads();
   // intramolecular pairs (eval_interacting_pairs_deriv, V11/lib/model.cpp:1241-1259)
-  const float e_intra = L.rows ? pair_terms_rows<G>(L, S, K, l) : pair_terms_scatter<G>(L, S, K, l);
+  float e_intra;
+  if constexpr (WIDE) e_intra = pair_terms_wide(L, S, K, lane);
+  else e_intra = L.rows ? pair_terms_rows<G>(L, S, K, l) : pair_terms_scatter<G>(L, S, K, l);
   const float e_sum = gsum<G>(e_inter + e_intra);
   if (!__any(want(e_sum))) { g = 0.0f; return e_sum; }
   __syncthreads();
@@ -527,8 +635,8 @@ __device__ float eval_deriv(const LigView& L, const Scratch& S, const EvalK& K, 
   // record.  Atoms beyond G lanes take further passes, each adding in turn.
   if (l < L.N) { S.nacc[2 * l] = make_float4(0, 0, 0, 0); S.nacc[2 * l + 1] = make_float4(0, 0, 0, 0); }
   __syncthreads();
-  for (int i0 = 0; i0 < L.A; i0 += G) {
-    const int i = i0 + l;
+  for (int i0 = 0; i0 < L.A; i0 += WIDE ? 64 : G) {
+    const int i = i0 + (WIDE ? lane : l);
     float v[6] = {0, 0, 0, 0, 0, 0};
     int node = -1;
     if (i < L.A) {
@@ -539,11 +647,13 @@ __device__ float eval_deriv(const LigView& L, const Scratch& S, const EvalK& K, 
     }
     seg_scan<G>(v, node);
     const int next = __shfl_down(node, 1, G);
-    if (node >= 0 && (l == G - 1 || next != node)) {
-      float4 a = S.nacc[2 * node], b = S.nacc[2 * node + 1];
-      a.x += v[0]; a.y += v[1]; a.z += v[2]; b.x += v[3]; b.y += v[4]; b.z += v[5];
-      S.nacc[2 * node] = a; S.nacc[2 * node + 1] = b;
-    }
+    const bool last = node >= 0 && (l == G - 1 || next != node);
+    for (int r = 0; r < (WIDE ? 4 : 1); ++r)   // wide: the rows are the group's passes, in turn
+      if (last && (!WIDE || lane >> 4 == r)) {
+        float4 a = S.nacc[2 * node], b = S.nacc[2 * node + 1];
+        a.x += v[0]; a.y += v[1]; a.z += v[2]; b.x += v[3]; b.y += v[4]; b.z += v[5];
+        S.nacc[2 * node] = a; S.nacc[2 * node + 1] = b;
+      }
   }
   __syncthreads();
   // subtree sums: the subtree of node k is the preorder range [k, subtree_end_k); the torque

@@ -641,7 +641,7 @@ const std::vector<uint32_t>& pair_chunks(const Ligand& L, int G) {
   return out;
 }
 
-vd_lig_header pack_ligand(const Ligand& L, std::vector<float>& blob, int G) {
+vd_lig_header pack_ligand(const Ligand& L, std::vector<float>& blob, int G, bool wide) {
   auto pad16 = [&]() { while (blob.size() % 4) blob.push_back(0.f); };
   auto as_f = [](uint32_t u) { float f; std::memcpy(&f, &u, 4); return f; };
   vd_lig_header h;
@@ -712,6 +712,22 @@ vd_lig_header pack_ligand(const Ligand& L, std::vector<float>& blob, int G) {
         blob.push_back(as_f(ch < h.n_chunks ? words[(size_t)ch * G + l] : pad));
       }
   pad16();
+  if (wide) {
+    // per pass of four chunks and atom, eight bytes: for each chunk the pass's slot (chunk * 16 + slot)
+    // whose pair has the atom first, and the one whose pair has it second; 64 where there is none
+    h.off_ent = (int)blob.size();
+    std::vector<uint8_t> ent((size_t)groups * A * 8, 64);
+    for (int ch = 0; ch < h.n_chunks; ++ch)
+      for (int l = 0; l < G; ++l) {
+        const uint32_t w = pairs[(size_t)ch * G + l];
+        if (w == VD_NO_PAIR) continue;
+        uint8_t* pass = &ent[(size_t)(ch / 4) * A * 8];
+        pass[(w & 255) * 8 + 2 * (ch % 4)] = (uint8_t)(ch % 4 * G + l);
+        pass[((w >> 8) & 255) * 8 + 2 * (ch % 4) + 1] = (uint8_t)(ch % 4 * G + l);
+      }
+    for (size_t k = 0; k < ent.size(); k += 4) { float f; std::memcpy(&f, &ent[k], 4); blob.push_back(f); }
+    pad16();
+  }
   return h;
 }
 

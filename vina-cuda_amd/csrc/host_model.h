@@ -98,8 +98,9 @@ Ligand parse_ligand_pdbqt(const std::string& text);
 void parse_receptor_pdbqt(const std::string& text, std::vector<double>& xyz, std::vector<int>& xs);
 
 // Appends a ligand's packed record to a device blob (16-byte words), with its pairs chunked for
-// chain groups of G lanes; returns the header.
-vd_lig_header pack_ligand(const Ligand& L, std::vector<float>& blob, int G);
+// chain groups of G lanes; returns the header.  wide (G = 16): with the slot words of a launch that
+// gives each chain a whole wavefront.
+vd_lig_header pack_ligand(const Ligand& L, std::vector<float>& blob, int G, bool wide = false);
 
 // Synthetic inputs (recipes of the benchmark configurations).
 void synth_receptor(int n_atoms, double cube, double cavity_radius, uint64_t seed,

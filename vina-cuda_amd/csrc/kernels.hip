@@ -217,6 +217,10 @@ __host__ __device__ inline int lig_floats(int A, int N) { return 4 * A + 8 * N +
 __host__ __device__ inline int group_floats(int A, int N, int G, int dense) {
   return 12 * N + 8 * A + 4 * (G + 1) + (dense ? G * G + 2 * G : 0);
 }
+// a wide launch's one group: the exchange row has a slot per lane
+__host__ __device__ inline int wide_floats(int A, int N, int dense) {
+  return group_floats(A, N, 16, dense) + 4 * (64 - 16);
+}
 
 template <int G>
 __device__ __forceinline__ void stage_ligand(const float4* __restrict__ blob, const vd_lig_header& h, float* lds, int lane) {
@@ -241,6 +245,7 @@ __device__ __forceinline__ void make_views(const float4* __restrict__ blob, cons
   S.frc = S.xyz + Amax;
   S.fx = S.frc + Amax;
   H = reinterpret_cast<float*>(S.fx + G + 1);
+  L.ent = nullptr;
 }
 
 // Writes a chain's best energy, conformation and heavy-atom coordinates (call after
@@ -323,7 +328,8 @@ __device__ Conf initial_conf(const vd_mc_consts& P, uint32_t stream, uint32_t ch
 // History); 2 QuickVina-W gate (qvw_interesting) with its records: the searched start point, each
 // BFGS iteration's end point and the point where the search stops go to the chain's own buffer,
 // the search's last point to the ligand's global buffer (QVW/inc/cuda/quasi_newton.cuh:2236-2410).
-template <int G, int POL>
+// WIDE: the four rows of the wavefront carry one chain (G = 16; see pair_terms_wide).
+template <int G, int POL, bool WIDE = false>
 __device__ void mc_chain_flat(const LigView& L, const Scratch& S, const EvalK& K, const vd_mc_consts& P, int depth,
                               int max_steps, uint32_t stream, uint32_t chain, bool valid, int l, float* out_e,
                               float* out_conf, float* out_heavy, int& evals, History* hist, const GlobalHist* gh,
@@ -388,7 +394,7 @@ __device__ void mc_chain_flat(const LigView& L, const Scratch& S, const EvalK& K
     // 98 -> 83 ms, RILC-BFGS 59 -> 56.5 ms alone; four chains seldom all fail together (under 2 %).
     float ge, rge;
     bool decrease = false;
-    const float fe = eval_deriv<G>(L, S, K, xe, l, ge, &rge, [&](float e) {
+    const float fe = eval_deriv<G, WIDE>(L, S, K, xe, l, ge, &rge, [&](float e) {
       decrease = POL < 0 ? e - fxp < 1e-4f * stp * dn_pg : !(e > finit + stp * dgtest);
       return start || (trial && (decrease || count + 1 >= 10));
     });
@@ -520,7 +526,7 @@ __device__ void mc_chain_flat(const LigView& L, const Scratch& S, const EvalK& K
   }
   const Conf best = stash_get<G>(S.stash, kSlotBest);
   set_coords<G>(L, S, best, l);
-  if (valid) write_chain<G>(L, S, best, best_e, chain, l, out_e, out_conf, out_heavy);
+  if (valid && (!WIDE || threadIdx.x < G)) write_chain<G>(L, S, best, best_e, chain, l, out_e, out_conf, out_heavy);
 }
 
 // W = minimum waves per SIMD the register allocation must allow (2 = unconstrained); a tuning knob:
@@ -574,6 +580,43 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W, 8))) void
       for (int gi = 0; gi < CPW; ++gi) sum += __shfl(evals, gi * G);
       if (lane == 0) atomicAdd(a.slot_evals + wi.x, (unsigned long long)sum);
     }
+  }
+}
+
+// A wide launch's chains: items are (ligand slot, chain).  Three waves per SIMD (168 registers, 184
+// bytes of spills) against two (217, none): large-box QuickVina2 batch of 200 ligands 149 against
+// 163 ms, dense BFGS of 96 the same.
+template <int MODE>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void vd_mc_wide_kernel(McArgs a) {
+  extern __shared__ float4 lds4[];
+  float* lds = reinterpret_cast<float*>(lds4);
+  const int lane = threadIdx.x, l = lane & 15;
+  int cur = -1;
+  for (int it = 0;; ++it) {
+    int item = 0;
+    if (lane == 0) item = atomicAdd(a.queue, 1);
+    item = __shfl(item, 0);
+    if (item >= a.n_items) break;
+    const int2 wi = a.items[item];
+    const vd_lig_header h = a.headers[wi.x];
+    if (wi.x != cur) {
+      __syncthreads();
+      stage_ligand<16>(a.blob, h, lds, lane);
+      __syncthreads();
+      cur = wi.x;
+    }
+    LigView L; Scratch S; float* H;
+    make_views<16>(a.blob, h, lds, a.Amax, a.Nmax, MODE == 0, 0, L, S, H);
+    H += 4 * (64 - 16);
+    L.ent = reinterpret_cast<const uint2*>(reinterpret_cast<const uint32_t*>(a.blob) + h.off_ent);
+    int evals = 0;
+    History hist;
+    if constexpr (MODE == 2) hist.init(a.hist + (long long)blockIdx.x * a.hist_stride, h.n_torsions);
+    GlobalHist gh{};
+    mc_chain_flat<16, MODE - 1, true>(L, S, a.K, a.P, h.search_depth, h.bfgs_steps, a.streams[wi.x], (uint32_t)wi.y, true, l,
+                                      a.out_e + a.out_off[wi.x].x, a.out_conf + a.out_off[wi.x].y,
+                                      a.out_heavy + a.out_off[wi.x].z, evals, &hist, &gh, nullptr, false, H);
+    if (lane == 0) atomicAdd(a.slot_evals + wi.x, (unsigned long long)evals);
   }
 }
 
@@ -745,6 +788,26 @@ hipError_t launch_eval(int G, const EvalArgs& a, int blocks, hipStream_t s) {
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
+}
+
+int wide_lds_bytes(int Amax, int Nmax, int dense) { return 4 * (lig_floats(Amax, Nmax) + wide_floats(Amax, Nmax, dense)); }
+
+hipError_t launch_mc_wide(const McArgs& a, int blocks, hipStream_t s) {
+  const int lds = wide_lds_bytes(a.Amax, a.Nmax, a.P.local_search == 0);
+  if (!a.queue || !a.items || (a.P.policy == 1 && !a.hist) || a.P.policy == 2) return hipErrorInvalidValue;
+  if (a.P.local_search == 0) hipLaunchKernelGGL(vd_mc_wide_kernel<0>, dim3(blocks), dim3(64), lds, s, a);
+  else if (a.P.policy == 1) hipLaunchKernelGGL(vd_mc_wide_kernel<2>, dim3(blocks), dim3(64), lds, s, a);
+  else hipLaunchKernelGGL(vd_mc_wide_kernel<1>, dim3(blocks), dim3(64), lds, s, a);
+  return hipGetLastError();
+}
+
+int max_resident_wide_blocks(int mode, int lds_bytes) {
+  int n = 0;
+  const hipError_t e =
+      mode == 0 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, vd_mc_wide_kernel<0>, 64, lds_bytes)
+      : mode == 2 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, vd_mc_wide_kernel<2>, 64, lds_bytes)
+                  : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, vd_mc_wide_kernel<1>, 64, lds_bytes);
+  return e == hipSuccess ? n : 0;
 }
 
 template <int MODE, int W>

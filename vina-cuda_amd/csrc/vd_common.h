@@ -61,6 +61,7 @@ struct vd_lig_header {
   int chunk_lanes;    // lanes per chain group the chunks were built for
   int pair_rows;      // 1: slot l of every chunk holds a pair whose first atom is l
   int reserved;
+  int off_ent;        // uint32 index of the slot words of a wide launch (see pair_terms_wide), 0: none
 };
 
 // Uniform-grid description of the 17 maps, plain FP32 layout map[t][z][y][x].
