@@ -40,3 +40,30 @@ def test_both_forms_agree_bit_for_bit(scene, heavy, tors, seed):
         assert np.array_equal(a[pick], b)
     key = [(r.e, r.e_inter, r.e_intra, r.inside) for r in few[2]]
     assert [key[k] for k in pick] == [(r.e, r.e_inter, r.e_intra, r.inside) for r in many[2]]
+
+
+@pytest.mark.parametrize("poses", [3, 400])
+def test_heaviest_first_keeps_every_pose_in_its_place(scene, poses):
+    """Workgroups start with the heaviest ligands' poses: a library gives what each ligand gives alone."""
+    import vdock
+    specs = [(9, 2, 21), (50, 9, 22), (1, 0, 23), (24, 3, 24), (33, 8, 25), (12, 4, 26)]
+    ids, confs = [], []
+    for s in specs:
+        ids.append(scene.add_ligand(vdock.synth_ligand(*s)))
+        T = scene.ligand_info(ids[-1]).n_torsions
+        rng = np.random.default_rng(s[2])
+        c = np.zeros((poses, 7 + T), dtype=np.float32)
+        c[:, :3] = rng.uniform(-6, 6, (poses, 3))
+        q = rng.normal(size=(poses, 4))
+        c[:, 3:7] = q / np.linalg.norm(q, axis=1, keepdims=True)
+        c[:, 7:] = rng.uniform(-np.pi, np.pi, (poses, T))
+        confs.append(c)
+    p = vdock.post_params(max_steps=3)
+    print("poses", poses, flush=True)
+    scene.postprocess(ids, confs, p)
+    both = [scene.post_results(k) for k in range(len(ids))]
+    for k, i in enumerate(ids):
+        scene.postprocess([i], [confs[k]], p)
+        modes, conf, xyz = scene.post_results(0)
+        assert [(m.pose, m.e, m.rmsd_lb, m.rmsd_ub) for m in modes] == [(m.pose, m.e, m.rmsd_lb, m.rmsd_ub) for m in both[k][0]]
+        assert np.array_equal(conf, both[k][1]) and np.array_equal(xyz, both[k][2])

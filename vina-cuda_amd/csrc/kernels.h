@@ -50,6 +50,7 @@ struct RefineArgs {
   const uint32_t* pairs;            // pair chunks of 64 words
   const uint16_t* ent;              // slots per (chunk, atom), several wavefronts per pose only
   const vdr::RefHeader* hdr;        // per ligand slot; max_steps = the step budget per stage
+  const int* order;                 // the pose of every workgroup
   const int* pose_lig;              // ligand slot per pose
   const long long* conf_off;        // per pose: offset of its conformation (7 + T doubles)
   const long long* coords_off;      // per pose: offset of its coordinates (3 A doubles)

@@ -669,7 +669,7 @@ __global__ __launch_bounds__(64) void vd_eval_kernel(EvalArgs a) {
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void vd_refine_kernel(RefineArgs a) {
   extern __shared__ double lds_d[];
-  const int pose = blockIdx.x, l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int pose = a.order[blockIdx.x], l = threadIdx.x & 63, w = threadIdx.x >> 6;
   const vdr::RefHeader h = a.hdr[a.pose_lig[pose]];
   vdr::Pose P;
   vdr::carve(P, lds_d, a.Amax, a.Nmax);
