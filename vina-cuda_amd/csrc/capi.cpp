@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <mutex>
 #include <numeric>
@@ -223,7 +224,8 @@ struct vd_ctx {
   // after the search: receptor cells of the direct evaluation (built on first use per box)
   bool nc_ready = false;
   vdr::NcD nck{};
-  DevBuf<double4> nc_atoms;
+  DevBuf<double4> nc_atoms, nc_sorted;       // the cells' lists; the receptor atoms they are taken from
+  DevBuf<long long> nc_bin;
   DevBuf<int> nc_start;
   DevBuf<double> lutd;                       // FP64 pair table of the refinement
   DevBuf<uint8_t> ref_rows;                  // its row of each XS type pair
@@ -777,7 +779,8 @@ namespace {
 // 2 A (n per axis exactly, so the cells tile it), and each cell lists every typed receptor atom
 // within the cutoff of its brick grown by 1e-3 A (a point the device's float arithmetic puts in
 // the cell is covered even when it lies a rounding error outside), as FP64 coordinates and XS
-// type.  Coarser cells when the lists would pass 2^26 entries (very large boxes).
+// type.  Coarser cells when the lists would pass 2^26 entries (very large boxes).  Bins of the cells'
+// size over the box grown by the cutoff spare most of the brick tests, which the device does.
 void build_nc(vd_ctx* c) {
   if (!c->maps_ready) throw ArgError(VD_ERR_ARG, "no search box: call vd_grid_populate first");
   if (c->rec_xs.empty()) throw ArgError(VD_ERR_ARG, "no receptor atoms: call vd_set_receptor first");
@@ -794,62 +797,58 @@ void build_nc(vd_ctx* c) {
     if (near) typed.push_back((int)i);
   }
   for (double target = 2.0;; target *= 1.5) {
-    int n[3]; double span[3], cs[3];
+    NcLists nl{};
+    double span[3];
     for (int k = 0; k < 3; ++k) {
       span[k] = b.end[k] - b.begin[k];
-      n[k] = std::max(1, (int)std::ceil(span[k] / target));
-      cs[k] = span[k] / n[k];
+      nl.n[k] = std::max(1, (int)std::ceil(span[k] / target));
+      nl.lo[k] = b.begin[k];
+      nl.cell[k] = span[k] / nl.n[k];
+      nl.nb[k] = (int)std::ceil((span[k] + 2 * grow) / nl.cell[k]) + 1;
+      nl.reach[k] = (int)std::ceil(2 * grow / nl.cell[k]) + 1;
     }
-    // bins of the same size over the box grown by the cutoff speed up the brick tests
-    int nb[3], reach[3];
-    for (int k = 0; k < 3; ++k) {
-      nb[k] = (int)std::ceil((span[k] + 2 * grow) / cs[k]) + 1;
-      reach[k] = (int)std::ceil(2 * grow / cs[k]) + 1;
-    }
-    std::vector<std::vector<int>> bins((size_t)nb[0] * nb[1] * nb[2]);
-    for (int i : typed) {
-      int bi[3];
+    nl.cut2 = grow * grow;
+    // the atoms by bin: stable counting sorts by x, y and z
+    std::vector<int> order(typed), next(typed.size());
+    std::vector<std::array<int, 3>> bin(c->rec_xs.size());
+    for (int i : typed)
       for (int k = 0; k < 3; ++k)
-        bi[k] = std::min(nb[k] - 1, std::max(0, (int)std::floor((c->rec_xyz[3 * i + k] - (b.begin[k] - grow)) / cs[k])));
-      bins[((size_t)bi[2] * nb[1] + bi[1]) * nb[0] + bi[0]].push_back(i);
+        bin[i][k] = std::min(nl.nb[k] - 1, std::max(0, (int)std::floor((c->rec_xyz[3 * i + k] - (b.begin[k] - grow)) / nl.cell[k])));
+    for (int k = 0; k < 3; ++k) {
+      std::vector<int> at(nl.nb[k] + 1, 0);
+      for (int i : order) ++at[bin[i][k] + 1];
+      for (int j = 0; j < nl.nb[k]; ++j) at[j + 1] += at[j];
+      for (int i : order) next[at[bin[i][k]]++] = i;
+      order.swap(next);
     }
-    const long long ncell = (long long)n[0] * n[1] * n[2];
+    std::vector<double4> atoms;
+    std::vector<long long> key;
+    for (int i : order) {
+      atoms.push_back(make_double4(c->rec_xyz[3 * i], c->rec_xyz[3 * i + 1], c->rec_xyz[3 * i + 2], (double)c->rec_xs[i]));
+      key.push_back(((long long)bin[i][2] * nl.nb[1] + bin[i][1]) * nl.nb[0] + bin[i][0]);
+    }
+    const long long ncell = (long long)nl.n[0] * nl.n[1] * nl.n[2];
     std::vector<int> start(ncell + 1, 0);
-    std::vector<double4> list;
-    bool too_big = false;
-    for (int z = 0; z < n[2] && !too_big; ++z)
-      for (int y = 0; y < n[1] && !too_big; ++y)
-        for (int x = 0; x < n[0]; ++x) {
-          const int id[3] = {x, y, z};
-          double lo[3], hi[3];
-          for (int k = 0; k < 3; ++k) { lo[k] = b.begin[k] + cs[k] * id[k]; hi[k] = b.begin[k] + cs[k] * (id[k] + 1); }
-          for (int bz = z; bz <= std::min(nb[2] - 1, z + reach[2]); ++bz)
-            for (int by = y; by <= std::min(nb[1] - 1, y + reach[1]); ++by)
-              for (int bx = x; bx <= std::min(nb[0] - 1, x + reach[0]); ++bx)
-                for (int i : bins[((size_t)bz * nb[1] + by) * nb[0] + bx]) {
-                  double dd = 0;
-                  for (int k = 0; k < 3; ++k) {
-                    const double v = c->rec_xyz[3 * i + k];
-                    const double d = v < lo[k] ? lo[k] - v : (v > hi[k] ? v - hi[k] : 0.0);
-                    dd += d * d;
-                  }
-                  if (dd >= grow * grow) continue;
-                  list.push_back(make_double4(c->rec_xyz[3 * i], c->rec_xyz[3 * i + 1], c->rec_xyz[3 * i + 2], (double)c->rec_xs[i]));
-                }
-          const long long cell = ((long long)z * n[1] + y) * n[0] + x;
-          start[cell + 1] = (int)list.size();
-          if (list.size() > (size_t)(1 << 26)) { too_big = true; break; }
-        }
-    if (too_big) continue;
-    c->nc_atoms.ensure(list.size());
-    c->nc_start.ensure(start.size());
-    if (!list.empty())
-      HIP_CHECK(hipMemcpy(c->nc_atoms.p, list.data(), list.size() * sizeof(double4), hipMemcpyHostToDevice));
-    HIP_CHECK(hipMemcpy(c->nc_start.p, start.data(), start.size() * sizeof(int), hipMemcpyHostToDevice));
+    c->nc_sorted.ensure(atoms.size()); c->nc_bin.ensure(key.size()); c->nc_start.ensure(start.size());
+    if (!atoms.empty()) {
+      HIP_CHECK(hipMemcpyAsync(c->nc_sorted.p, atoms.data(), atoms.size() * sizeof(double4), hipMemcpyHostToDevice, c->stream));
+      HIP_CHECK(hipMemcpyAsync(c->nc_bin.p, key.data(), key.size() * sizeof(long long), hipMemcpyHostToDevice, c->stream));
+    }
+    nl.atoms = c->nc_sorted.p; nl.bin = c->nc_bin.p; nl.n_atoms = (int)atoms.size();
+    HIP_CHECK(vdl::launch_nc_lists(false, nl, c->nc_start.p, nullptr, c->stream));
+    HIP_CHECK(hipMemcpyAsync(start.data() + 1, c->nc_start.p, ncell * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HIP_CHECK(hipStreamSynchronize(c->stream));
+    long long total = 0;
+    for (long long j = 1; j <= ncell && total <= (1 << 26); ++j) start[j] = (int)(total += start[j]);
+    if (total > (1 << 26)) continue;
+    c->nc_atoms.ensure(total);
+    HIP_CHECK(hipMemcpyAsync(c->nc_start.p, start.data(), start.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
+    if (total > 0) HIP_CHECK(vdl::launch_nc_lists(true, nl, c->nc_start.p, c->nc_atoms.p, c->stream));
+    HIP_CHECK(hipStreamSynchronize(c->stream));   // start goes out of scope
     vdr::NcD& k = c->nck;
     k.atoms = c->nc_atoms.p; k.start = c->nc_start.p;
     for (int j = 0; j < 3; ++j) {
-      k.lo[j] = b.begin[j]; k.hi[j] = b.end[j]; k.inv_cell[j] = n[j] / span[j]; k.n[j] = n[j];
+      k.lo[j] = b.begin[j]; k.hi[j] = b.end[j]; k.inv_cell[j] = nl.n[j] / span[j]; k.n[j] = nl.n[j];
     }
     c->nc_ready = true;
     return;
@@ -1160,7 +1159,7 @@ void vd_destroy(vd_ctx* c) {
   c->blob.release(); c->io_a.release(); c->io_b.release(); c->io_c.release();
   c->batch.e.release(); c->batch.conf.release(); c->batch.heavy.release();
   c->tune_e.release(); c->tune_conf.release(); c->tune_heavy.release();
-  c->nc_atoms.release(); c->nc_start.release(); c->ref_in.release(); c->ref_out.release(); c->ref_xyz.release();
+  c->nc_atoms.release(); c->nc_sorted.release(); c->nc_bin.release(); c->nc_start.release(); c->ref_in.release(); c->ref_out.release(); c->ref_xyz.release();
   c->ref_res.release(); c->ref_lig.release(); c->ref_order.release(); c->ref_evals.release(); c->ref_coff.release(); c->ref_xoff.release();
   c->lutd.release(); c->ref_rows.release(); c->ref_geo.release(); c->ref_ent.release(); c->ref_pairs.release(); c->ref_hdr.release();
   c->pin_eval.release(); c->eval_clock.release();

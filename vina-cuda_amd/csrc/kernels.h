@@ -63,7 +63,20 @@ struct RefineArgs {
   int Amax, Nmax, nmax;
 };
 
+// Receptor lists of the refinement's cells (vd_nc_lists_kernel): typed atoms near the box, sorted by
+// bin (x fastest) and, within a bin, by index; bins of the cells' size over the box grown by the cutoff.
+struct NcLists {
+  const double4* atoms;             // x, y, z, XS type
+  const long long* bin;             // per atom
+  int n_atoms;
+  double lo[3], cell[3];            // the box's corner, edges of a cell
+  int n[3], nb[3], reach[3];        // cells, bins; a cell's atoms lie in bins [id, id + reach] per axis
+  double cut2;                      // an atom closer than this (squared) to a cell's brick is listed
+};
+
 namespace vdl {
+// fill = false: the length of every cell's list to start[cell]; true: the lists, cell c's from start[c].
+hipError_t launch_nc_lists(bool fill, const NcLists& b, int* start, double4* list, hipStream_t s);
 int refine_lds_bytes(int waves, int Amax, int Nmax, int nmax);
 hipError_t launch_refine(int waves, const RefineArgs& a, int poses, hipStream_t s);   // waves per pose: 1 or 4
 int mc_lds_bytes(int G, int Amax, int Nmax, int dense);
