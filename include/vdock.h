@@ -195,7 +195,8 @@ int vd_set_class_overlap(vd_ctx* ctx, int on);
  * the same parameters replay it without packing or re-uploading anything on the host; the seed may
  * differ between calls (the graph's kernel nodes are updated).  A replay gives the results of the
  * eager path bit for bit.  Up to four captured batches are kept per context (least recently used
- * dropped); a batch whose buffers another call has grown since is captured again, and batches of
+ * dropped); a batch whose buffers another call has grown since, or whose box has changed, is
+ * captured again, and batches of
  * more than four classes run eagerly.  on = 0 (default) drops the captured graphs.  vd_last_launches
  * then gives each launch the whole graph's span.  No counterpart in the reference (one
  * kernel_monte launch per ligand, main_procedure_cu.cpp:527-956). */

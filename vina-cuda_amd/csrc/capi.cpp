@@ -146,7 +146,8 @@ struct GraphEntry {
   vd_dock_params p{};                 // seed zeroed
   std::vector<std::pair<int, int>> shapes;   // (lanes per chain, waves per SIMD) per ligand
   bool overlap = false;
-  std::vector<const void*> outs;     // the batch's result buffers at capture time
+  std::vector<const void*> outs;     // the batch's result buffers, the maps and the pair table at capture time
+  std::array<double, 9> box{};        // the box of the maps at capture time
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   uint32_t seed = 0;                  // the seed the instantiated graph holds
@@ -1876,12 +1877,14 @@ bool graph_dock(vd_ctx* c, const std::vector<int>& ids, const std::vector<LigPla
   key.seed = 0;
   std::vector<std::pair<int, int>> shapes;
   for (const LigPlan& pl : plans) shapes.push_back(std::make_pair(pl.G, pl.W));
-  const std::vector<const void*> outs{c->batch.e.p, c->batch.conf.p, c->batch.heavy.p};
+  const std::vector<const void*> outs{c->batch.e.p, c->batch.conf.p, c->batch.heavy.p, c->edges.p, c->lutp.p};
+  std::array<double, 9> box;
+  for (int k = 0; k < 3; ++k) { box[k] = c->box.begin[k]; box[3 + k] = c->box.end[k]; box[6 + k] = c->box.n[k]; }
   std::unique_ptr<GraphEntry> g;
   for (size_t k = 0; k < c->graphs.size(); ++k) {
     GraphEntry& e = *c->graphs[k];
     if (e.ids != ids || std::memcmp(&e.p, &key, sizeof key) != 0 || e.shapes != shapes || e.overlap != overlap) continue;
-    bool valid = e.outs == outs;
+    bool valid = e.outs == outs && e.box == box;
     for (const GraphClass& gc : e.cls) valid = valid && gc.ptrs == slot_ptrs(c->mc[gc.slot]);
     bool nodes = true;   // a kernel node to update per class
     for (const GraphClass& gc : e.cls) nodes = nodes && gc.node;
@@ -1896,7 +1899,7 @@ bool graph_dock(vd_ctx* c, const std::vector<int>& ids, const std::vector<LigPla
       prepare_class(c, c->mc[slot++], cl.first, cl.second, plans, p, (overlap && !last) ? 0.5 : 1.0);
     }
     g = capture_batch(c, classes, overlap);
-    g->ids = ids; g->p = key; g->shapes = shapes; g->overlap = overlap; g->outs = outs;
+    g->ids = ids; g->p = key; g->shapes = shapes; g->overlap = overlap; g->outs = outs; g->box = box;
   }
   // a launch that a failed eager call left in flight still uses its slot's buffers, which the
   // graph rewrites from another stream: wait for it first
