@@ -496,7 +496,6 @@ int mc_mode(const vd_mc_consts& P) {
 // A tighter register budget only pays when the LDS of a launch lets the extra waves in: the
 // loosest budget (waves per SIMD) that reaches the residency W reaches.
 int loosest_budget(int G, int W, int mode, int lds) {
-  if (mode == 0) return 2;
   const int occ = vdl::max_resident_mc_blocks(G, W, mode, lds);
   for (int w = 2; w < W; ++w)
     if (vdl::max_resident_mc_blocks(G, w, mode, lds) >= occ) return w;
@@ -660,7 +659,11 @@ LigPlan plan_for(vd_ctx* c, int id, const vd_dock_params* p, bool single_launch)
   pl.G = pick_group(c, L, p->chains_per_wave);
   if (single_launch && p->chains_per_wave == 0 && (long long)p->chains * pl.G / 64 < 8LL * std::max(c->n_cu, 1)) pl.G = 64;
   pl.W = p->waves_per_simd ? p->waves_per_simd : pick_waves(c, L, pl.G);
-  if (p->local_search != VD_LS_RILC_BFGS) pl.W = 2;
+  // Dense BFGS: three waves per SIMD (168 registers, 144 bytes of spills) for the 64-lane class of a batch
+  // (nine batches of 96 ligands 1,385 -> 1,344 ms with the 16-lane class at three as well, which alone
+  // loses: 123 -> 130 ms); a launch of one ligand rarely has the chains for a third (24 atoms, 2,048
+  // chains 18.4 -> 19.2 ms).
+  if (p->local_search != VD_LS_RILC_BFGS) pl.W = pl.G == 64 && !single_launch && p->waves_per_simd == 0 ? 3 : 2;
   const int rilc = p->local_search == VD_LS_RILC_BFGS;
   pl.depth = p->search_depth > 0 ? p->search_depth : heur_depth((int)L.atoms.size(), pl.T, rilc);
   pl.bfgs = p->bfgs_steps > 0 ? p->bfgs_steps : heur_bfgs((int)L.atoms.size(), rilc);
@@ -1668,10 +1671,11 @@ double item_cost(const LigPlan& pl, int atoms, int pair_slots) { return (double)
 //           item, a unit being steps x iterations x (atoms + half the pair slots + 146), and 9.2e-7 ms
 //           per step, iteration and evaluation microsecond of a 64-lane chain (on 256 CUs)
 //   item    7.6e-5 ms per unit by itself, 1.6 times that among others
-// Dense BFGS takes 2.5 times the rest's and 3.3 times the item's figure, which is nearly the same ratio.
-// An item goes wide when its own time passes 0.7 of the rest's: over 20 batches of 256 dense-BFGS
-// ligands 184 ms a batch without wide launches, 170, 169, 169 with the line at 0.6, 0.7, 0.8, and over
-// 21 of 512 ligands under QuickVina2 173 ms, 160, 161, 166 (0.7 is the best of both sets together).  Every
+// Dense BFGS takes 2.1 times the rest's and 3.3 times the item's figure.  An item goes wide when its own
+// time passes 0.7 (dense 0.48) of the rest's: over 21 batches of 512 ligands under QuickVina2 173 ms a
+// batch without wide launches, 160, 161, 166 with the line at 0.7, 0.6, 0.8; over 20 of 96 with dense
+// BFGS 181 ms without, 163, 147, 143 at 0.8, 0.6, 0.5, and over 12 of those 142, 142, 143, 145, 148 at
+// 0.45, 0.5, 0.4, 0.55, 0.3.  Every
 // ligand of a small batch goes wide.  Kernels, ms, narrow -> wide: 3 ligands of 32 chains 5.1 -> 3.4,
 // 30 of 128 40 -> 25, 64 of 256 78 -> 50 (dense BFGS 172 -> 120), 128 of 256 88 -> 71.
 // Half of its residency for the wide launch, so that the narrow one's half fits beside it from the
@@ -1698,9 +1702,10 @@ void wide_ligands(vd_ctx* c, std::vector<LigPlan>& plans, const vd_dock_params* 
     }
   }
   rest *= 256.0 / std::max(1, c->n_cu);
+  const double line = p->local_search == VD_LS_RILC_BFGS ? 0.7 : 0.48;
   for (size_t k = 0; k < plans.size(); ++k) {
     const int A = (int)lig_at(c, plans[k].id).atoms.size();
-    if (plans[k].G == 16 && A > 16 && A <= vdk::kWideAtoms && 7.6e-5 * units[k] > 0.7 * rest) plans[k].wide = true;
+    if (plans[k].G == 16 && A > 16 && A <= vdk::kWideAtoms && 7.6e-5 * units[k] > line * rest) plans[k].wide = true;
   }
 }
 

@@ -945,10 +945,10 @@ __device__ __attribute__((noinline)) bool qvw_interesting(const History& h, cons
 // lane k, position and orientation in lanes G-6 .. G-1; see the lane layout above).  Dimension c
 // of lane l is dense_dim(l); the lanes of the other G - n lanes hold zeros in every vector, so
 // their rows and columns of a G x G matrix would stay zero and only ever meet zeros: the matrix
-// keeps the n x n block, in the group's G x G area.  Lane l owns row dense_dim(l), kept
+// keeps the n x n block.  Lane l owns row dense_dim(l), kept
 // column-major (entry (c, c') at H[c' n + c]) so that the lanes' accesses at one c' are
 // consecutive words: no LDS bank conflicts (row-major, the lanes would hit one bank).  Sums run
-// over the dimensions in lane order.  vbuf (2 G floats after the G x G area) broadcasts vectors.
+// over the dimensions in lane order.  vbuf (2 G floats before the matrix) broadcasts vectors.
 // Every lane of the wavefront calls these (they fence); `on` selects the groups whose matrix is
 // written.
 template <int G> __device__ __forceinline__ int dense_dim(int l, int T) {

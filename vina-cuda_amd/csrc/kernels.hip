@@ -209,14 +209,19 @@ __global__ __launch_bounds__(256) void vd_edge_kernel(const float* __restrict__ 
 // ------------------------------------------------------------------------------------------
 // LDS layout of one wave: ligand (atoms 4A, node_o 4N, node_a 4N floats), the conformation
 // stash, then per chain group the node area 12N, xyz 4A, frc 4A, the pair-force exchange row
-// 4(G+1), and for dense BFGS H G*G + 2G.  The node area holds the frame rows from the kinematics
+// 4(G+1), and for dense BFGS 2G and H.  The node area holds the frame rows from the kinematics
 // until the atoms are placed, then the per-node force and moment sums of the adjoint (8N): an
 // evaluation reads the frames only in its intermolecular pass, which ends (with a fence) before
 // the sums are cleared.  The pair words stay in global memory (read once per evaluation,
 // coalesced, L2-resident).
 __host__ __device__ inline int lig_floats(int A, int N) { return 4 * A + 8 * N + kStashSlots * kStashSlotFloats; }
+// H is n x n for the n = 6 + torsions = 5 + nodes of the launch's largest ligand, to a multiple of four: with
+// G x G floats (16 KB of 64 lanes) seven 64-lane waves fitted a CU's LDS, which now takes all its
+// registers allow (4,096 chains of a 60-atom ligand with 16 torsions 154 -> 130 ms; nine batches of 96
+// ligands 1,470 -> 1,385 ms).
+__host__ __device__ inline int dense_floats(int N, int G) { return 2 * G + ((N + 5) * (N + 5) < G * G ? ((N + 5) * (N + 5) + 3) / 4 * 4 : G * G); }
 __host__ __device__ inline int group_floats(int A, int N, int G, int dense) {
-  return 12 * N + 8 * A + 4 * (G + 1) + (dense ? G * G + 2 * G : 0);
+  return 12 * N + 8 * A + 4 * (G + 1) + (dense ? dense_floats(N, G) : 0);
 }
 // a wide launch's one group: the exchange row has a slot per lane
 __host__ __device__ inline int wide_floats(int A, int N, int dense) {
@@ -337,6 +342,8 @@ __device__ void mc_chain_flat(const LigView& L, const Scratch& S, const EvalK& K
                               const float* given, bool ls_only, float* H) {
   const uint32_t k0 = P.seed, k1 = stream;
   const int n_ent = P.mutation_quirk ? (1 + L.T) : (2 + L.T);
+  float* const vbuf = H;   // dense BFGS: 2 G floats, then the matrix
+  H += 2 * G;
   enum { kMutate = 0, kStart = 1, kTrial = 2, kDone = 3 };
   // MC state; the current conformation lives in the stash (kSlotTmp)
   {
@@ -438,15 +445,15 @@ __device__ void mc_chain_flat(const LigView& L, const Scratch& S, const EvalK& K
         if (iter_end) { if (!(gnorm >= 1e-5f)) ls_done = true; else upd = true; }
         const float yy = gsum<G>(y * y), yp = gsum<G>(y * d);
         dense_set_diag<G>(H, stp * yp / yy, l, L.T, iter_end && dn_step == 0 && upd && fabsf(yy) > kEpsFl);   // first step: scaled diagonal
-        const float mhy = dense_minus_hv<G>(H, H + G * G, y, l, L.T);
+        const float mhy = dense_minus_hv<G>(H, vbuf, y, l, L.T);
         const float yhy = -gsum<G>(y * mhy);
         const float r = 1.0f / (stp * yp);
-        dense_update<G>(H, H + G * G, mhy, d, stp, r, yhy, iter_end && upd && !(stp * yp < kEpsFl), l, L.T);
+        dense_update<G>(H, vbuf, mhy, d, stp, r, yhy, iter_end && upd && !(stp * yp < kEpsFl), l, L.T);
         if (iter_end && !ls_done) { ++dn_step; if (dn_step < max_steps) begin = true; else ls_done = true; }
       }
       if (__any(begin)) {      // an iteration starts at x: p = -H g
         if (begin) { stash_put<G>(S.stash, kSlotPrev, x); gp = g; fxp = fx; prev_rg = x_rg; }
-        const float pn = dense_minus_hv<G>(H, H + G * G, g, l, L.T);
+        const float pn = dense_minus_hv<G>(H, vbuf, g, l, L.T);
         const float pg = gsum<G>(pn * g);
         if (begin) { d = pn; dn_pg = pg; stp = 1.0f; count = 0; phase = kTrial; }
       }
@@ -900,7 +907,7 @@ static hipError_t launch_mc_mode(int G, const McArgs& a, int blocks, int lds, hi
 
 hipError_t launch_mc(int G, int W, const McArgs& a, int blocks, hipStream_t s) {
   const int lds = mc_lds_bytes(G, a.Amax, a.Nmax, a.P.local_search == 0);
-  if (a.P.local_search == 0) return launch_mc_mode<0, 2>(G, a, blocks, lds, s);
+  if (a.P.local_search == 0) return W == 3 ? launch_mc_mode<0, 3>(G, a, blocks, lds, s) : launch_mc_mode<0, 2>(G, a, blocks, lds, s);
   if (a.P.policy == 1) {
     if (!a.hist) return hipErrorInvalidValue;
     switch (W) {
@@ -936,7 +943,7 @@ static const void* mc_fn_mode(int G) {
 
 // The instantiation launch_mc launches for (G, W, a), the same dispatch.
 const void* mc_kernel_fn(int G, int W, const McArgs& a) {
-  if (a.P.local_search == 0) return mc_fn_mode<0, 2>(G);
+  if (a.P.local_search == 0) return W == 3 ? mc_fn_mode<0, 3>(G) : mc_fn_mode<0, 2>(G);
   const int mode = a.P.policy == 1 ? 2 : a.P.policy == 2 ? 3 : 1;
   const int w = (W == 3 || W == 4) ? W : 2;
   switch (mode * 8 + w) {
@@ -1035,7 +1042,7 @@ static int occupancy(int G, int lds_bytes) {
 
 // mode: 0 dense BFGS, 1 RILC-BFGS, 2 RILC-BFGS with the QuickVina2 history, 3 with QuickVina-W's
 int max_resident_mc_blocks(int G, int W, int mode, int lds_bytes) {
-  if (mode == 0) return occupancy<0, 2>(G, lds_bytes);
+  if (mode == 0) return W == 3 ? occupancy<0, 3>(G, lds_bytes) : occupancy<0, 2>(G, lds_bytes);
   if (mode == 2) return W == 3 ? occupancy<2, 3>(G, lds_bytes) : W == 4 ? occupancy<2, 4>(G, lds_bytes) : occupancy<2, 2>(G, lds_bytes);
   if (mode == 3) return W == 3 ? occupancy<3, 3>(G, lds_bytes) : W == 4 ? occupancy<3, 4>(G, lds_bytes) : occupancy<3, 2>(G, lds_bytes);
   return W == 3 ? occupancy<1, 3>(G, lds_bytes) : W == 4 ? occupancy<1, 4>(G, lds_bytes) : occupancy<1, 2>(G, lds_bytes);
