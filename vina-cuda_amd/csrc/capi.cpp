@@ -1702,11 +1702,18 @@ void wide_ligands(vd_ctx* c, std::vector<LigPlan>& plans, const vd_dock_params* 
     }
   }
   rest *= 256.0 / std::max(1, c->n_cu);
-  const double line = p->local_search == VD_LS_RILC_BFGS ? 0.7 : 0.48;
-  for (size_t k = 0; k < plans.size(); ++k) {
+  // a ligand that must stay narrow (16 atoms have another pair layout) ends the batch anyway: wide
+  // chains next to it pay only for ligands well above it
+  double line = (p->local_search == VD_LS_RILC_BFGS ? 0.7 : 0.48) * rest / 7.6e-5;
+  auto can = [&](size_t k) {
     const int A = (int)lig_at(c, plans[k].id).atoms.size();
-    if (plans[k].G == 16 && A > 16 && A <= vdk::kWideAtoms && 7.6e-5 * units[k] > line * rest) plans[k].wide = true;
-  }
+    return plans[k].G == 16 && A > 16 && A <= vdk::kWideAtoms;
+  };
+  const double narrow_line = line;
+  for (size_t k = 0; k < plans.size(); ++k)
+    if (plans[k].G == 16 && !can(k) && units[k] > narrow_line) line = std::max(line, 1.25 * units[k]);
+  for (size_t k = 0; k < plans.size(); ++k)
+    if (can(k) && units[k] > line) plans[k].wide = true;
 }
 
 // Overlap applies to batches of exactly two classes, besides a wide launch.  Measured on the
