@@ -484,6 +484,9 @@ void make_edges(vd_ctx* c) {
   HIP_CHECK(hipStreamSynchronize(c->stream));
 }
 
+// Workgroups of a vd_eval launch, at most.
+int eval_blocks_max(const vd_ctx* c) { return 16 * std::max(c->n_cu, 1); }
+
 // Algorithmic bytes of one evaluation in the MC kernel: the eight map corners of every typed
 // atom (8 x 4 B) and one interpolation quad of the pair table per intramolecular pair (16 B).
 double eval_bytes(const vd_lig_header& h) { return 32.0 * h.n_heavy + 16.0 * h.n_pairs; }
@@ -1125,8 +1128,6 @@ int vd_create(int device, vd_ctx** out) {
     HIP_CHECK(hipEventCreate(&c->ev0));
     HIP_CHECK(hipEventCreate(&c->ev1));
     HIP_CHECK(hipEventCreate(&c->ev_base));
-    c->eval_clock.ensure(2);
-    HIP_CHECK(hipMemset(c->eval_clock.p, 0, 16));
     HIP_CHECK(hipDeviceGetAttribute(&c->clock_khz, hipDeviceAttributeWallClockRate, device));
     for (int k = 0; k < kMcSlots; ++k) {
       HIP_CHECK(hipEventCreate(&c->mc[k].ev0));
@@ -1136,6 +1137,8 @@ int vd_create(int device, vd_ctx** out) {
     hipDeviceProp_t prop;
     HIP_CHECK(hipGetDeviceProperties(&prop, device));
     c->n_cu = prop.multiProcessorCount;
+    c->eval_clock.ensure(1 + (size_t)eval_blocks_max(c));
+    HIP_CHECK(hipMemset(c->eval_clock.p, 0, (1 + (size_t)eval_blocks_max(c)) * 8));
     c->lds_max = (int)prop.sharedMemPerBlock;
     c->scratch = scratch_for_current_device(device);
     upload_lut(c);
@@ -1411,8 +1414,8 @@ int vd_eval(vd_ctx* c, int id, long long n, const float* conf, float* e, float* 
     a.K = make_evalk(c, v_intra, v_inter, slope);
     a.conf = conf; a.n_conf = n; a.e = e; a.grad = grad;
     // Host arrays up to kEvalDirectBytes go through page-locked memory that the kernel reads and
-    // writes itself: no copies to wait for (one pose of a 34-atom ligand 88 -> 27 us, 5,003 poses of a
-    // 75-atom one 190 -> 146 us).  Larger ones are copied to the device: a staging area of their size
+    // writes itself: no copies to wait for (one pose of a 34-atom ligand 88 -> 26 us, 5,003 poses of a
+    // 75-atom one 194 -> 125 us).  Larger ones are copied to the device: a staging area of their size
     // and a second pass over them on the host would cost more than the copies.
     const bool direct = !device_ptrs && (n_in + n_out + (size_t)n) * 4 <= kEvalDirectBytes;
     if (direct) {
@@ -1425,7 +1428,7 @@ int vd_eval(vd_ctx* c, int id, long long n, const float* conf, float* e, float* 
       a.conf = c->io_a.p; a.e = c->io_b.p; a.grad = c->io_c.p;
     }
     const long long per_block = 64 / G;
-    const int blocks = (int)std::min<long long>((n + per_block - 1) / per_block, (long long)c->n_cu * 16);
+    const int blocks = (int)std::min<long long>((n + per_block - 1) / per_block, (long long)eval_blocks_max(c));
     HIP_CHECK(vdl::launch_eval(G, a, blocks, c->stream));
     c->eval_timed = true;
     if (!direct && !device_ptrs) {
@@ -1441,10 +1444,12 @@ int vd_eval(vd_ctx* c, int id, long long n, const float* conf, float* e, float* 
 }
 
 double vd_eval_last_ms(const vd_ctx* c) {
-  unsigned long long t[2];
   if (!c || !c->eval_timed || hipSetDevice(c->device) != hipSuccess) return 0.0;
-  if (hipMemcpy(t, c->eval_clock.p, sizeof t, hipMemcpyDeviceToHost) != hipSuccess) return 0.0;
-  return t[1] > t[0] ? (double)(t[1] - t[0]) / c->clock_khz : 0.0;
+  // words of earlier launches' further workgroups hold earlier ticks
+  std::vector<unsigned long long> t(1 + (size_t)eval_blocks_max(c));
+  if (hipMemcpy(t.data(), c->eval_clock.p, t.size() * 8, hipMemcpyDeviceToHost) != hipSuccess) return 0.0;
+  const unsigned long long last = *std::max_element(t.begin() + 1, t.end());
+  return last > t[0] ? (double)(last - t[0]) / c->clock_khz : 0.0;
 }
 
 int vd_dock_params_default(vd_dock_params* p) {

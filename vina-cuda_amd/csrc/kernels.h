@@ -41,7 +41,7 @@ struct EvalArgs {
   vdk::EvalK K;
   const float* conf; long long n_conf;
   float* e; float* grad;
-  unsigned long long* clock;        // the launch's first and last device clock tick (the second only grows)
+  unsigned long long* clock;        // the launch's first device clock tick, and every workgroup's last
 };
 
 // Refinement launch (vd_refine_kernel, FP64): one pose per workgroup.

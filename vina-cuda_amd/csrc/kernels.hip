@@ -665,7 +665,8 @@ __global__ __launch_bounds__(64) void vd_eval_kernel(EvalArgs a) {
       if (l >= G - 6) go[l - (G - 6)] = g;
     }
   }
-  if (lane == 0) atomicMax(a.clock + 1, (unsigned long long)wall_clock64());
+  // a word per workgroup: a maximum of 4,096 workgroups over one word took 45 us of a launch
+  if (lane == 0) a.clock[1 + blockIdx.x] = (unsigned long long)wall_clock64();
 }
 
 // ------------------------------------------------------------------------------------------
