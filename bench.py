@@ -719,7 +719,7 @@ def main():
                        "hbm_traffic_GBs": round(traffic / (avg_span / 1000.0) / 1e9, 1) if traffic else None,
                        "hbm_traffic_frac": round(traffic / (avg_span / 1000.0) / 1e9 / HBM_PEAK_GBS, 4) if traffic else None,
                        "binding_resource": "the vector-memory data path (TA/TD) that serves the gathers of map "
-                                           "corner records and pair-table quads through L1/L2; the 64-lane "
+                                           "edge records and pair-table quads through L1/L2; the 64-lane "
                                            "instantiation is also VALU-bound (no dense contraction, so no MFMA "
                                            "bound)",
                        "counters_by_instantiation_profiled": valu,
