@@ -1,0 +1,52 @@
+"""What the kernels ask of the compiler, read from the unoptimised code of the device sources: it
+holds whatever a compiler's passes make of it, where a run shows today's build only."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+CSRC = os.path.join(ROOT, "vina-cuda_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def functions(tmp_path_factory):
+    """Mangled name -> body, of kernels.hip as the front end emits it."""
+    out = str(tmp_path_factory.mktemp("ir") / "kernels.ll")
+    subprocess.check_call([HIPCC, "-O1", "-std=c++17", "--offload-arch=gfx950", "--cuda-device-only", "-emit-llvm", "-S",
+                           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Xclang", "-disable-llvm-passes",
+                           "-w", "-o", out, os.path.join(CSRC, "kernels.hip")])
+    with open(out) as f:
+        return {m.group(1): m.group(2) for m in re.finditer(r"^define [^@]*@(\S+?)\(.*?\{$(.*?)^\}", f.read(), re.M | re.S)}
+
+
+def calls(body, *names):
+    """The calls of a body to any of the named functions, in order."""
+    found = re.findall(r"call [^@]*@(\S+?)\(", body)
+    return [n for f in found for n in names if re.search(r"\d%s[A-Z]" % n, f)]
+
+
+def test_rows_of_a_wide_chain_update_a_node_in_turn(functions):
+    """A node whose atoms lie in several rows of 16 lanes: each row's update is fenced from the next."""
+    wide = [b for n, b in functions.items() if re.match(r"_ZN3vdk10eval_derivILi16ELb1", n)]
+    assert len(wide) == 3   # the three modes
+    for body in wide:
+        assert calls(body, "add_to_node", "wave_sync") == ["add_to_node", "wave_sync"]
+
+
+def test_exchange_row_of_a_wide_chain_is_fenced(functions):
+    """Slots written by all lanes, read by the lanes that own their atoms, written again."""
+    body, = [b for n, b in functions.items() if n.startswith("_ZN3vdk15pair_terms_wide")]
+    assert re.search(r"call [^@]*@_ZN3vdk9wave_sync", body)
+    order = re.findall(r"call [^@]*@(_ZN3vdk9wave_sync|_ZZN3vdk15pair_terms_wide\S*?RK?15HIP_vector_typeIfLj4EES9_IjLj2EE)", body)
+    assert ["sync" if "wave_sync" in o else "take" for o in order] == ["sync", "take", "take", "sync"]
+
+
+def test_wave_sync_is_a_fence_and_a_barrier(functions):
+    for ns in ("3vdk", "3vdr"):
+        body, = [b for n, b in functions.items() if n.startswith("_ZN%s9wave_syncEv" % ns)]
+        assert 'fence syncscope("wavefront") acq_rel' in body and "@llvm.amdgcn.wave.barrier" in body

@@ -473,6 +473,14 @@ __device__ float pair_terms_scatter(const LigView& L, const Scratch& S, const Ev
   return e_intra;
 }
 
+// Orders the LDS accesses of one wavefront where a lane reads or updates what other lanes wrote: the
+// hardware takes them in order, and this keeps the compiler, which sees one lane's accesses only, from
+// moving or merging them.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // ---- Wide launches: one chain per wavefront with the arithmetic of a 16-lane group.
 // Four rows of 16 lanes carry the same chain.  What a 16-lane group does in turn -- atoms l, l + 16,
 // ...; chunk after chunk of pairs; the passes of the node scan -- the rows do side by side, and the
@@ -545,13 +553,21 @@ __device__ inline float pair_terms_wide(const LigView& L, const Scratch& S, cons
     pair_term(p.q, p.rem, ck, e, dor);
     S.fx[lane] = p.ok ? make_float4(p.rx, p.ry, p.rz, dor) : make_float4(0, 0, 0, 0);
     e_intra = add_rows(e_intra, p.ok ? e : 0.0f);
+    wave_sync();   // every slot is written before any is read
     take8(f0, p.s0);
     if (two) take8(f1, p.s1);
+    wave_sync();   // and read before the next pass writes it
     p = n;
   }
   if (lane < L.A) S.frc[lane] = f0;
   if (lane + 64 < L.A) S.frc[lane + 64] = f1;
   return e_intra;
+}
+
+__device__ __forceinline__ void add_to_node(const Scratch& S, int node, const float (&v)[6]) {
+  float4 a = S.nacc[2 * node], b = S.nacc[2 * node + 1];
+  a.x += v[0]; a.y += v[1]; a.z += v[2]; b.x += v[3]; b.y += v[4]; b.z += v[5];
+  S.nacc[2 * node] = a; S.nacc[2 * node + 1] = b;
 }
 
 // Energy and gradient of one conformation per group (model::eval_deriv,
@@ -648,12 +664,16 @@ __device__ float eval_deriv(const LigView& L, const Scratch& S, const EvalK& K, 
     seg_scan<G>(v, node);
     const int next = __shfl_down(node, 1, G);
     const bool last = node >= 0 && (l == G - 1 || next != node);
-    for (int r = 0; r < (WIDE ? 4 : 1); ++r)   // wide: the rows are the group's passes, in turn
-      if (last && (!WIDE || lane >> 4 == r)) {
-        float4 a = S.nacc[2 * node], b = S.nacc[2 * node + 1];
-        a.x += v[0]; a.y += v[1]; a.z += v[2]; b.x += v[3]; b.y += v[4]; b.z += v[5];
-        S.nacc[2 * node] = a; S.nacc[2 * node + 1] = b;
+    if constexpr (WIDE) {
+      // the rows are the group's passes, in turn: a node whose atoms lie in several rows takes each row's
+      // sums on top of the ones before, so the four updates must stay apart
+      for (int r = 0; r < 4; ++r) {
+        if (last && lane >> 4 == r) add_to_node(S, node, v);
+        wave_sync();
       }
+    } else if (last) {
+      add_to_node(S, node, v);
+    }
   }
   __syncthreads();
   // subtree sums: the subtree of node k is the preorder range [k, subtree_end_k); the torque
