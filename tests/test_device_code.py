@@ -50,3 +50,12 @@ def test_wave_sync_is_a_fence_and_a_barrier(functions):
     for ns in ("3vdk", "3vdr"):
         body, = [b for n, b in functions.items() if n.startswith("_ZN%s9wave_syncEv" % ns)]
         assert 'fence syncscope("wavefront") acq_rel' in body and "@llvm.amdgcn.wave.barrier" in body
+
+
+def test_half_rows_of_the_map_table_are_read_at_their_alignment(functions):
+    """Half 1 of a 48-byte row lies at a multiple of 8 bytes, so no read of a half may promise 16."""
+    body, = [b for n, b in functions.items() if re.match(r"_ZN12_GLOBAL__N_19load_half", n)]
+    reads = re.findall(r"load <4 x float>, ptr \S+, align (\d+)", body)
+    copies = re.findall(r"@llvm.memcpy\S*\(ptr align \d+ \S+, ptr align (\d+)", body)
+    assert reads and all(int(a) <= 8 for a in reads + copies)
+    assert [calls(b, "load_half") for n, b in functions.items() if re.match(r"_ZN12_GLOBAL__N_114vd_grid_kernel", n)] == [["load_half"]]

@@ -52,6 +52,13 @@ template <int LP> struct GridTile {
 
 // One lane's half of a row, and its addition to the lane's sums: acc[k] += value of index pick k.
 struct HalfRow { float4 a; float2 b; };
+// A row of twelve floats leaves its second half at a multiple of 8 bytes only, and the type has to say
+// so (global memory takes a 16-byte load at 8-byte alignment whole).
+typedef float float4_a8 __attribute__((ext_vector_type(4), aligned(8)));
+__device__ __forceinline__ HalfRow load_half(const float* r) {
+  const float4_a8 a = *reinterpret_cast<const float4_a8*>(r);
+  return {make_float4(a.x, a.y, a.z, a.w), *reinterpret_cast<const float2*>(r + 4)};
+}
 template <int I> __device__ __forceinline__ float value(const HalfRow& v) {
   if constexpr (I == 0) return v.a.x;
   else if constexpr (I == 1) return v.a.y;
@@ -149,9 +156,7 @@ __global__ __launch_bounds__(64) void vd_grid_kernel(const float4* __restrict__ 
               const uint32_t half = ((meta[u] >> 24) & 3u) == 0 ? 4u : 6u;   // uniform
 #pragma unroll
               for (int h = 0; h < H; ++h) {
-                const float* r = rows + (__umul24(bin, 2 * half) + half * (LP == 2 ? q : h));
-                v[u][h].a = *reinterpret_cast<const float4*>(r);
-                v[u][h].b = *reinterpret_cast<const float2*>(r + 4);
+                v[u][h] = load_half(rows + (__umul24(bin, 2 * half) + half * (LP == 2 ? q : h)));
               }
             }
           }
