@@ -57,5 +57,6 @@ def test_half_rows_of_the_map_table_are_read_at_their_alignment(functions):
     body, = [b for n, b in functions.items() if re.match(r"_ZN12_GLOBAL__N_19load_half", n)]
     reads = re.findall(r"load <4 x float>, ptr \S+, align (\d+)", body)
     copies = re.findall(r"@llvm.memcpy\S*\(ptr align \d+ \S+, ptr align (\d+)", body)
-    assert reads and all(int(a) <= 8 for a in reads + copies)
-    assert [calls(b, "load_half") for n, b in functions.items() if re.match(r"_ZN12_GLOBAL__N_114vd_grid_kernel", n)] == [["load_half"]]
+    assert reads + copies and all(int(a) <= 8 for a in reads + copies)
+    kernels = [b for n, b in functions.items() if re.match(r"_ZN12_GLOBAL__N_114vd_grid_kernel", n)]
+    assert kernels and all(calls(b, "load_half") == ["load_half"] for b in kernels)

@@ -1300,7 +1300,7 @@ int vd_grid_populate(vd_ctx* c, const vd_box* box) {
     c->maps.ensure((size_t)VD_XS_SIZE * c->gd.plane);
     HIP_CHECK(hipEventRecord(c->ev0, c->stream));
     HIP_CHECK(vdl::launch_grid(c->grid_atoms.p, c->grid_cells.p, gcl, c->lut_rows.p, c->maps.p,
-                               c->gd, c->stream));
+                               c->gd, c->n_cu, c->stream));
     HIP_CHECK(hipEventRecord(c->ev1, c->stream));
     HIP_CHECK(hipStreamSynchronize(c->stream));
     c->grid_ms = elapsed_ms(c);

@@ -164,7 +164,7 @@ const int kGridPick[VD_GRID_CLASSES][VD_GRID_PER_HALF] = {{VD_GRID_PICK_PLAIN}, 
                                                           {VD_GRID_PICK_BONDING}};
 
 void Precalculated::grid_rows(std::vector<float>& out, uint32_t meta[VD_XS_SIZE]) const {
-  out.clear();
+  out.assign(8, 0.0f);   // a row of zeros: what lanes without an atom in reach read
   for (int t1 = 0; t1 < VD_XS_SIZE; ++t1) {
     const bool acc = xs_is_acceptor(t1), don = xs_is_donor(t1);
     const int cls = xs_is_hydrophobic(t1) ? 1 : acc || don ? 2 : 0;

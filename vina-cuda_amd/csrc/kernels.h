@@ -86,7 +86,7 @@ int wide_lds_bytes(int Amax, int Nmax, int dense);
 int max_resident_wide_blocks(int mode, int lds_bytes);
 hipError_t launch_mc_wide(const McArgs& a, int blocks, hipStream_t s);
 hipError_t launch_grid(const float4* atoms, const int2* cells, const GridCells& gc, const float* lut, float* maps,
-                       const vd_grid_desc& gd, hipStream_t s);
+                       const vd_grid_desc& gd, int n_cu, hipStream_t s);
 // Edge records of the maps (VD_XS_SIZE * dim0 (dim1-1)(dim2-1) float4) from the canonical maps,
 // both on the device.
 hipError_t launch_edges(const float* maps, float4* edges, const vd_grid_desc& gd, hipStream_t s);

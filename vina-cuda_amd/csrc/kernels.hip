@@ -27,8 +27,8 @@ namespace {
 // come from a host-built cell list (cells of VD_GCELL A over the box grown by the 8 A cutoff, one
 // contiguous atom range per x-row of cells).  Each range is read 64 atoms at a time, one per lane
 // in a single coalesced load; a ballot of the lanes whose atom lies within the cutoff of the tile
-// box lists the atoms worth a pass, and the loop takes them in index order (GU per pass, all their
-// table reads in flight before any is added), reading each atom from its lane with readlane.  For
+// box lists the atoms worth a pass, and the loop takes them in index order (GU per pass, their
+// table reads before any is added), reading each atom from its lane with readlane.  For
 // every atom within the cutoff of a point, one row of the map LUT gives the contribution to all 17
 // maps: 4 values per half for a receptor type that neither is hydrophobic nor bonds, up to 6 for the
 // others, 16 and 8 bytes per lane.  Every point adds its atoms in the
@@ -38,6 +38,13 @@ namespace {
 // bytes) took 232 us at 81^3 and 1.91 ms at 188^3, these 202 us and 1.64 ms; one lane per point
 // 236 us and 1.79 ms, four atoms per pass 224 us and 1.79 ms, loads not masked by the cutoff 210 us
 // and 1.70 ms.
+// FEW: a launch of few tiles is bound by the length of a wavefront's chain of waits instead, and takes
+// as long as its longest.  Two things shorten that chain: all rows of cells are looked up at once, a
+// row per lane, and every lane reads, those out of reach the row of zeros at the table's start, so that
+// no branch stands between the reads of a pass (around masked reads the compiler has the second atom's
+// wait for the first's).  Kernel times with masked reads -> FEW: a 1 A box 21.6 -> 18.4 us, 8 A 34 ->
+// 28.5, 16 A 59.6 -> 50, 24 A 134 -> 127, 35 A 296 -> 297, 40 A 422 -> 425, 70 A 1,385 -> 1,431; in a
+// cavity, whose tiles reach few atoms, 30 A 63.5 -> 59.6, 35 A 106 -> 96, 40 A 149 -> 153.
 constexpr int GU = 2;   // receptor atoms per pass of the grid kernel's loop
 
 __device__ __forceinline__ float lane_f(float v, int j) {
@@ -52,12 +59,15 @@ template <int LP> struct GridTile {
 
 // One lane's half of a row, and its addition to the lane's sums: acc[k] += value of index pick k.
 struct HalfRow { float4 a; float2 b; };
-// A row of twelve floats leaves its second half at a multiple of 8 bytes only, and the type has to say
-// so (global memory takes a 16-byte load at 8-byte alignment whole).
-typedef float float4_a8 __attribute__((ext_vector_type(4), aligned(8)));
+// A row of twelve floats leaves its second half at a multiple of 8 bytes only, and the read has to say
+// so (global memory takes a 16-byte load at 8-byte alignment whole).  Copied in this form the two loads
+// stay in order, and a plain row's sums wait for the first only; through a vector type of alignment 8
+// they were swapped (81^3 177 -> 185 us).
 __device__ __forceinline__ HalfRow load_half(const float* r) {
-  const float4_a8 a = *reinterpret_cast<const float4_a8*>(r);
-  return {make_float4(a.x, a.y, a.z, a.w), *reinterpret_cast<const float2*>(r + 4)};
+  HalfRow v;
+  __builtin_memcpy(&v.a, __builtin_assume_aligned(r, 8), 16);
+  __builtin_memcpy(&v.b, __builtin_assume_aligned(r + 4, 8), 8);
+  return v;
 }
 template <int I> __device__ __forceinline__ float value(const HalfRow& v) {
   if constexpr (I == 0) return v.a.x;
@@ -92,7 +102,7 @@ __device__ __forceinline__ void add_row(uint32_t meta, HalfSums& s, const HalfRo
 }
 #undef VD_KEEP
 
-template <int LP>
+template <int LP, bool FEW>
 __global__ __launch_bounds__(64) void vd_grid_kernel(const float4* __restrict__ atoms, const int2* __restrict__ cells,
                                                      GridCells gc, const float* __restrict__ lut, float* __restrict__ maps,
                                                      vd_grid_desc gd, int tiles_x, int tiles_y) {
@@ -117,10 +127,29 @@ __global__ __launch_bounds__(64) void vd_grid_kernel(const float4* __restrict__ 
   const int cy0 = max(0, (int)floorf((lo_y - cut) * inv)), cy1 = min(gc.n[1] - 1, (int)floorf((hi_y + cut) * inv));
   const int cz0 = max(0, (int)floorf((lo_z - cut) * inv)), cz1 = min(gc.n[2] - 1, (int)floorf((hi_z + cut) * inv));
   HalfSums acc[H] = {};
-  for (int cz = cz0; cz <= cz1; ++cz)
-    for (int cy = cy0; cy <= cy1; ++cy) {
-      const int row = (cz * gc.n[1] + cy) * gc.n[0];
-      const int begin = cells[row + cx0].x, end = cells[row + cx1].y;   // cells of one x-row are contiguous
+  const int ny = cy1 - cy0 + 1, rows = ny * max(0, cz1 - cz0 + 1);
+  for (int outer = FEW ? 0 : cz0; FEW ? 64 * outer < rows : outer <= cz1; ++outer) {
+    // few tiles: every lane looks up a row, and those that hold atoms are taken in turn
+    uint64_t left = 0;
+    int row_begin = 0, row_end = 0;
+    if constexpr (FEW) {
+      const int r = 64 * outer + lane;
+      if (r < rows) {
+        const int first = ((cz0 + r / ny) * gc.n[1] + cy0 + r % ny) * gc.n[0];
+        row_begin = cells[first + cx0].x; row_end = cells[first + cx1].y;
+      }
+      left = __ballot(row_end > row_begin);
+    }
+    for (int cy = cy0; FEW ? left != 0 : cy <= cy1; ++cy) {
+      int begin, end;   // cells of one x-row are contiguous
+      if constexpr (FEW) {
+        const int i = __builtin_ctzll(left);
+        left &= left - 1;
+        begin = __builtin_amdgcn_readlane(row_begin, i); end = __builtin_amdgcn_readlane(row_end, i);
+      } else {
+        const int first = (outer * gc.n[1] + cy) * gc.n[0];
+        begin = cells[first + cx0].x; end = cells[first + cx1].y;
+      }
       for (int base = begin; base < end; base += 64) {
         // this lane's atom of the chunk, and whether it can reach the tile at all
         const int k = base + lane;
@@ -146,29 +175,31 @@ __global__ __launch_bounds__(64) void vd_grid_kernel(const float4* __restrict__ 
           for (int u = 0; u < GU; ++u) {
             const float ax = lane_f(mine.x, j[u]), ay = lane_f(mine.y, j[u]), az = lane_f(mine.z, j[u]);
             meta[u] = (uint32_t)__builtin_amdgcn_readlane(__float_as_int(mine.w), j[u]);
-            const float* rows = lut + 4 * (meta[u] & 0xFFFFFFu);
             const float dx = ax - px, dy = ay - py, dz = az - pz;
             const float r2 = dx * dx + dy * dy + dz * dz;
             use[u] = has[u] && inside && r2 <= VD_CUTOFF_SQR;
-            if (use[u]) {
+            const uint32_t type_rows = 4 * (meta[u] & 0xFFFFFFu);
+            if (FEW || use[u]) {
               // a plain row's lane reads past its own 16 bytes; the table ends with room for that
               const uint32_t bin = (uint32_t)(VD_LUT_FACTOR * r2);
               const uint32_t half = ((meta[u] >> 24) & 3u) == 0 ? 4u : 6u;   // uniform
 #pragma unroll
               for (int h = 0; h < H; ++h) {
-                v[u][h] = load_half(rows + (__umul24(bin, 2 * half) + half * (LP == 2 ? q : h)));
+                const uint32_t o = __umul24(bin, 2 * half) + half * (LP == 2 ? q : h);
+                v[u][h] = load_half(FEW ? lut + (use[u] ? type_rows + o : 0u) : lut + type_rows + o);
               }
             }
           }
 #pragma unroll
           for (int u = 0; u < GU; ++u) {
-            if (!use[u]) continue;
+            if (!FEW && !use[u]) continue;
 #pragma unroll
             for (int h = 0; h < H; ++h) add_row(meta[u], acc[h], v[u][h]);
           }
         }
       }
     }
+  }
   if (inside) {
     const size_t o = (size_t)x + (size_t)gd.dim[0] * ((size_t)y + (size_t)gd.dim[1] * z);
     constexpr int types[2][VD_GRID_PER_HALF] = {VD_GRID_TYPES};
@@ -853,11 +884,15 @@ int mc_lds_bytes(int G, int Amax, int Nmax, int dense) {
 constexpr int kGridLanesPerPoint = 2;
 
 hipError_t launch_grid(const float4* atoms, const int2* cells, const GridCells& gc, const float* lut, float* maps,
-                       const vd_grid_desc& gd, hipStream_t s) {
+                       const vd_grid_desc& gd, int n_cu, hipStream_t s) {
   using T = GridTile<kGridLanesPerPoint>;
   const int tx = (gd.dim[0] + T::TX - 1) / T::TX, ty = (gd.dim[1] + T::TY - 1) / T::TY, tz = (gd.dim[2] + T::TZ - 1) / T::TZ;
-  hipLaunchKernelGGL(vd_grid_kernel<kGridLanesPerPoint>, dim3(tx * ty * tz), dim3(64), 0, s, atoms, cells, gc, lut, maps, gd,
-                     tx, ty);
+  if (tx * ty * tz <= 112 * n_cu)   // 35 A boxes and smaller; both sides are given above vd_grid_kernel
+    hipLaunchKernelGGL((vd_grid_kernel<kGridLanesPerPoint, true>), dim3(tx * ty * tz), dim3(64), 0, s, atoms, cells, gc, lut,
+                       maps, gd, tx, ty);
+  else
+    hipLaunchKernelGGL((vd_grid_kernel<kGridLanesPerPoint, false>), dim3(tx * ty * tz), dim3(64), 0, s, atoms, cells, gc, lut,
+                       maps, gd, tx, ty);
   return hipGetLastError();
 }
 

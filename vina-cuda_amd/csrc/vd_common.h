@@ -15,7 +15,8 @@
 // differ by radius, by the hydrophobic match (only if t1 is hydrophobic) and by the hydrogen bond
 // (only if t1 is a donor or an acceptor).  A row (t1, bin) holds each value once, in two halves of
 // VD_GRID_HALF(class) floats, for the types kGridTypes[half]; type k of either half takes the half's
-// value of index VD_GRID_PICK_<class>[k].  The rows of a type start at a multiple of 16 bytes; half 1
+// value of index VD_GRID_PICK_<class>[k].  The table starts with a row of
+// zeros (eight floats).  The rows of a type start at a multiple of 16 bytes; half 1
 // of a row of six-float halves lies at a multiple of 8 only.
 #define VD_GRID_CLASSES 3            // of t1: 0 plain, 1 hydrophobic, 2 bonding (donor or acceptor)
 #define VD_GRID_PER_HALF 9           // types per half (half 1 has 8: its entry 7 is none, -1)
