@@ -60,3 +60,11 @@ def test_half_rows_of_the_map_table_are_read_at_their_alignment(functions):
     assert reads + copies and all(int(a) <= 8 for a in reads + copies)
     kernels = [b for n, b in functions.items() if re.match(r"_ZN12_GLOBAL__N_114vd_grid_kernel", n)]
     assert kernels and all(calls(b, "load_half") == ["load_half"] for b in kernels)
+
+
+def test_every_compiled_form_is_launched(functions):
+    """Dense BFGS takes three waves per SIMD on 64 lanes only; the map kernel has two forms."""
+    names = [m.groups() for m in (re.match(r"_ZN12_GLOBAL__N_112vd_mc_kernelILi(\d+)ELi(\d)ELi(\d)E", n) for n in functions) if m]
+    assert {n for n in names if n[1] == "0"} == {("64", "0", "2"), ("32", "0", "2"), ("16", "0", "2"), ("64", "0", "3")}
+    assert {n for n in names if n[1] != "0"} == {(g, m, w) for g in ("16", "32", "64") for m in "123" for w in "234"}
+    assert len([n for n in functions if re.match(r"_ZN12_GLOBAL__N_114vd_grid_kernelILb", n)]) == 2

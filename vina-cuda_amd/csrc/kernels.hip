@@ -21,9 +21,9 @@ using namespace vdk;
 namespace {
 
 // ------------------------------------------------------------------------------------------
-// Grid maps.  A workgroup is one wavefront and owns a compact tile of points (x fastest), LP
-// lanes per point: lane l works on point l / LP and, with LP = 2, on half l % 2 of the map types
-// (with LP = 1 on both).  The receptor atoms that can reach the tile
+// Grid maps.  A workgroup is one wavefront and owns a compact tile of points (x fastest), two
+// lanes per point: lane l works on point l / 2 and half l % 2 of the map types.  The receptor atoms
+// that can reach the tile
 // come from a host-built cell list (cells of VD_GCELL A over the box grown by the 8 A cutoff, one
 // contiguous atom range per x-row of cells).  Each range is read 64 atoms at a time, one per lane
 // in a single coalesced load; a ballot of the lanes whose atom lies within the cutoff of the tile
@@ -31,8 +31,8 @@ namespace {
 // table reads before any is added), reading each atom from its lane with readlane.  For
 // every atom within the cutoff of a point, one row of the map LUT gives the contribution to all 17
 // maps: 4 values per half for a receptor type that neither is hydrophobic nor bonds, up to 6 for the
-// others, 16 and 8 bytes per lane.  Every point adds its atoms in the
-// order of the cell list, whatever the tile shape or LP, so neither changes a map value.
+// others, 16 and 8 bytes per lane.  Every point adds its atoms in the order of the cell list,
+// whatever the tile shape, so it does not change a map value.
 // What bounds it is the L2's delivery to the L1s (a wavefront's 32 points read 32 rows far apart:
 // 4e7 requests at 81^3, some 20 TB/s), with the vector units 70 % busy.  Rows of all 17 values (68
 // bytes) took 232 us at 81^3 and 1.91 ms at 188^3, these 202 us and 1.64 ms; one lane per point
@@ -51,18 +51,14 @@ __device__ __forceinline__ float lane_f(float v, int j) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
 }
 
-template <int LP> struct GridTile {
-  static constexpr int NP = 64 / LP;                 // points per wavefront
-  static constexpr int TX = 4, TY = NP >= 32 ? 4 : 2, TZ = NP / (TX * TY);
-  static constexpr int H = 2 / LP;                   // halves per lane
-};
+struct GridTile { static constexpr int TX = 4, TY = 4, TZ = 2; };   // points of a wavefront
 
 // One lane's half of a row, and its addition to the lane's sums: acc[k] += value of index pick k.
 struct HalfRow { float4 a; float2 b; };
 // A row of twelve floats leaves its second half at a multiple of 8 bytes only, and the read has to say
 // so (global memory takes a 16-byte load at 8-byte alignment whole).  Copied in this form the two loads
-// stay in order, and a plain row's sums wait for the first only; through a vector type of alignment 8
-// they were swapped (81^3 177 -> 185 us).
+// of a masked read stay in order, and a plain row's sums wait for the first only; through a vector type
+// of alignment 8 they were swapped.
 __device__ __forceinline__ HalfRow load_half(const float* r) {
   HalfRow v;
   __builtin_memcpy(&v.a, __builtin_assume_aligned(r, 8), 16);
@@ -102,14 +98,13 @@ __device__ __forceinline__ void add_row(uint32_t meta, HalfSums& s, const HalfRo
 }
 #undef VD_KEEP
 
-template <int LP, bool FEW>
+template <bool FEW>
 __global__ __launch_bounds__(64) void vd_grid_kernel(const float4* __restrict__ atoms, const int2* __restrict__ cells,
                                                      GridCells gc, const float* __restrict__ lut, float* __restrict__ maps,
                                                      vd_grid_desc gd, int tiles_x, int tiles_y) {
-  using T = GridTile<LP>;
-  constexpr int TX = T::TX, TY = T::TY, TZ = T::TZ, H = T::H;
+  constexpr int TX = GridTile::TX, TY = GridTile::TY, TZ = GridTile::TZ;
   const int tile = blockIdx.x, lane = threadIdx.x;
-  const int pt = lane / LP, q = lane % LP;
+  const int pt = lane / 2, q = lane % 2;
   const int tx0 = (tile % tiles_x) * TX, ty0 = ((tile / tiles_x) % tiles_y) * TY, tz0 = (tile / (tiles_x * tiles_y)) * TZ;
   const int lx = pt % TX, ly = (pt / TX) % TY, lz = pt / (TX * TY);
   const int x = tx0 + lx, y = ty0 + ly, z = tz0 + lz;
@@ -126,7 +121,7 @@ __global__ __launch_bounds__(64) void vd_grid_kernel(const float4* __restrict__ 
   const int cx0 = max(0, (int)floorf((lo_x - cut) * inv)), cx1 = min(gc.n[0] - 1, (int)floorf((hi_x + cut) * inv));
   const int cy0 = max(0, (int)floorf((lo_y - cut) * inv)), cy1 = min(gc.n[1] - 1, (int)floorf((hi_y + cut) * inv));
   const int cz0 = max(0, (int)floorf((lo_z - cut) * inv)), cz1 = min(gc.n[2] - 1, (int)floorf((hi_z + cut) * inv));
-  HalfSums acc[H] = {};
+  HalfSums acc = {};
   const int ny = cy1 - cy0 + 1, rows = ny * max(0, cz1 - cz0 + 1);
   for (int outer = FEW ? 0 : cz0; FEW ? 64 * outer < rows : outer <= cz1; ++outer) {
     // few tiles: every lane looks up a row, and those that hold atoms are taken in turn
@@ -168,7 +163,7 @@ __global__ __launch_bounds__(64) void vd_grid_kernel(const float4* __restrict__ 
             j[u] = has[u] ? __builtin_ctzll(todo) : 0;
             todo &= todo - 1;
           }
-          HalfRow v[GU][H];
+          HalfRow v[GU];
           uint32_t meta[GU];
           bool use[GU];
 #pragma unroll
@@ -183,18 +178,14 @@ __global__ __launch_bounds__(64) void vd_grid_kernel(const float4* __restrict__ 
               // a plain row's lane reads past its own 16 bytes; the table ends with room for that
               const uint32_t bin = (uint32_t)(VD_LUT_FACTOR * r2);
               const uint32_t half = ((meta[u] >> 24) & 3u) == 0 ? 4u : 6u;   // uniform
-#pragma unroll
-              for (int h = 0; h < H; ++h) {
-                const uint32_t o = __umul24(bin, 2 * half) + half * (LP == 2 ? q : h);
-                v[u][h] = load_half(FEW ? lut + (use[u] ? type_rows + o : 0u) : lut + type_rows + o);
-              }
+              const uint32_t o = __umul24(bin, 2 * half) + half * q;
+              v[u] = load_half(FEW ? lut + (use[u] ? type_rows + o : 0u) : lut + type_rows + o);
             }
           }
 #pragma unroll
           for (int u = 0; u < GU; ++u) {
             if (!FEW && !use[u]) continue;
-#pragma unroll
-            for (int h = 0; h < H; ++h) add_row(meta[u], acc[h], v[u][h]);
+            add_row(meta[u], acc, v[u]);
           }
         }
       }
@@ -203,15 +194,11 @@ __global__ __launch_bounds__(64) void vd_grid_kernel(const float4* __restrict__ 
   if (inside) {
     const size_t o = (size_t)x + (size_t)gd.dim[0] * ((size_t)y + (size_t)gd.dim[1] * z);
     constexpr int types[2][VD_GRID_PER_HALF] = {VD_GRID_TYPES};
+    const float sum[VD_GRID_PER_HALF] = {acc.s0, acc.s1, acc.s2, acc.s3, acc.s4, acc.s5, acc.s6, acc.s7, acc.s8};
 #pragma unroll
-    for (int h = 0; h < H; ++h) {
-      const HalfSums& s = acc[h];
-      const float sum[VD_GRID_PER_HALF] = {s.s0, s.s1, s.s2, s.s3, s.s4, s.s5, s.s6, s.s7, s.s8};
-#pragma unroll
-      for (int k = 0; k < VD_GRID_PER_HALF; ++k) {
-        const int t = LP == 1 ? types[h][k] : q ? types[1][k] : types[0][k];
-        if (t >= 0) maps[(size_t)t * gd.plane + o] = sum[k];
-      }
+    for (int k = 0; k < VD_GRID_PER_HALF; ++k) {
+      const int t = q ? types[1][k] : types[0][k];
+      if (t >= 0) maps[(size_t)t * gd.plane + o] = sum[k];
     }
   }
 }
@@ -880,19 +867,14 @@ int mc_lds_bytes(int G, int Amax, int Nmax, int dense) {
   return 4 * (lig_floats(Amax, Nmax) + (64 / G) * group_floats(Amax, Nmax, G, dense));
 }
 
-// Lanes per grid point of the grid kernel.
-constexpr int kGridLanesPerPoint = 2;
-
 hipError_t launch_grid(const float4* atoms, const int2* cells, const GridCells& gc, const float* lut, float* maps,
                        const vd_grid_desc& gd, int n_cu, hipStream_t s) {
-  using T = GridTile<kGridLanesPerPoint>;
+  using T = GridTile;
   const int tx = (gd.dim[0] + T::TX - 1) / T::TX, ty = (gd.dim[1] + T::TY - 1) / T::TY, tz = (gd.dim[2] + T::TZ - 1) / T::TZ;
   if (tx * ty * tz <= 112 * n_cu)   // 35 A boxes and smaller; both sides are given above vd_grid_kernel
-    hipLaunchKernelGGL((vd_grid_kernel<kGridLanesPerPoint, true>), dim3(tx * ty * tz), dim3(64), 0, s, atoms, cells, gc, lut,
-                       maps, gd, tx, ty);
+    hipLaunchKernelGGL(vd_grid_kernel<true>, dim3(tx * ty * tz), dim3(64), 0, s, atoms, cells, gc, lut, maps, gd, tx, ty);
   else
-    hipLaunchKernelGGL((vd_grid_kernel<kGridLanesPerPoint, false>), dim3(tx * ty * tz), dim3(64), 0, s, atoms, cells, gc, lut,
-                       maps, gd, tx, ty);
+    hipLaunchKernelGGL(vd_grid_kernel<false>, dim3(tx * ty * tz), dim3(64), 0, s, atoms, cells, gc, lut, maps, gd, tx, ty);
   return hipGetLastError();
 }
 
@@ -935,12 +917,14 @@ int max_resident_wide_blocks(int mode, int lds_bytes) {
   return e == hipSuccess ? n : 0;
 }
 
+// The budgets compiled: dense BFGS runs at three waves per SIMD on 64 lanes only (plan_for).
+template <int G, int MODE, int W> constexpr int kBudget = MODE == 0 && G < 64 ? 2 : W;
 template <int MODE, int W>
 static hipError_t launch_mc_mode(int G, const McArgs& a, int blocks, int lds, hipStream_t s) {
   switch (G) {
-    case 64: hipLaunchKernelGGL((vd_mc_kernel<64, MODE, W>), dim3(blocks), dim3(64), lds, s, a); break;
-    case 32: hipLaunchKernelGGL((vd_mc_kernel<32, MODE, W>), dim3(blocks), dim3(64), lds, s, a); break;
-    case 16: hipLaunchKernelGGL((vd_mc_kernel<16, MODE, W>), dim3(blocks), dim3(64), lds, s, a); break;
+    case 64: hipLaunchKernelGGL((vd_mc_kernel<64, MODE, kBudget<64, MODE, W>>), dim3(blocks), dim3(64), lds, s, a); break;
+    case 32: hipLaunchKernelGGL((vd_mc_kernel<32, MODE, kBudget<32, MODE, W>>), dim3(blocks), dim3(64), lds, s, a); break;
+    case 16: hipLaunchKernelGGL((vd_mc_kernel<16, MODE, kBudget<16, MODE, W>>), dim3(blocks), dim3(64), lds, s, a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -975,9 +959,9 @@ hipError_t launch_mc(int G, int W, const McArgs& a, int blocks, hipStream_t s) {
 template <int MODE, int W>
 static const void* mc_fn_mode(int G) {
   switch (G) {
-    case 64: return reinterpret_cast<const void*>(&vd_mc_kernel<64, MODE, W>);
-    case 32: return reinterpret_cast<const void*>(&vd_mc_kernel<32, MODE, W>);
-    case 16: return reinterpret_cast<const void*>(&vd_mc_kernel<16, MODE, W>);
+    case 64: return reinterpret_cast<const void*>(&vd_mc_kernel<64, MODE, kBudget<64, MODE, W>>);
+    case 32: return reinterpret_cast<const void*>(&vd_mc_kernel<32, MODE, kBudget<32, MODE, W>>);
+    case 16: return reinterpret_cast<const void*>(&vd_mc_kernel<16, MODE, kBudget<16, MODE, W>>);
     default: return nullptr;
   }
 }
@@ -1073,9 +1057,9 @@ static int occupancy(int G, int lds_bytes) {
   int n = 0;
   hipError_t e = hipErrorInvalidValue;
   switch (G) {
-    case 64: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, vd_mc_kernel<64, MODE, W>, 64, lds_bytes); break;
-    case 32: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, vd_mc_kernel<32, MODE, W>, 64, lds_bytes); break;
-    case 16: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, vd_mc_kernel<16, MODE, W>, 64, lds_bytes); break;
+    case 64: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, vd_mc_kernel<64, MODE, kBudget<64, MODE, W>>, 64, lds_bytes); break;
+    case 32: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, vd_mc_kernel<32, MODE, kBudget<32, MODE, W>>, 64, lds_bytes); break;
+    case 16: e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, vd_mc_kernel<16, MODE, kBudget<16, MODE, W>>, 64, lds_bytes); break;
     default: break;
   }
   return e == hipSuccess ? n : 0;
