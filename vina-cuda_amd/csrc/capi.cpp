@@ -208,9 +208,8 @@ struct vd_ctx {
   vd_lig_header eval_header{};
   // vd_eval's kernel takes its own start and end from the device's constant clock: a pair of events
   // around it lengthened every call by 18 us
-  DevBuf<unsigned long long> eval_clock;
-  int clock_khz = 100000;
-  bool eval_timed = false;
+  PinnedBuf<unsigned long long> eval_clock;   // its words, written by the kernel: reading them is no HIP call
+  int clock_khz = 100000, eval_blocks = 0;    // workgroups of the last launch
   DevBuf<float> io_a, io_b, io_c;
   BatchState batch;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -1138,7 +1137,6 @@ int vd_create(int device, vd_ctx** out) {
     HIP_CHECK(hipGetDeviceProperties(&prop, device));
     c->n_cu = prop.multiProcessorCount;
     c->eval_clock.ensure(1 + (size_t)eval_blocks_max(c));
-    HIP_CHECK(hipMemset(c->eval_clock.p, 0, (1 + (size_t)eval_blocks_max(c)) * 8));
     c->lds_max = (int)prop.sharedMemPerBlock;
     c->scratch = scratch_for_current_device(device);
     upload_lut(c);
@@ -1429,13 +1427,14 @@ int vd_eval(vd_ctx* c, int id, long long n, const float* conf, float* e, float* 
     }
     const long long per_block = 64 / G;
     const int blocks = (int)std::min<long long>((n + per_block - 1) / per_block, (long long)eval_blocks_max(c));
+    c->eval_blocks = 0;
     HIP_CHECK(vdl::launch_eval(G, a, blocks, c->stream));
-    c->eval_timed = true;
     if (!direct && !device_ptrs) {
       HIP_CHECK(hipMemcpyAsync(e, a.e, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream));
       HIP_CHECK(hipMemcpyAsync(grad, a.grad, n_out * 4, hipMemcpyDeviceToHost, c->stream));
     }
     HIP_CHECK(hipStreamSynchronize(c->stream));
+    c->eval_blocks = blocks;
     if (direct) {
       std::memcpy(grad, a.grad, n_out * 4);
       std::memcpy(e, a.e, (size_t)n * 4);
@@ -1444,11 +1443,9 @@ int vd_eval(vd_ctx* c, int id, long long n, const float* conf, float* e, float* 
 }
 
 double vd_eval_last_ms(const vd_ctx* c) {
-  if (!c || !c->eval_timed || hipSetDevice(c->device) != hipSuccess) return 0.0;
-  // words of earlier launches' further workgroups hold earlier ticks
-  std::vector<unsigned long long> t(1 + (size_t)eval_blocks_max(c));
-  if (hipMemcpy(t.data(), c->eval_clock.p, t.size() * 8, hipMemcpyDeviceToHost) != hipSuccess) return 0.0;
-  const unsigned long long last = *std::max_element(t.begin() + 1, t.end());
+  if (!c || c->eval_blocks == 0) return 0.0;
+  const unsigned long long* t = c->eval_clock.p;
+  const unsigned long long last = *std::max_element(t + 1, t + 1 + c->eval_blocks);
   return last > t[0] ? (double)(last - t[0]) / c->clock_khz : 0.0;
 }
 
