@@ -1395,15 +1395,15 @@ int vd_eval(vd_ctx* c, int id, long long n, const float* conf, float* e, float* 
     if (n == 0) return;
     const int T = L.n_torsions();
     const int G = pick_group(c, L, cpw);
-    // the record of the ligand last scored stays on the device (a ligand never changes)
+    // the record of the ligand last scored stays on the device (a ligand never changes); another one's is
+    // copied ahead of the kernel, without a wait of its own, and counts as kept once the call is through
+    Packed pk;   // the copy's source, until the wait for the kernel
     if (c->eval_id != id || c->eval_G != G) {
       c->eval_id = -1;
-      Packed pk = pack(c, G, {id});
+      pk = pack(c, G, {id});
       c->blob.ensure(pk.blob.size() / 4 + 1);
       HIP_CHECK(hipMemcpyAsync(c->blob.p, pk.blob.data(), pk.blob.size() * 4, hipMemcpyHostToDevice, c->stream));
-      HIP_CHECK(hipStreamSynchronize(c->stream));   // the copy's source ends with this block
       c->eval_header = pk.headers[0];
-      c->eval_id = id; c->eval_G = G;
     }
     const size_t n_in = (size_t)n * (7 + T), n_out = (size_t)n * (6 + T);
     EvalArgs a{};
@@ -1435,6 +1435,7 @@ int vd_eval(vd_ctx* c, int id, long long n, const float* conf, float* e, float* 
     }
     HIP_CHECK(hipStreamSynchronize(c->stream));
     c->eval_blocks = blocks;
+    c->eval_id = id; c->eval_G = G;
     if (direct) {
       std::memcpy(grad, a.grad, n_out * 4);
       std::memcpy(e, a.e, (size_t)n * 4);
