@@ -68,3 +68,13 @@ def test_every_compiled_form_is_launched(functions):
     assert {n for n in names if n[1] == "0"} == {("64", "0", "2"), ("32", "0", "2"), ("16", "0", "2"), ("64", "0", "3")}
     assert {n for n in names if n[1] != "0"} == {(g, m, w) for g in ("16", "32", "64") for m in "123" for w in "234"}
     assert len([n for n in functions if re.match(r"_ZN12_GLOBAL__N_114vd_grid_kernelILb", n)]) == 2
+
+
+@pytest.mark.parametrize("lanes", [16, 32, 64])
+def test_conformations_on_the_device_are_read_without_exchanges(functions, lanes):
+    """vd_eval_kernel on device memory: every lane loads its own numbers; only conformations in host
+    memory come in one load and are handed round."""
+    body = {host: next(b for n, b in functions.items() if n.startswith("_ZN12_GLOBAL__N_114vd_eval_kernelILi%dELb%dE" % (lanes, host)))
+            for host in (0, 1)}
+    assert not re.search(r"call [^@]*@_ZN3vdk\d+(gbcast|gget)", body[0])
+    assert len(re.findall(r"call [^@]*@_ZN3vdk6gbcast", body[1])) == 7

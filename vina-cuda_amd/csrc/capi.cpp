@@ -1428,7 +1428,7 @@ int vd_eval(vd_ctx* c, int id, long long n, const float* conf, float* e, float* 
     const long long per_block = 64 / G;
     const int blocks = (int)std::min<long long>((n + per_block - 1) / per_block, (long long)eval_blocks_max(c));
     c->eval_blocks = 0;
-    HIP_CHECK(vdl::launch_eval(G, a, blocks, c->stream));
+    HIP_CHECK(vdl::launch_eval(G, direct, a, blocks, c->stream));
     if (!direct && !device_ptrs) {
       HIP_CHECK(hipMemcpyAsync(e, a.e, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream));
       HIP_CHECK(hipMemcpyAsync(grad, a.grad, n_out * 4, hipMemcpyDeviceToHost, c->stream));

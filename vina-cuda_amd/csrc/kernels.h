@@ -90,7 +90,8 @@ hipError_t launch_grid(const float4* atoms, const int2* cells, const GridCells& 
 // Edge records of the maps (VD_XS_SIZE * dim0 (dim1-1)(dim2-1) float4) from the canonical maps,
 // both on the device.
 hipError_t launch_edges(const float* maps, float4* edges, const vd_grid_desc& gd, hipStream_t s);
-hipError_t launch_eval(int G, const EvalArgs& a, int blocks, hipStream_t s);
+// host: the conformations lie in page-locked host memory.
+hipError_t launch_eval(int G, bool host, const EvalArgs& a, int blocks, hipStream_t s);
 hipError_t launch_mc(int G, int W, const McArgs& a, int blocks, hipStream_t s);
 // The kernel function launch_mc launches for these arguments (to find its node in a captured graph).
 const void* mc_kernel_fn(int G, int W, const McArgs& a);

@@ -651,7 +651,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
   }
 }
 
-template <int G>
+// HOST: the conformations lie in host memory, two microseconds away: a conformation's 7 + T <= G
+// numbers in one load, a number per lane, a conformation ahead, handed round by broadcasts.  On the
+// device every lane reads what it needs, when it needs it: the broadcasts (through the LDS for groups of
+// 32) cost resident conformations up to 4 % (300,000 poses, kernel: 24-atom ligand on 64 lanes 605 ->
+// 599 us, 34 atoms on 32 lanes 619 -> 600, 42 atoms 791 -> 780).
+template <int G, bool HOST>
 __global__ __launch_bounds__(64) void vd_eval_kernel(EvalArgs a) {
   extern __shared__ float4 lds4[];
   float* lds = reinterpret_cast<float*>(lds4);
@@ -662,23 +667,27 @@ __global__ __launch_bounds__(64) void vd_eval_kernel(EvalArgs a) {
   LigView L; Scratch S; float* H;
   make_views<G>(a.blob, h, lds, h.n_atoms, h.n_nodes, 0, group, L, S, H);
   const int T = h.n_torsions, nc = 7 + T, ng = 6 + T;
-  // a conformation's 7 + T <= G numbers in one load, a number per lane, a conformation ahead: they
-  // may lie in host memory, two microseconds away
   const auto numbers = [&](long long c) { return l < nc ? a.conf[(c < a.n_conf ? c : 0) * nc + l] : 0.0f; };
   const long long stride = (long long)gridDim.x * CPW;
-  float next = numbers((long long)blockIdx.x * CPW + group);
+  float next = HOST ? numbers((long long)blockIdx.x * CPW + group) : 0.0f;
   stage_ligand<G>(a.blob, h, lds, lane);
   __syncthreads();
   for (long long base = (long long)blockIdx.x * CPW; base < a.n_conf; base += stride) {
     const long long c = base + group;
     const bool valid = c < a.n_conf;
-    const float x = next;
-    if (base + stride < a.n_conf) next = numbers(c + stride);
     Conf cf;
-    cf.px = gbcast<G, 0>(x); cf.py = gbcast<G, 1>(x); cf.pz = gbcast<G, 2>(x);
-    cf.q = Quat{gbcast<G, 3>(x), gbcast<G, 4>(x), gbcast<G, 5>(x), gbcast<G, 6>(x)};
-    const float tor = gget<G>(x, min(l + 6, G - 1));
-    cf.tor = (l >= 1 && l <= T) ? tor : 0.0f;
+    if constexpr (HOST) {
+      const float x = next;
+      if (base + stride < a.n_conf) next = numbers(c + stride);
+      cf.px = gbcast<G, 0>(x); cf.py = gbcast<G, 1>(x); cf.pz = gbcast<G, 2>(x);
+      cf.q = Quat{gbcast<G, 3>(x), gbcast<G, 4>(x), gbcast<G, 5>(x), gbcast<G, 6>(x)};
+      const float tor = gget<G>(x, min(l + 6, G - 1));
+      cf.tor = (l >= 1 && l <= T) ? tor : 0.0f;
+    } else {
+      const float* x = a.conf + (valid ? c : 0) * nc;
+      cf.px = x[0]; cf.py = x[1]; cf.pz = x[2]; cf.q = Quat{x[3], x[4], x[5], x[6]};
+      cf.tor = (l >= 1 && l <= T) ? x[6 + l] : 0.0f;
+    }
     float g;
     const float e = eval_deriv<G>(L, S, a.K, cf, l, g);
     if (valid) {
@@ -886,14 +895,19 @@ hipError_t launch_edges(const float* maps, float4* edges, const vd_grid_desc& gd
   return hipGetLastError();
 }
 
-hipError_t launch_eval(int G, const EvalArgs& a, int blocks, hipStream_t s) {
-  const int lds = mc_lds_bytes(G, a.header.n_atoms, a.header.n_nodes, 0);
+template <bool HOST>
+static void launch_eval_form(int G, const EvalArgs& a, int blocks, int lds, hipStream_t s) {
   switch (G) {
-    case 64: hipLaunchKernelGGL(vd_eval_kernel<64>, dim3(blocks), dim3(64), lds, s, a); break;
-    case 32: hipLaunchKernelGGL(vd_eval_kernel<32>, dim3(blocks), dim3(64), lds, s, a); break;
-    case 16: hipLaunchKernelGGL(vd_eval_kernel<16>, dim3(blocks), dim3(64), lds, s, a); break;
-    default: return hipErrorInvalidValue;
+    case 64: hipLaunchKernelGGL((vd_eval_kernel<64, HOST>), dim3(blocks), dim3(64), lds, s, a); break;
+    case 32: hipLaunchKernelGGL((vd_eval_kernel<32, HOST>), dim3(blocks), dim3(64), lds, s, a); break;
+    default: hipLaunchKernelGGL((vd_eval_kernel<16, HOST>), dim3(blocks), dim3(64), lds, s, a);
   }
+}
+hipError_t launch_eval(int G, bool host, const EvalArgs& a, int blocks, hipStream_t s) {
+  if (G != 64 && G != 32 && G != 16) return hipErrorInvalidValue;
+  const int lds = mc_lds_bytes(G, a.header.n_atoms, a.header.n_nodes, 0);
+  if (host) launch_eval_form<true>(G, a, blocks, lds, s);
+  else launch_eval_form<false>(G, a, blocks, lds, s);
   return hipGetLastError();
 }
 
