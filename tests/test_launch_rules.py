@@ -1,0 +1,39 @@
+"""The launch rules on the host: the header is compiled into a small library of its own, so every line
+is checked without a device.  256 compute units, an MI355X's."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+CUS = 256
+SHIM = """
+#include "launch_rules.h"
+extern "C" {
+int refine_waves(int n_cu, long long poses, long long atoms) { return vd::refine_waves(n_cu, poses, atoms); }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    (d / "shim.cpp").write_text(SHIM)
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC",
+                           "-I", os.path.join(ROOT, "vina-cuda_amd", "csrc"), "-o", str(d / "shim.so"), str(d / "shim.cpp")])
+    return C.CDLL(str(d / "shim.so"))
+
+
+# (atoms of every ligand, poses, wavefronts per pose): sizes at which one of the two took at least 1.1
+# times the other's time
+@pytest.mark.parametrize("atoms,poses,waves", [
+    (1, 20, 1), (3, 500, 1), (6, 1000, 1), (11, 500, 4), (11, 1000, 1), (11, 2000, 1), (14, 1000, 4), (14, 2000, 1),
+    (17, 1100, 4), (17, 1800, 1), (21, 1400, 4), (24, 1100, 4), (24, 2000, 1), (28, 1500, 4), (34, 2000, 4), (42, 2000, 4),
+    (64, 2000, 4), (64, 2049, 1), (64, 5120, 1), (42, 20, 4)])
+def test_refinement_takes_the_faster_form(rules, atoms, poses, waves):
+    f = rules.refine_waves
+    f.argtypes = [C.c_int, C.c_longlong, C.c_longlong]
+    assert f(CUS, poses, atoms * poses) == waves
+    assert f(CUS, 0, 0) == 1

@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "host_model.h"
+#include "launch_rules.h"
 #include "kernels.h"
 
 namespace {
@@ -924,18 +925,6 @@ vdr::RefHeader pack_ref(const vd::Ligand& L, std::vector<double4>& geo, std::vec
   return h;
 }
 
-// Wavefronts per pose of a refinement launch.  A pose takes some 100 evaluations one after the other,
-// so a launch takes at least as long as its longest pose: four wavefronts per pose halve that
-// (20 poses of a 63-atom ligand 4.1 -> 2.0 ms), at the price of the slots in which three wait while
-// the first walks the tree.  As long as one wavefront per pose would leave no pose waiting for a slot
-// (eight per CU at the kernel's registers) the shorter pose is the shorter launch: 2,000 poses of
-// 63-atom ligands 14.8 -> 12.6 ms, of 41-atom ones 7.5 -> 6.8, of 21-atom ones 3.0 -> 3.2; beyond,
-// throughput counts (5,120 poses 19.7 -> 20.5, 10.7 -> 12.1, 4.4 -> 6.6 ms).  Ligands whose team does
-// not fit the LDS of a workgroup take one wavefront.
-int refine_waves(const vd_ctx* c, long long poses, int Amax, int Nmax, int nmax) {
-  return poses <= 8LL * c->n_cu && vdl::refine_lds_bytes(4, Amax, Nmax, nmax) <= c->lds_max ? 4 : 1;
-}
-
 // One refinement launch over poses of several ligands: ligand ids[k] owns poses[k] poses, their
 // conformations concatenated in conf.  Fills per pose the refined conformation, all-atom
 // coordinates and vd_refined.
@@ -956,14 +945,16 @@ RefineOut run_refine(vd_ctx* c, const std::vector<int>& ids, const std::vector<i
   std::vector<uint16_t> ent;
   std::vector<vdr::RefHeader> hdr;
   int Amax = 1, Nmax = 1, nmax = 1;
-  long long n_poses = 0;
+  long long n_poses = 0, pose_atoms = 0;
   for (size_t k = 0; k < ids.size(); ++k) {
     const vd::Ligand& L = lig_at(c, ids[k]);
     Amax = std::max(Amax, (int)L.atoms.size()); Nmax = std::max(Nmax, (int)L.nodes.size());
     nmax = std::max(nmax, 6 + L.n_torsions());
     n_poses += std::max(poses[k], 0);
+    pose_atoms += (long long)std::max(poses[k], 0) * (int)L.atoms.size();
   }
-  const int waves = refine_waves(c, n_poses, Amax, Nmax, nmax);
+  int waves = vd::refine_waves(c->n_cu, n_poses, pose_atoms);
+  if (vdl::refine_lds_bytes(waves, Amax, Nmax, nmax) > c->lds_max) waves = 1;   // a team that does not fit
   for (int id : ids) {
     const vd::Ligand& L = lig_at(c, id);
     if (L.n_torsions() + 7 > 64) throw ArgError(VD_ERR_CAPACITY, "ligand has too many torsions for the refinement");

@@ -1,0 +1,28 @@
+// Launch shapes chosen by size, as plain host functions (no HIP types), so that each line can be checked
+// without a device.
+#pragma once
+#include <algorithm>
+
+namespace vd {
+
+// Wavefronts per pose of a refinement launch of `poses` poses with `pose_atoms` atoms in all, on n_cu
+// compute units.  A pose takes some 100 evaluations one after the other, so a launch takes at least as
+// long as its longest pose: four wavefronts per pose halve that (20 poses of a 63-atom ligand 4.1 ->
+// 2.0 ms), at the price of the slots in which three wait while the first walks the tree.  As long as one
+// wavefront per pose would leave no pose waiting for a slot (eight per CU at the kernel's registers) the
+// shorter pose is the shorter launch for ligands of some 35 atoms and more: 2,000 poses of 63-atom ligands
+// 14.8 -> 12.6 ms, of 41-atom ones 7.5 -> 6.8; beyond, throughput counts (5,120 poses 19.7 -> 20.5, 10.7
+// -> 12.1 ms).  A smaller ligand's team shares less work, and two or three teams per CU already take
+// longer than eight single wavefronts.  Time of one wavefront over time of four, by atoms: 6 atoms 0.95 at
+// 20 poses, 0.52 at 2,000; 11 atoms 1.14 up to 600 poses, 1.11 at 800, 0.90 at 1,000, 0.58 at 2,000; 14
+// 1.33 at 1,000, 1.02 at 1,200, 0.82 at 2,000; 21 1.19 at 1,400, 1.02 at 1,700, 0.94 at 2,000; 24 1.20 at
+// 1,100, 0.88 at 1,500; 28 1.26 at 1,400, 1.12 at 2,000.  The line runs between, from 3 poses per CU at
+// 10 atoms to 8 at 30.
+inline int refine_waves(int n_cu, long long poses, long long pose_atoms) {
+  if (poses <= 0) return 1;
+  const double atoms = (double)pose_atoms / poses;
+  if (atoms < 10) return 1;
+  return poses <= std::min(8.0, 3.0 + 0.25 * (atoms - 10)) * n_cu ? 4 : 1;
+}
+
+}  // namespace vd
