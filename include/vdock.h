@@ -160,14 +160,14 @@ typedef struct {
 /* One MC kernel launch of the last vd_dock / vd_dock_batch / vd_dock_batch_plain call (the
  * autotuner's trial launches excluded), in launch order.  The kernel is
  * vd_mc_kernel<lanes_per_chain, mode, waves_per_simd>; mode 0 dense BFGS, 1 RILC-BFGS,
- * 2 RILC-BFGS with the QuickVina2 history; a first record of lanes_per_chain 16 with one item per
- * chain is vd_mc_wide_kernel<mode> (vd_set_class_overlap).  eval_bytes = algorithmic bytes of its evaluations:
- * per evaluation 32 B per heavy atom (eight map corners) and 16 B per intramolecular pair (one
+ * 2 RILC-BFGS with the QuickVina2 history, 3 with QuickVina-W's; with wide = 1 it is
+ * vd_mc_wide_kernel of the same arguments (vd_set_class_overlap), one chain per wavefront in the
+ * arithmetic of lanes_per_chain = 16.  eval_bytes = algorithmic bytes of its evaluations: per evaluation 32 B per heavy atom (eight map corners) and 16 B per intramolecular pair (one
  * interpolation quad of the pair table).  No counterpart in the reference (which prints only
  * per-ligand kernel times, V11/lib/main_procedure_cu.cpp:975-994); it serves the roofline measurement. */
 typedef struct {
   int lanes_per_chain, mode, waves_per_simd;
-  int blocks, items, ligands, persistent;
+  int blocks, items, ligands, persistent, wide;
   double kernel_ms;
   unsigned long long evals;
   double eval_bytes;

@@ -122,6 +122,7 @@ struct McSlot {
   }
 };
 constexpr size_t kEvalDirectBytes = 4u << 20;   // vd_eval's host arrays the kernel reads and writes in place
+static_assert(sizeof(vd_launch) == 64, "callers hold arrays of it");
 constexpr int kMcSlots = 4;   // at most four hardware queues per process on these devices
 
 // A persistent batch captured as a hipGraph (vd_set_graphs): every stage of one vd_dock_batch
@@ -554,7 +555,7 @@ void mc_prepare(vd_ctx* c, McSlot& s, int G, int W, Packed&& pk, std::vector<uin
     throw ArgError(VD_ERR_CAPACITY, "ligand too large for the LDS layout (" + std::to_string(lds) + " bytes of " +
                                         std::to_string(c->lds_max) + " per workgroup)");
   const int mode = mc_mode(P);
-  W = wide ? 2 : loosest_budget(G, W, mode, lds);
+  W = wide ? vdl::kWideWaves : loosest_budget(G, W, mode, lds);
   int blocks = (int)s.h_items.size();
   if (persistent) {
     a.queue = s.queue.p;
@@ -574,7 +575,7 @@ void mc_prepare(vd_ctx* c, McSlot& s, int G, int W, Packed&& pk, std::vector<uin
   s.G = G; s.W = W; s.wide = wide; s.blocks = blocks; s.persistent = persistent;
   s.rec = vd_launch{};
   s.rec.lanes_per_chain = G; s.rec.waves_per_simd = W; s.rec.blocks = blocks; s.rec.items = (int)s.h_items.size();
-  s.rec.ligands = (int)s.h_headers.size(); s.rec.persistent = persistent ? 1 : 0;
+  s.rec.ligands = (int)s.h_headers.size(); s.rec.persistent = persistent ? 1 : 0; s.rec.wide = wide ? 1 : 0;
   s.rec.mode = mode;
   s.h_evals.assign(s.h_headers.size(), 0);
 }

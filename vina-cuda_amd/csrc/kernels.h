@@ -81,7 +81,9 @@ int refine_lds_bytes(int waves, int Amax, int Nmax, int nmax);
 hipError_t launch_refine(int waves, const RefineArgs& a, int poses, hipStream_t s);   // waves per pose: 1 or 4
 int mc_lds_bytes(int G, int Amax, int Nmax, int dense);
 int max_resident_mc_blocks(int G, int W, int mode, int lds_bytes);
-// Wide launches (one chain per wavefront in 16-lane arithmetic; modes 0 to 2, persistent only)
+// Wide launches (one chain per wavefront in 16-lane arithmetic; modes 0 to 2, persistent only), built for
+// kWideWaves waves per SIMD
+constexpr int kWideWaves = 3;
 int wide_lds_bytes(int Amax, int Nmax, int dense);
 int max_resident_wide_blocks(int mode, int lds_bytes);
 hipError_t launch_mc_wide(const McArgs& a, int blocks, hipStream_t s);

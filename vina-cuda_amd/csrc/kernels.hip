@@ -614,11 +614,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W, 8))) void
   }
 }
 
-// A wide launch's chains: items are (ligand slot, chain).  Three waves per SIMD (168 registers, 184
-// bytes of spills) against two (217, none): large-box QuickVina2 batch of 200 ligands 149 against
-// 163 ms, dense BFGS of 96 the same.
-template <int MODE>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void vd_mc_wide_kernel(McArgs a) {
+// A wide launch's chains: items are (ligand slot, chain).  Three waves per SIMD (168 registers; 236
+// bytes of spills under dense BFGS, 184 under RILC-BFGS, 336 with the QuickVina2 history) against two
+// (217 and none under RILC-BFGS): large-box QuickVina2 batch of 200 ligands 149 against 163 ms, dense
+// BFGS of 96 the same.
+// Its template arguments are vd_mc_kernel's: lanes whose arithmetic it takes, mode, waves per SIMD.
+template <int G, int MODE, int W>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W, 8))) void vd_mc_wide_kernel(McArgs a) {
+  static_assert(G == 16, "");
   extern __shared__ float4 lds4[];
   float* lds = reinterpret_cast<float*>(lds4);
   const int lane = threadIdx.x, l = lane & 15;
@@ -916,18 +919,18 @@ int wide_lds_bytes(int Amax, int Nmax, int dense) { return 4 * (lig_floats(Amax,
 hipError_t launch_mc_wide(const McArgs& a, int blocks, hipStream_t s) {
   const int lds = wide_lds_bytes(a.Amax, a.Nmax, a.P.local_search == 0);
   if (!a.queue || !a.items || (a.P.policy == 1 && !a.hist) || a.P.policy == 2) return hipErrorInvalidValue;
-  if (a.P.local_search == 0) hipLaunchKernelGGL(vd_mc_wide_kernel<0>, dim3(blocks), dim3(64), lds, s, a);
-  else if (a.P.policy == 1) hipLaunchKernelGGL(vd_mc_wide_kernel<2>, dim3(blocks), dim3(64), lds, s, a);
-  else hipLaunchKernelGGL(vd_mc_wide_kernel<1>, dim3(blocks), dim3(64), lds, s, a);
+  if (a.P.local_search == 0) hipLaunchKernelGGL((vd_mc_wide_kernel<16, 0, kWideWaves>), dim3(blocks), dim3(64), lds, s, a);
+  else if (a.P.policy == 1) hipLaunchKernelGGL((vd_mc_wide_kernel<16, 2, kWideWaves>), dim3(blocks), dim3(64), lds, s, a);
+  else hipLaunchKernelGGL((vd_mc_wide_kernel<16, 1, kWideWaves>), dim3(blocks), dim3(64), lds, s, a);
   return hipGetLastError();
 }
 
 int max_resident_wide_blocks(int mode, int lds_bytes) {
   int n = 0;
   const hipError_t e =
-      mode == 0 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, vd_mc_wide_kernel<0>, 64, lds_bytes)
-      : mode == 2 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, vd_mc_wide_kernel<2>, 64, lds_bytes)
-                  : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, vd_mc_wide_kernel<1>, 64, lds_bytes);
+      mode == 0 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, vd_mc_wide_kernel<16, 0, kWideWaves>, 64, lds_bytes)
+      : mode == 2 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, vd_mc_wide_kernel<16, 2, kWideWaves>, 64, lds_bytes)
+                  : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, vd_mc_wide_kernel<16, 1, kWideWaves>, 64, lds_bytes);
   return e == hipSuccess ? n : 0;
 }
 

@@ -85,13 +85,14 @@ class Mode(C.Structure):
 
 class Launch(C.Structure):
     _fields_ = [("lanes_per_chain", C.c_int), ("mode", C.c_int), ("waves_per_simd", C.c_int), ("blocks", C.c_int),
-                ("items", C.c_int), ("ligands", C.c_int), ("persistent", C.c_int), ("kernel_ms", C.c_double),
+                ("items", C.c_int), ("ligands", C.c_int), ("persistent", C.c_int), ("wide", C.c_int), ("kernel_ms", C.c_double),
                 ("evals", C.c_ulonglong), ("eval_bytes", C.c_double), ("start_ms", C.c_double)]
 
     @property
     def kernel(self):
         """Name of the launched kernel as a profiler lists it (template arguments)."""
-        return "vd_mc_kernel<%d, %d, %d>" % (self.lanes_per_chain, self.mode, self.waves_per_simd)
+        return "%s<%d, %d, %d>" % ("vd_mc_wide_kernel" if self.wide else "vd_mc_kernel",
+                                   self.lanes_per_chain, self.mode, self.waves_per_simd)
 
 
 _lib = None
