@@ -13,6 +13,15 @@ SHIM = """
 #include "launch_rules.h"
 extern "C" {
 int refine_waves(int n_cu, long long poses, long long atoms) { return vd::refine_waves(n_cu, poses, atoms); }
+// (lanes, waves, wide) per ligand -> launches (size, first ligand of each to out), overlap
+int classes(int n, const int* lanes, const int* waves, const int* wide, int* out, int* overlap) {
+  std::vector<vd::LigPlan> plans;
+  for (int k = 0; k < n; ++k) plans.push_back(vd::LigPlan{k, lanes[k], waves[k], 1, 1, 1, 1, 1, wide[k] != 0});
+  const vd::Classes c = vd::batch_classes(plans);
+  for (const auto& e : c) { *out++ = (int)e.second.size(); *out++ = e.second[0]; }
+  *overlap = vd::may_overlap(c);
+  return (int)c.size();
+}
 }
 """
 
@@ -37,3 +46,25 @@ def test_refinement_takes_the_faster_form(rules, atoms, poses, waves):
     f.argtypes = [C.c_int, C.c_longlong, C.c_longlong]
     assert f(CUS, poses, atoms * poses) == waves
     assert f(CUS, 0, 0) == 1
+
+
+def classes(rules, plans):
+    n = len(plans)
+    a = [(C.c_int * n)(*col) for col in zip(*plans)]
+    out, overlap = (C.c_int * (2 * n))(), C.c_int()
+    k = rules.classes(n, *a, out, C.byref(overlap))
+    return [(out[2 * i], out[2 * i + 1]) for i in range(k)], bool(overlap.value)
+
+
+def test_wide_ligands_of_any_budget_share_one_launch(rules):
+    # two 16-lane budgets, as the autotuner may choose, heavy ligands in both
+    assert classes(rules, [(16, 3, 0), (16, 4, 0), (16, 3, 1), (16, 4, 1)]) == ([(2, 2), (1, 0), (1, 1)], True)
+    assert classes(rules, [(16, 3, 1), (64, 3, 0), (16, 3, 0)]) == ([(1, 0), (1, 2), (1, 1)], True)
+    assert classes(rules, [(16, 3, 1), (16, 2, 1)]) == ([(2, 0)], False)
+
+
+def test_classes_that_run_one_after_the_other(rules):
+    assert classes(rules, [(16, 3, 0), (64, 3, 0)]) == ([(1, 0), (1, 1)], True)
+    assert classes(rules, [(16, 3, 0)]) == ([(1, 0)], False)
+    assert classes(rules, [(16, 3, 0), (32, 3, 0), (64, 3, 0)])[1] is False
+    assert classes(rules, [(16, 3, 1), (16, 3, 0), (32, 3, 0), (64, 3, 0)])[1] is False

@@ -652,7 +652,7 @@ void run_mc(vd_ctx* c, int G, int W, const Packed& pk, const std::vector<uint32_
   mc_collect(c, s, st, nullptr);
 }
 
-struct LigPlan { int id, G, W, depth, bfgs, T, H, chains; bool wide = false; };
+using vd::LigPlan;
 // single_launch: the ligand gets a launch of its own (vd_dock, the plain per-ligand loop).  Its
 // only parallelism is its chains, so unless they fill two waves per SIMD at the tuned width, it
 // runs one chain per wavefront, the most wavefronts such a launch can have.
@@ -1641,17 +1641,9 @@ int vd_dock_noalloc(vd_ctx* c, int id, const vd_dock_params* p, const float* d_i
 
 namespace {
 
-// The launch classes of a persistent batch: ligand indices per launch form, wide launches first.
-struct ClassKey {
-  int narrow, G, W;   // narrow: 0 for a wide launch; lanes per chain, waves per SIMD
-  bool operator<(const ClassKey& o) const { return std::tie(narrow, G, W) < std::tie(o.narrow, o.G, o.W); }
-};
-using Classes = std::map<ClassKey, std::vector<int>>;
-Classes batch_classes(const std::vector<LigPlan>& plans) {
-  Classes classes;
-  for (size_t k = 0; k < plans.size(); ++k) classes[ClassKey{plans[k].wide ? 0 : 1, plans[k].G, plans[k].W}].push_back((int)k);
-  return classes;
-}
+using vd::batch_classes;
+using vd::ClassKey;
+using vd::Classes;
 
 // Estimated cost of a work item (the chains of one wavefront): steps x iterations x (atoms + pairs).
 double item_cost(const LigPlan& pl, int atoms, int pair_slots) { return (double)pl.depth * pl.bfgs * (atoms + 0.5 * pair_slots + 16); }
@@ -1711,15 +1703,7 @@ void wide_ligands(vd_ctx* c, std::vector<LigPlan>& plans, const vd_dock_params* 
     if (can(k) && units[k] > line) plans[k].wide = true;
 }
 
-// Overlap applies to batches of exactly two classes, besides a wide launch.  Measured on the
-// screening batch (a 16-lane class whose waves mostly wait, a 64-lane class that keeps the vector
-// units busy): 3 % shorter steps.  With more classes it lost: on a 4,096-ligand batch of five classes a fourth stream
-// shared a hardware queue with the third (four queues per process), and capped classes that
-// outlast the uncapped one keep half their CU slots empty to the end.
-bool overlap_of(const vd_ctx* c, const Classes& classes) {
-  const size_t wide = !classes.empty() && classes.begin()->first.narrow == 0;
-  return c->overlap_classes && (classes.size() == 2 || (wide && classes.size() == 3));
-}
+bool overlap_of(const vd_ctx* c, const Classes& classes) { return c->overlap_classes && vd::may_overlap(classes); }
 
 // Host work of one class of a persistent batch -- its ligand records, launch tables and work items
 // in decreasing estimated cost -- prepared into launch slot s.  share: the fraction of its resident
