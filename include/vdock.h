@@ -136,7 +136,8 @@ typedef struct {
   int policy;            /* VD_MC_VINA, VD_MC_QVINA2 or VD_MC_QVINAW (the last two with RILC-BFGS) */
   int mutation_quirk;    /* 1: mutate one of 1+T entities like the reference GPU host tables */
   int chains_per_wave;   /* 1, 2, 4; 0 = per ligand size bucket (vd_set_autotune) */
-  int waves_per_simd;    /* register budget of the MC kernel: 2, 3 or 4 resident waves per SIMD; 0 = per size bucket */
+  int waves_per_simd;    /* register budget of the MC kernel: 2, 3 or 4 resident waves per SIMD; 0 = per size bucket
+                            (dense BFGS: 2, and with 0 three for the 64-lane class of a batch) */
   uint32_t seed;         /* chain c of ligand id draws from the Philox stream keyed (seed, id) at
                             counter c: ids count from 0 in the order of vd_add_ligand, as the
                             reference's ligands count in the order of its batch */

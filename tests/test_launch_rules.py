@@ -13,6 +13,12 @@ SHIM = """
 #include "launch_rules.h"
 extern "C" {
 int refine_waves(int n_cu, long long poses, long long atoms) { return vd::refine_waves(n_cu, poses, atoms); }
+int dense_waves(int lanes, int batch) { return vd::dense_waves(lanes, batch != 0); }
+int trial_waves(int lanes, int rilc, int batch, int* out) {
+  const std::vector<int> w = vd::trial_waves(lanes, rilc != 0, batch != 0);
+  std::copy(w.begin(), w.end(), out);
+  return (int)w.size();
+}
 // (lanes, waves, wide) per ligand -> launches (size, first ligand of each to out), overlap
 int classes(int n, const int* lanes, const int* waves, const int* wide, int* out, int* overlap) {
   std::vector<vd::LigPlan> plans;
@@ -68,3 +74,12 @@ def test_classes_that_run_one_after_the_other(rules):
     assert classes(rules, [(16, 3, 0)]) == ([(1, 0)], False)
     assert classes(rules, [(16, 3, 0), (32, 3, 0), (64, 3, 0)])[1] is False
     assert classes(rules, [(16, 3, 1), (16, 3, 0), (32, 3, 0), (64, 3, 0)])[1] is False
+
+
+@pytest.mark.parametrize("lanes", [16, 32, 64])
+@pytest.mark.parametrize("batch", [0, 1])
+def test_autotuner_times_what_the_call_runs(rules, lanes, batch):
+    out = (C.c_int * 4)()
+    trials = out[:rules.trial_waves(lanes, 0, batch, out)]
+    assert trials == [rules.dense_waves(lanes, batch)] == [3 if lanes == 64 and batch else 2]
+    assert out[:rules.trial_waves(lanes, 1, batch, out)] == [3, 4, 2]

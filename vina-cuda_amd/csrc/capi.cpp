@@ -663,11 +663,7 @@ LigPlan plan_for(vd_ctx* c, int id, const vd_dock_params* p, bool single_launch)
   pl.G = pick_group(c, L, p->chains_per_wave);
   if (single_launch && p->chains_per_wave == 0 && (long long)p->chains * pl.G / 64 < 8LL * std::max(c->n_cu, 1)) pl.G = 64;
   pl.W = p->waves_per_simd ? p->waves_per_simd : pick_waves(c, L, pl.G);
-  // Dense BFGS: three waves per SIMD (168 registers, 144 bytes of spills) for the 64-lane class of a batch
-  // (nine batches of 96 ligands 1,385 -> 1,344 ms with the 16-lane class at three as well, which alone
-  // loses: 123 -> 130 ms); a launch of one ligand rarely has the chains for a third (24 atoms, 2,048
-  // chains 18.4 -> 19.2 ms).
-  if (p->local_search != VD_LS_RILC_BFGS) pl.W = pl.G == 64 && !single_launch && p->waves_per_simd == 0 ? 3 : 2;
+  if (p->local_search != VD_LS_RILC_BFGS) pl.W = p->waves_per_simd ? 2 : vd::dense_waves(pl.G, !single_launch);
   const int rilc = p->local_search == VD_LS_RILC_BFGS;
   pl.depth = p->search_depth > 0 ? p->search_depth : heur_depth((int)L.atoms.size(), pl.T, rilc);
   pl.bfgs = p->bfgs_steps > 0 ? p->bfgs_steps : heur_bfgs((int)L.atoms.size(), rilc);
@@ -677,14 +673,14 @@ LigPlan plan_for(vd_ctx* c, int id, const vd_dock_params* p, bool single_launch)
 
 // Autotuner: for every size bucket of the batch not tuned yet, a representative ligand docks the
 // same fixed work -- 64 chains per CU (enough to fill every wavefront slot at four chains per
-// wavefront and four wavefronts per SIMD), at most six MC steps -- under each admissible
-// (lanes per chain, waves per SIMD) pair, in a persistent launch whose LDS layout is sized for the
+// wavefront and four wavefronts per SIMD), at most six MC steps -- under each (lanes per chain, waves
+// per SIMD) pair that the call (batch: a batched one) may run, in a persistent launch whose LDS layout is sized for the
 // whole batch as the batched launch's is.  The pairs within 10 % of the fastest run again and
 // keep their shorter time; among those within 2 % of the fastest, the first in a fixed preference
 // order wins (wider groups first, then 3, 4, 2 waves per SIMD), so that timing noise does not flip
 // the choice between runs.  Every chain follows the same trajectory under every pair up to
 // rounding (the random stream does not depend on the layout), so the work is the same.
-void autotune(vd_ctx* c, const std::vector<int>& ids, const vd_dock_params* p) {
+void autotune(vd_ctx* c, const std::vector<int>& ids, const vd_dock_params* p, bool batch) {
   std::map<int, int> rep;
   for (int id : ids) { const int b = size_bucket(lig_at(c, id)); if (!c->tuned.count(b) && !rep.count(b)) rep[b] = id; }
   if (rep.empty()) return;
@@ -706,8 +702,7 @@ void autotune(vd_ctx* c, const std::vector<int>& ids, const vd_dock_params* p) {
     struct Trial { int G, W, W_run; double ms; };
     std::vector<Trial> trials;   // preference order
     for (int G = 64; G >= gmin; G /= 2)
-      for (int W : {3, 4, 2})
-        if (rilc || W == 2) trials.push_back({G, W, W, 1e300});
+      for (int W : vd::trial_waves(G, rilc, batch)) trials.push_back({G, W, W, 1e300});
     auto run = [&](Trial& t) {
       vd_dock_params q = *p;
       q.chains = chains; q.chains_per_wave = 64 / t.G;
@@ -1485,7 +1480,7 @@ void dock_one(vd_ctx* c, int id, const vd_dock_params* p, const float* init_conf
   need_device(c);
   if (!c->maps_ready) throw ArgError(VD_ERR_ARG, "no maps");
   if (st) std::memset(st, 0, sizeof(*st));
-  if (c->autotune_on && (p->chains_per_wave == 0 || p->waves_per_simd == 0)) autotune(c, {id}, p);
+  if (c->autotune_on && (p->chains_per_wave == 0 || p->waves_per_simd == 0)) autotune(c, {id}, p, false);
   c->launches.clear();
   pl = plan_for(c, id, p, true);
   if (ls_only) pl.depth = 0;
@@ -1942,7 +1937,7 @@ static int dock_many(vd_ctx* c, int n, const int* ids, const vd_dock_params* p, 
     if (!c->maps_ready) throw ArgError(VD_ERR_ARG, "no maps");
     if (st) std::memset(st, 0, sizeof(*st));
     if (c->autotune_on && (p->chains_per_wave == 0 || p->waves_per_simd == 0))
-      autotune(c, std::vector<int>(ids, ids + n), p);
+      autotune(c, std::vector<int>(ids, ids + n), p, persistent);
     c->launches.clear();
     std::vector<LigPlan> plans;
     for (int k = 0; k < n; ++k) plans.push_back(plan_for(c, ids[k], p, !persistent));

@@ -39,6 +39,17 @@ inline bool may_overlap(const Classes& classes) {
   return classes.size() == 2 || (wide && classes.size() == 3);
 }
 
+// Waves per SIMD of a dense-BFGS launch: three (168 registers, 144 bytes of spills) for the 64-lane class
+// of a batch (nine batches of 96 ligands 1,427 -> 1,311 ms); on 16 lanes a third loses (123 -> 130 ms),
+// and a launch of one ligand rarely has the chains for it (24 atoms, 2,048 chains 18.4 -> 19.2 ms).
+inline int dense_waves(int G, bool batch) { return G == 64 && batch ? 3 : 2; }
+
+// The budgets the autotuner times for G lanes per chain, in order of preference: those that the call
+// would run.
+inline std::vector<int> trial_waves(int G, bool rilc, bool batch) {
+  return rilc ? std::vector<int>{3, 4, 2} : std::vector<int>{dense_waves(G, batch)};
+}
+
 // Wavefronts per pose of a refinement launch of `poses` poses with `pose_atoms` atoms in all, on n_cu
 // compute units.  A pose takes some 100 evaluations one after the other, so a launch takes at least as
 // long as its longest pose: four wavefronts per pose halve that (20 poses of a 63-atom ligand 4.1 ->
