@@ -13,6 +13,7 @@ SHIM = """
 #include "launch_rules.h"
 extern "C" {
 int refine_waves(int n_cu, long long poses, long long atoms) { return vd::refine_waves(n_cu, poses, atoms); }
+size_t grown_size(size_t have, size_t need, size_t least, size_t most) { return vd::grown_size(have, need, least, most); }
 int dense_waves(int lanes, int batch) { return vd::dense_waves(lanes, batch != 0); }
 int trial_waves(int lanes, int rilc, int batch, int* out) {
   const std::vector<int> w = vd::trial_waves(lanes, rilc != 0, batch != 0);
@@ -83,3 +84,19 @@ def test_autotuner_times_what_the_call_runs(rules, lanes, batch):
     trials = out[:rules.trial_waves(lanes, 0, batch, out)]
     assert trials == [rules.dense_waves(lanes, batch)] == [3 if lanes == 64 and batch else 2]
     assert out[:rules.trial_waves(lanes, 1, batch, out)] == [3, 4, 2]
+
+
+def test_growing_arrays_cost_few_allocations(rules):
+    f = rules.grown_size
+    f.argtypes, f.restype = [C.c_size_t] * 4, C.c_size_t
+    least, most = 4096, 1 << 20
+    have, allocations = 0, 0
+    for need in range(1, most + 1, 97):
+        new = f(have, need, least, most)
+        assert need <= new <= most and new >= least
+        allocations += new != have
+        have = new
+    assert allocations <= 10
+    assert f(0, 300000, least, most) == 300000   # the first one takes what it needs
+    assert f(5000, 100, least, most) == 5000
+    assert f(900000, 1000000, least, most) == most

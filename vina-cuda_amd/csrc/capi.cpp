@@ -121,7 +121,12 @@ struct McSlot {
     ev0 = ev1 = nullptr; stream = nullptr;   // the streams are the process's (device_stream)
   }
 };
-constexpr size_t kEvalDirectBytes = 4u << 20;   // vd_eval's host arrays the kernel reads and writes in place
+// vd_eval's host arrays the kernel reads and writes in place, at most.  Copied -> in place, by size: 56 KB
+// 65 -> 20 us, 350 KB 61 -> 36, 1.3 MB 107 -> 89, 2.3 MB 212 -> 185, 3.4 MB 215 -> 218, 3.7 MB 341 -> 312,
+// 6 MB 442 -> 466, 10 MB 880 -> 730, 14.9 MB 1,277 -> 1,070: mixed from 3 MB on, and page-locked memory
+// costs some 0.3 us per KB when it is taken.
+constexpr size_t kEvalDirectBytes = 4u << 20;
+constexpr size_t kEvalLeastFloats = 16384;   // of the memory first taken for them
 static_assert(sizeof(vd_launch) == 64, "callers hold arrays of it");
 constexpr int kMcSlots = 4;   // at most four hardware queues per process on these devices
 
@@ -241,6 +246,7 @@ struct vd_ctx {
   DevBuf<long long> ref_coff, ref_xoff;
   PostState post;
   PinnedBuf<float> pin_eval;                     // vd_eval's small host arrays, read and written by the kernel
+  std::vector<PinnedBuf<float>> pin_eval_old;    // smaller ones it has grown out of
   PinnedBuf<float> pin_e, pin_conf, pin_heavy;   // per-chain results of a batch, for pose lists
   PinnedBuf<double> pin_cout, pin_xout;          // refinement outputs
   PinnedBuf<double4> pin_res;
@@ -1155,6 +1161,7 @@ void vd_destroy(vd_ctx* c) {
   c->ref_res.release(); c->ref_lig.release(); c->ref_order.release(); c->ref_evals.release(); c->ref_coff.release(); c->ref_xoff.release();
   c->lutd.release(); c->ref_rows.release(); c->ref_geo.release(); c->ref_ent.release(); c->ref_pairs.release(); c->ref_hdr.release();
   c->pin_eval.release(); c->eval_clock.release();
+  for (PinnedBuf<float>& b : c->pin_eval_old) b.release();
   c->pin_e.release(); c->pin_conf.release(); c->pin_heavy.release();
   c->pin_cout.release(); c->pin_xout.release(); c->pin_res.release();
   if (c->ev0) (void)hipEventDestroy(c->ev0);
@@ -1404,7 +1411,14 @@ int vd_eval(vd_ctx* c, int id, long long n, const float* conf, float* e, float* 
     // and a second pass over them on the host would cost more than the copies.
     const bool direct = !device_ptrs && (n_in + n_out + (size_t)n) * 4 <= kEvalDirectBytes;
     if (direct) {
-      c->pin_eval.ensure(n_in + n_out + (size_t)n);
+      const size_t size = vd::grown_size(c->pin_eval.n, n_in + n_out + (size_t)n, kEvalLeastFloats, kEvalDirectBytes / 4);
+      if (size > c->pin_eval.n) {
+        // the one it grows out of is kept until the context ends: giving it back takes some 400 us, and
+        // all of them together are smaller than the last
+        if (c->pin_eval.p) c->pin_eval_old.push_back(c->pin_eval);
+        c->pin_eval = PinnedBuf<float>();
+        c->pin_eval.ensure(size);
+      }
       std::memcpy(c->pin_eval.p, conf, n_in * 4);
       a.conf = c->pin_eval.p; a.grad = c->pin_eval.p + n_in; a.e = c->pin_eval.p + n_in + n_out;
     } else if (!device_ptrs) {

@@ -2,11 +2,21 @@
 // without a device.
 #pragma once
 #include <algorithm>
+#include <cstddef>
 #include <map>
 #include <tuple>
 #include <vector>
 
 namespace vd {
+
+// The size to give a buffer of `have` elements that must hold `need`: at least twice what it had, within
+// [least, most], so that arrays that grow from call to call cost a few allocations and not one each
+// (60 calls of vd_eval on 100, 150, ... 3,050 poses, page-locked memory: 30 ms taken to size, 4.0 grown,
+// 5.9 when the arrays were copied to device buffers taken to size).
+inline size_t grown_size(size_t have, size_t need, size_t least, size_t most) {
+  if (need <= have) return have;
+  return std::max({need, least, std::min(2 * have, most)});
+}
 
 // How a ligand of a batch is docked: id; lanes per chain, waves per SIMD; MC steps, local-search
 // iterations; torsions, heavy atoms, chains; wide: one chain per wavefront in 16-lane arithmetic.
