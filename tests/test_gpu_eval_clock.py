@@ -1,7 +1,8 @@
-"""Reading vd_eval's kernel time touches no stream: the words lie in page-locked memory the kernel has
-written.  So it may be read in the middle of a graph capture (where a copy would be refused and end the
-capture), waits for nobody, and costs the front end's device-pointer call, which reads it each time,
-nothing."""
+"""Reading vd_eval's kernel time waits for nobody else and may happen in the middle of a graph capture
+(where a copy on the null stream would be refused and end the capture): the words lie in page-locked
+memory the kernel has written, or, after many workgroups on small host arrays, come over on the
+context's own stream.  For the front end's device-pointer call, which reads them each time, it is no
+call of the runtime at all."""
 import ctypes as C
 import re
 
@@ -20,7 +21,8 @@ def hip_runtime():
     return C.CDLL(path)
 
 
-@pytest.mark.parametrize("n", [1, 70000])   # one workgroup, and as many as a launch takes
+# one workgroup, more than write to the host's memory, and arrays that are copied
+@pytest.mark.parametrize("n", [1, 3000, 70000])
 def test_time_read_during_a_capture(module_ctx, n):
     import vdock
     from vdock import workloads
@@ -30,8 +32,9 @@ def test_time_read_during_a_capture(module_ctx, n):
     conf = np.zeros((n, 7 + ctx.ligand_info(lid).n_torsions), dtype=np.float32)
     conf[:, 3] = 1
     ctx.eval(lid, conf)
-    before = ctx.eval_last_ms()
-    assert before > 0
+    first = ctx.eval_last_ms()
+    assert first > 0
+    ctx.eval(lid, conf)   # its time is read for the first time during the capture
     hip = hip_runtime()
     stream, graph = C.c_void_p(), C.c_void_p()
     assert hip.hipStreamCreate(C.byref(stream)) == 0
@@ -40,4 +43,5 @@ def test_time_read_during_a_capture(module_ctx, n):
     during = ctx.eval_last_ms()
     assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0 and graph.value
     assert hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(stream) == 0
-    assert during == before
+    assert 0.1 * first < during < 10 * first
+    assert ctx.eval_last_ms() == during
