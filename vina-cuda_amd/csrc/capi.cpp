@@ -1718,7 +1718,9 @@ void wide_ligands(vd_ctx* c, std::vector<LigPlan>& plans, const vd_dock_params* 
   }
   rest *= 256.0 / std::max(1, c->n_cu);
   // a ligand that must stay narrow (16 atoms have another pair layout) ends the batch anyway: wide
-  // chains next to it pay only for ligands well above it
+  // chains next to it pay only for ligands well above it.  288 batches of 3 to 80 ligands of 10 to 24
+  // atoms took 0.780, 0.788, 0.813, 0.858 of the time without wide launches with the factor at 1.0, 1.25,
+  // 1.5, 2, and at most 1.07, 1.04, 1.04, 1.02
   double line = (p->local_search == VD_LS_RILC_BFGS ? 0.7 : 0.48) * rest / 7.6e-5;
   auto can = [&](size_t k) {
     const int A = (int)lig_at(c, plans[k].id).atoms.size();
