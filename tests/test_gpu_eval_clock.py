@@ -4,7 +4,6 @@ memory the kernel has written, or, after many workgroups on small host arrays, c
 context's own stream.  For the front end's device-pointer call, which reads them each time, it is no
 call of the runtime at all."""
 import ctypes as C
-import re
 
 import numpy as np
 import pytest
@@ -12,13 +11,6 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 CAPTURE_GLOBAL = 0   # hipStreamCaptureModeGlobal
-
-
-def hip_runtime():
-    """The HIP runtime that libvdock has loaded."""
-    with open("/proc/self/maps") as f:
-        path, = {m.group(0) for m in re.finditer(r"/\S*libamdhip64\.so\S*", f.read())}
-    return C.CDLL(path)
 
 
 # one workgroup, more than write to the host's memory, and arrays that are copied
@@ -35,7 +27,7 @@ def test_time_read_during_a_capture(module_ctx, n):
     first = ctx.eval_last_ms()
     assert first > 0
     ctx.eval(lid, conf)   # its time is read for the first time during the capture
-    hip = hip_runtime()
+    hip = C.CDLL(vdock.LIB_PATH)   # looks names up in the library's own HIP runtime
     stream, graph = C.c_void_p(), C.c_void_p()
     assert hip.hipStreamCreate(C.byref(stream)) == 0
     print("capture begins", flush=True)
